@@ -1137,25 +1137,14 @@ std::vector<double> GpuVectorState::marginal_w0(size_t qbit, int basis)
 
 // ------------------------------------------- allocation-free marginal w0
 
-// The scratch of marginal_w0_noalloc: kNormBlocks partial sums per column
-// (columns at stride kNormBlocks), then one w0 per column.  516 KiB; each GPU
-// the library runs on holds its own copy until the process ends.  Every call
-// overwrites the entries it reads, so nothing needs clearing between calls.
+// The scratch of marginal_w0_noalloc: kMargBlocks partial sums per column,
+// then one w0 per column, then the columns' counts of finished workgroups
+// (zero at the start, and left zero by every call).  515 KiB; each GPU the
+// library runs on holds its own copy until the process ends.
 static constexpr size_t kNoAllocMaxCols = 256;
-static constexpr size_t kNoAllocW0 = kNoAllocMaxCols * size_t(kNormBlocks);
-static __device__ __align__(256) double scratch[kNoAllocW0 + kNoAllocMaxCols];
-
-// w0 of each column: the partials summed one after another from 0.0, the
-// order w0_from_partials uses on the host.
-__global__ void __launch_bounds__(kBlock) k_sum_partials(const double* __restrict__ part, unsigned nblocks,
-                                                         unsigned ncols, double* __restrict__ out)
-{
-    const unsigned c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncols) return;
-    double s = 0.0;
-    for (unsigned b = 0; b < nblocks; ++b) s += part[size_t(c) * nblocks + b];
-    out[c] = s;
-}
+static constexpr size_t kNoAllocW0 = kNoAllocMaxCols * size_t(kMargBlocks);
+static constexpr size_t kNoAllocDone = kNoAllocW0 + kNoAllocMaxCols;
+static __device__ __align__(256) double scratch[kNoAllocDone + kNoAllocMaxCols / 2];
 
 // The device address of `scratch` on each device, looked up once per device
 // with that device current.  The array's name is not a device address in
@@ -1205,10 +1194,8 @@ void GpuVectorState::marginal_w0_noalloc(size_t qbit, double* w0s, size_t len)
     double* part = noalloc_scratch(dev);
     double* w = part + kNoAllocW0;
     const int p = int(nr_bits_ - 1 - qbit);
-    launch_marginal_cols(prec_ == PREC_C64, col_ptr(0), dim(), uint32_t(nc), dim() / 2, p, BASIS_Z, part, stream_);
-    hipLaunchKernelGGL(k_sum_partials, dim3(unsigned((nc + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream_, part,
-                       kNormBlocks, unsigned(nc), w);
-    HIP_OK(hipGetLastError());
+    launch_marginal_cols(prec_ == PREC_C64, col_ptr(0), dim(), uint32_t(nc), dim() / 2, p, BASIS_Z, part,
+                         reinterpret_cast<uint32_t*>(part + kNoAllocDone), w, stream_);
     HIP_OK(hipMemcpyAsync(w0s, w, nc * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_OK(hipStreamSynchronize(stream_));
 }

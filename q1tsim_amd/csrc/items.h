@@ -31,13 +31,16 @@ struct TreeDesc {
     const double* lev[16];   // lev[0] unused
 };
 
-// One column's outcome-0 weight of one qubit: kNormBlocks partial sums on
-// the device, summed in order into one value.
+// One column's outcome-0 weight of one qubit: partial sums of up to
+// kMargBlocks workgroups, added by the one that finishes last.
 struct MargItem {
     const void* amp;
     uint64_t nwork;   // dim / 2
     int32_t p;        // index bit of the qubit
     int32_t basis;    // 0 Z, 1 X, 2 Y
+    uint64_t chunk0 = 0;   // first workgroup (filled by the queue)
+    uint32_t blocks = 0;   // workgroups (filled by the queue)
+    uint32_t pad = 0;
 };
 
 // Collapse of one column onto outcome 0 (dst0, scale s0) and/or 1 (dst1, s1)
@@ -163,7 +166,7 @@ private:
         hipStream_t s;
     };
     std::vector<Release> rel_;
-    uint64_t coll_chunks_ = 0, op_chunks_ = 0, basis_chunks_ = 0, level_chunks_[16] = {};
+    uint64_t marg_chunks_ = 0, coll_chunks_ = 0, op_chunks_ = 0, basis_chunks_ = 0, level_chunks_[16] = {};
 
     // device and pinned host buffers: inputs, then outputs
     char* dbuf_ = nullptr;
@@ -189,11 +192,13 @@ public:
     static void give(std::unique_ptr<ItemQueue> q);
 };
 
-// Partial sums of the outcome-0 weight of bit p for `ncols` columns at
-// stride col_stride into partial[c * kNormBlocks + b] (the arithmetic of
-// the queue's marginal items; used by the allocation-free marginal).
+// Outcome-0 weight of bit p of `ncols` (at most 65535) columns at stride
+// col_stride into w0[c], without an item table (the arithmetic of the queue's
+// marginal items; used by the allocation-free marginal).  Scratch: kMargBlocks
+// doubles per column in `partial` and one count per column in `done`, zero
+// before the call and after it.
 void launch_marginal_cols(bool c64, const void* amp, uint64_t col_stride, uint32_t ncols, uint64_t nwork, int p,
-                          int basis, double* partial, hipStream_t s);
+                          int basis, double* partial, uint32_t* done, double* w0, hipStream_t s);
 
 // Maximum ColOp arity: dense on 1-2 targets, diagonal on up to 3, phases
 // and swaps; anything else is applied by the per-gate kernels.
