@@ -232,7 +232,7 @@ public:
     void* col_ptr(size_t c) const;
     // Device scratch buffers kept between calls, one per use; growing one
     // synchronises the stream first.
-    enum ScratchSlot { SLOT_MATRIX = 0, SLOT_PROGRAM = 1, SLOT_FUSED = 2, SLOT_COUNT = 3 };
+    enum ScratchSlot { SLOT_MATRIX = 0, SLOT_PROGRAM = 1, SLOT_COLUMNS = 2, SLOT_COUNT = 3 };
     void* scratch(int slot, size_t bytes);
     void* scratch_matrix(size_t bytes) { return scratch(SLOT_MATRIX, bytes); }
     void apply_op(const GateOp& op, size_t col_begin, size_t col_end);

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "dense.h"
 #include "kernels.h"
 #include "sweep.h"
 
@@ -71,14 +72,18 @@ __global__ void __launch_bounds__(kBlock) k_dense2(V* __restrict__ amp, uint64_t
     }
 }
 
-// K-qubit dense update (K = 3..5), matrix staged in LDS.
-template <typename V, int K>
-__global__ void __launch_bounds__(kBlock) k_denseK(V* __restrict__ amp, uint64_t col_stride, uint64_t nwork,
-                                                   PosList pos, uint64_t cmask, Targets tg, const V* __restrict__ mat)
+template <typename V> struct Mat8 {
+    V m[64];
+};
+
+// Three-qubit dense update, matrix staged in LDS (wider gates: dense.hip).
+template <typename V>
+__global__ void __launch_bounds__(kBlock) k_dense3(V* __restrict__ amp, uint64_t col_stride, uint64_t nwork,
+                                                   PosList pos, uint64_t cmask, Targets tg, Mat8<V> mat)
 {
-    constexpr int D = 1 << K;
+    constexpr int K = 3, D = 1 << K;
     __shared__ V sm[D * D];
-    for (int t = threadIdx.x; t < D * D; t += blockDim.x) sm[t] = mat[t];
+    if (threadIdx.x < D * D) sm[threadIdx.x] = mat.m[threadIdx.x];
     __syncthreads();
     uint64_t off[D];
 #pragma unroll
@@ -103,38 +108,6 @@ __global__ void __launch_bounds__(kBlock) k_denseK(V* __restrict__ amp, uint64_t
             for (int c = 1; c < D; ++c) acc = cmac(acc, sm[r * D + c], v[c]);
             a[i | off[r]] = acc;
         }
-    }
-}
-
-// Dense update for 6..12 target qubits: one workgroup per amplitude group,
-// the group staged in LDS, matrix rows read from global memory.
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_dense_big(V* __restrict__ amp, uint64_t col_stride, uint64_t ngroups,
-                                                      PosList pos, uint64_t cmask, Targets tg,
-                                                      const V* __restrict__ mat)
-{
-    extern __shared__ unsigned char smem_raw[];
-    V* sg = reinterpret_cast<V*>(smem_raw);
-    const int K = tg.cnt, D = 1 << K;
-    V* a = amp + uint64_t(blockIdx.y) * col_stride;
-    for (uint64_t g = blockIdx.x; g < ngroups; g += gridDim.x) {
-        const uint64_t base = deposit(g, pos) | cmask;
-        for (int l = threadIdx.x; l < D; l += blockDim.x) {
-            uint64_t o = 0;
-            for (int q = 0; q < K; ++q)
-                if ((l >> (K - 1 - q)) & 1) o |= uint64_t(1) << tg.t[q];
-            sg[l] = a[base | o];
-        }
-        __syncthreads();
-        for (int r = threadIdx.x; r < D; r += blockDim.x) {
-            V acc = mkc<V>(0, 0);
-            for (int c = 0; c < D; ++c) acc = cmac(acc, mat[uint64_t(r) * D + c], sg[c]);
-            uint64_t o = 0;
-            for (int q = 0; q < K; ++q)
-                if ((r >> (K - 1 - q)) & 1) o |= uint64_t(1) << tg.t[q];
-            a[base | o] = acc;
-        }
-        __syncthreads();
     }
 }
 
@@ -895,36 +868,35 @@ static void launch_op(const GateOp& op, V* amp, uint64_t col_stride, size_t ncol
                 ps = gs.prof_begin();
                 hipLaunchKernelGGL(k_dense2<V>, dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride, nwork,
                                    pl, op.ctrl_mask, uint64_t(1) << op.targets[0], uint64_t(1) << op.targets[1], m4);
-            } else {
+            } else if (kt == 3) {
                 Targets tg{};
                 tg.cnt = kt;
                 for (int q = 0; q < kt; ++q) tg.t[q] = op.targets[q];
-                const size_t d = size_t(1) << kt;
-                std::vector<V> hm(d * d);
-                for (size_t k = 0; k < d * d; ++k) hm[k] = to_v<V>(op.m[k]);
-                V* dm = static_cast<V*>(gs.scratch_matrix(hm.size() * sizeof(V)));
+                Mat8<V> m8{};
+                for (int k = 0; k < 64; ++k) m8.m[k] = to_v<V>(op.m[k]);
+                kname = "k_dense3";
+                ps = gs.prof_begin();
+                hipLaunchKernelGGL(k_dense3<V>, dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride, nwork,
+                                   pl, op.ctrl_mask, tg, m8);
+            } else {
+                const DensePlan dp = plan_dense(op, n, ny, sizeof(V));
+                V* scratch = dp.scratch_bytes
+                                 ? static_cast<V*>(gs.scratch(GpuVectorState::SLOT_COLUMNS, dp.scratch_bytes))
+                                 : nullptr;
+                const bool host_packed = dp.K <= kHostPackK;
+                std::vector<V> hm(op.m.size());
+                if (host_packed) pack_dense<V>(op.m.data(), dp.K, hm.data());
+                else
+                    for (size_t k = 0; k < hm.size(); ++k) hm[k] = to_v<V>(op.m[k]);
+                // packed, or as given and then packed
+                V* dm = static_cast<V*>(gs.scratch_matrix((host_packed ? 1 : 2) * dp.matrix_bytes));
                 if (hipMemcpyAsync(dm, hm.data(), hm.size() * sizeof(V), hipMemcpyHostToDevice, st) != hipSuccess ||
                     hipStreamSynchronize(st) != hipSuccess)
                     throw Error(ERR_HIP, "matrix upload failed");
-                kname = kt <= 5 ? "k_denseK" : "k_dense_big";
+                kname = dp.tiles ? "k_dense_tile" : "k_dense_rows";
                 ps = gs.prof_begin();
-                if (kt == 3)
-                    hipLaunchKernelGGL((k_denseK<V, 3>), dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride,
-                                       nwork, pl, op.ctrl_mask, tg, dm);
-                else if (kt == 4)
-                    hipLaunchKernelGGL((k_denseK<V, 4>), dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride,
-                                       nwork, pl, op.ctrl_mask, tg, dm);
-                else if (kt == 5)
-                    hipLaunchKernelGGL((k_denseK<V, 5>), dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride,
-                                       nwork, pl, op.ctrl_mask, tg, dm);
-                else {
-                    // a group of 2^kt amplitudes in dynamic LDS: 64 KiB for 12 complex128 targets
-                    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dense_big<V>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(d * sizeof(V))) != hipSuccess)
-                        throw Error(ERR_HIP, "LDS attribute of the wide dense kernel");
-                    hipLaunchKernelGGL(k_dense_big<V>, dim3(grid_for(nwork * kBlock), ny), dim3(kBlock), d * sizeof(V),
-                                       st, a, col_stride, nwork, pl, op.ctrl_mask, tg, dm);
-                }
+                launch_dense<V>(dp, op, n, a, col_stride, ny, host_packed ? nullptr : dm,
+                                host_packed ? dm : dm + hm.size(), scratch, st);
             }
             break;
         }
