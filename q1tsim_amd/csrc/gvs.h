@@ -235,6 +235,10 @@ public:
     enum ScratchSlot { SLOT_MATRIX = 0, SLOT_PROGRAM = 1, SLOT_COLUMNS = 2, SLOT_COUNT = 3 };
     void* scratch(int slot, size_t bytes);
     void* scratch_matrix(size_t bytes) { return scratch(SLOT_MATRIX, bytes); }
+    // Pinned host memory for a flush's table (kept with the state's item
+    // queue, so it outlives the state): the copy from it is over when the
+    // flush has synchronised.
+    char* stage(size_t bytes) { return iq().stage(bytes, stream_); }
     void apply_op(const GateOp& op, size_t col_begin, size_t col_end);
 
     // planner: learned cost model (not owned) and mode; recording of sweeps
@@ -344,6 +348,7 @@ private:
     size_t slot_cap_[SLOT_COUNT] = {0, 0, 0};
     std::unique_ptr<ItemQueue> iq_;       // the single-state operations' queue
     ItemQueue& iq();
+    void staged_done() { if (iq_) iq_->stage_done(); }   // the stream is synchronised
 
     CostModel* cost_model_ = nullptr;
     int plan_mode_ = PLAN_GREEDY;

@@ -788,6 +788,7 @@ void GpuVectorState::flush()
     else
         apply_queue_plain(0, counts_.size());
     HIP_OK(hipStreamSynchronize(stream_));
+    staged_done();
     stats_.gate_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     queue_.clear();
     prof_collect();

@@ -143,6 +143,12 @@ public:
     // the queue moves to another owner); pending inputs are dropped
     void detach();
 
+    // Pinned host memory of at least `bytes` for a table that the caller
+    // copies to the device on `s`; contents are lost at the next call, which
+    // waits for `s` unless stage_done() has said that it was synchronised.
+    char* stage(size_t bytes, hipStream_t s);
+    void stage_done() { stage_stream_ = nullptr; }
+
     double w0(size_t item) const;
     const uint64_t* indices(size_t job) const;
     const double* tops(size_t job) const;
@@ -175,12 +181,19 @@ private:
     size_t hin_cap_ = 0;
     char* hout_ = nullptr;
     size_t hout_cap_ = 0;
+    char* stage_ = nullptr;
+    size_t stage_cap_ = 0;
+    hipStream_t stage_stream_ = nullptr;   // a copy from stage_ may be in flight here
     hipEvent_t in_done_ = nullptr;   // the last input upload has completed
     hipStream_t last_stream_ = nullptr;
     size_t out_w0_ = 0, out_idx_ = 0, out_top_ = 0;   // offsets in hout_
     std::vector<uint64_t> res_run0_, res_col0_;         // of the last launch
     uint64_t launches_ = 0;
 };
+
+// `bytes` of pinned host memory to device memory on `s`; both 16-byte aligned,
+// with 16-byte granules readable and writable to the end.
+void upload_table(void* dst, const void* pinned, size_t bytes, hipStream_t s);
 
 // Queues kept for reuse (their pinned and device buffers survive): states
 // come and go by the thousand, a queue's buffers would not.

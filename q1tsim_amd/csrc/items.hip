@@ -43,6 +43,38 @@ __device__ __forceinline__ uint64_t insert_zero(uint64_t j, int p)
     return ((j >> p) << (p + 1)) | (j & (bit - 1));
 }
 
+// ------------------------------------------------------------- uploads
+
+// Host table to device memory, read by a kernel over the bus.  The copy
+// engine's hand-over to the compute queue takes about 40 us before the kernel
+// that needs the table starts; this kernel's successor starts at once (17
+// qubits complex64, 60 KB of sweep programs, time from the call that starts the
+// upload to the first sweep: hipMemcpyAsync 75 us, and 65 us with a
+// synchronisation before the sweep's launch; this kernel 43 us).
+__global__ void __launch_bounds__(kBlock) k_upload(const uint4* __restrict__ from, uint4* __restrict__ to, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) to[i] = from[i];
+}
+
+// Tables up to 1 MiB: above, the copy itself outweighs the hand-over.
+static constexpr size_t kUploadKernelBytes = size_t(1) << 20;
+
+void upload_table(void* dst, const void* pinned, size_t bytes, hipStream_t s)
+{
+    if (!bytes) return;
+    if (bytes > kUploadKernelBytes) {
+        IQ_OK(hipMemcpyAsync(dst, pinned, bytes, hipMemcpyHostToDevice, s));
+        return;
+    }
+    void* from = nullptr;
+    IQ_OK(hipHostGetDevicePointer(&from, const_cast<void*>(pinned), 0));
+    const uint32_t n = uint32_t((bytes + 15) / 16);
+    hipLaunchKernelGGL(k_upload, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, static_cast<const uint4*>(from),
+                       static_cast<uint4*>(dst), n);
+    IQ_OK(hipGetLastError());
+}
+
 // ------------------------------------------------------------ marginals
 
 // One-qubit marginals: bound by HBM reads.  A column's work units (pairs of
@@ -523,6 +555,7 @@ ItemQueue::~ItemQueue()
     if (dbuf_) (void)hipFree(dbuf_);
     if (hin_) (void)hipHostFree(hin_);
     if (hout_) (void)hipHostFree(hout_);
+    if (stage_) (void)hipHostFree(stage_);
     if (in_done_) (void)hipEventDestroy(in_done_);
 }
 
@@ -689,7 +722,7 @@ void ItemQueue::launch(hipStream_t s)
     put(o_u, u_.data(), u_.size() * sizeof(double));
     if (!marg_.empty()) std::memset(hin_ + o_done, 0, marg_.size() * sizeof(uint32_t));
     if (in_bytes) {
-        IQ_OK(hipMemcpyAsync(dbuf_, hin_, in_bytes, hipMemcpyHostToDevice, s));
+        upload_table(dbuf_, hin_, in_bytes, s);
         launches_ += 1;
     }
     IQ_OK(hipEventRecord(in_done_, s));
@@ -804,6 +837,22 @@ void ItemQueue::launch(hipStream_t s)
     for (uint64_t& c : level_chunks_) c = 0;
 }
 
+char* ItemQueue::stage(size_t bytes, hipStream_t s)
+{
+    if (stage_stream_) IQ_OK(hipStreamSynchronize(stage_stream_));
+    stage_stream_ = nullptr;
+    if (bytes > stage_cap_) {
+        if (stage_) IQ_OK(hipHostFree(stage_));
+        stage_ = nullptr;
+        stage_cap_ = 0;
+        const size_t cap = std::max<size_t>(bytes, size_t(1) << 18) * 3 / 2;
+        IQ_OK(hipHostMalloc(reinterpret_cast<void**>(&stage_), cap, hipHostMallocDefault));
+        stage_cap_ = cap;
+    }
+    stage_stream_ = s;
+    return stage_;
+}
+
 double ItemQueue::w0(size_t item) const { return reinterpret_cast<const double*>(hout_ + out_w0_)[item]; }
 
 const uint64_t* ItemQueue::indices(size_t job) const
@@ -820,6 +869,8 @@ void ItemQueue::detach()
 {
     if (last_stream_) (void)hipStreamSynchronize(last_stream_);
     last_stream_ = nullptr;
+    if (stage_stream_) (void)hipStreamSynchronize(stage_stream_);
+    stage_stream_ = nullptr;
     // the upload event belongs to the last owner's stream, which may be
     // destroyed and its handle reused: the next owner records a fresh one
     if (in_done_) (void)hipEventDestroy(in_done_);

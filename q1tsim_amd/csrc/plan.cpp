@@ -71,14 +71,22 @@ namespace {
 
 // The gates a pass skips, as far as later gates are concerned: a later gate
 // may run before them only if it commutes with every one of them.
+// `rounded`, given for programs that keep the queue's rounding, says that the
+// gate's arithmetic rounds: two such gates keep their order, since their
+// products commute only up to rounding.
 struct Blocker {
     uint64_t any = 0;   // bits the skipped gates touch
     uint64_t nd = 0;    // bits they act on non-diagonally
-    bool blocks(uint64_t touched, uint64_t nondiag) const { return (touched & nd) || (nondiag & any); }
-    void add(uint64_t touched, uint64_t nondiag)
+    bool rnd = false;   // one of them rounds
+    bool blocks(uint64_t touched, uint64_t nondiag, bool rounded = false) const
+    {
+        return (touched & nd) || (nondiag & any) || (rounded && rnd);
+    }
+    void add(uint64_t touched, uint64_t nondiag, bool rounded = false)
     {
         any |= touched;
         nd |= nondiag;
+        rnd = rnd || rounded;
     }
 };
 
@@ -327,6 +335,26 @@ uint32_t dense_form(const cdouble* m)
     return SWF_GENERAL;
 }
 
+// Does applying the gate round?  Permutations and factors of +-1, +-i do not:
+// they commute bit for bit with any gate that they commute with.
+bool rounds(const GateOp& op)
+{
+    switch (op.kind) {
+    case OpKind::Identity:
+    case OpKind::Swap2:
+        return false;
+    case OpKind::PhaseOnes:
+        return op.m[0] != cdouble(0, 1) && op.m[0] != cdouble(0, -1) && op.m[0] != cdouble(-1, 0);
+    case OpKind::Dense: {
+        if (op.targets.size() != 1) return true;
+        const uint32_t f = dense_form(op.m.data());
+        return f != SWF_SWAP && f != SWF_Y;
+    }
+    default:
+        return true;
+    }
+}
+
 // Where local bit b lives in a phase with register bits `regs`: register
 // index (number of register bits below b) or thread-index bit (number of
 // non-register bits below b).
@@ -409,42 +437,78 @@ static bool writeback_gate(const GateOp& op, const LocalMap& lm)
     return true;
 }
 
+// What the register phases ask of a gate of a sweep, worked out once per sweep.
+struct PhaseGate {
+    uint64_t touched = 0, nd = 0;   // touched_bits, nondiag_bits
+    int target = -1;                // local bit of a one-target dense gate
+    bool dense = false;
+    bool wb = false;                // writeback_gate
+    bool ok = false;                // sweepable
+    bool diag = false;              // sweepable and neither dense nor a swap
+    bool rnd = false;               // `keep` programs: the gate rounds
+};
+struct PhaseGates {
+    std::vector<PhaseGate> g;   // by queue index - first
+    size_t first = 0;
+    uint64_t all = 0;           // bits of all gates
+    bool keep;                  // gates that round keep their order
+    const PhaseGate& operator[](size_t i) const { return g[i - first]; }
+    PhaseGates(const std::vector<PendingGate>& q, const std::vector<size_t>& gates, const LocalMap& lm, bool keep)
+        : keep(keep)
+    {
+        if (gates.empty()) return;
+        const auto mm = std::minmax_element(gates.begin(), gates.end());
+        first = *mm.first;
+        g.resize(*mm.second - first + 1);
+        for (size_t i : gates) {
+            const GateOp& op = q[i].op;
+            PhaseGate& p = g[i - first];
+            p.touched = touched_bits(op);
+            p.nd = nondiag_bits(op);
+            all |= p.touched;
+            p.dense = op.kind == OpKind::Dense;
+            p.ok = sweepable(op, nullptr);
+            if (p.dense && op.targets.size() == 1) p.target = lm.local_of[op.targets[0]];
+            p.wb = writeback_gate(op, lm);
+            p.diag = p.ok && !p.dense && op.kind != OpKind::Swap2;
+            p.rnd = keep && rounds(op);
+        }
+    }
+};
+
 // How a register phase over `regs` runs a gate: as an op on the registers
 // (dense gates with their target in a register, diagonal gates), in the
 // write-back map (SWAP, and X / CX whose target is not a register bit), or
 // not at all.
 enum PhaseRole { ROLE_NONE, ROLE_OP, ROLE_WRITEBACK };
-static PhaseRole phase_role(const GateOp& op, const LocalMap& lm, uint32_t regs)
+static PhaseRole phase_role(const PhaseGate& g, uint32_t regs)
 {
-    if (op.kind == OpKind::Dense && op.targets.size() == 1 && lm.local_of[op.targets[0]] >= 0 &&
-        ((regs >> lm.local_of[op.targets[0]]) & 1))
-        return sweepable(op, nullptr) ? ROLE_OP : ROLE_NONE;
-    if (writeback_gate(op, lm)) return ROLE_WRITEBACK;
-    if (sweepable(op, nullptr) && op.kind != OpKind::Dense && op.kind != OpKind::Swap2) return ROLE_OP;
-    return ROLE_NONE;
+    if (g.target >= 0 && ((regs >> g.target) & 1)) return g.ok ? ROLE_OP : ROLE_NONE;
+    if (g.wb) return ROLE_WRITEBACK;
+    return g.diag ? ROLE_OP : ROLE_NONE;
 }
 
 // Gates of `pending` a register phase over register bits `regs` takes:
 // write-back gates (SWAP, X, CX on local bits: applied as the phase writes
 // the tile back, so later gates on their bits wait for the next phase),
 // dense gates whose target is a register bit and diagonal gates (any bits),
-// in order; a gate not taken blocks its bits for the rest.
-size_t phase_absorb(const std::vector<PendingGate>& q, const std::vector<size_t>& pending, const LocalMap& lm,
-                    uint32_t regs, std::vector<size_t>* chosen, std::vector<size_t>* rest)
+// in order; a gate not taken blocks its bits for the rest, and once every bit
+// is blocked no later gate can be taken.
+size_t phase_absorb(const PhaseGates& pg, const std::vector<size_t>& pending, uint32_t regs,
+                    std::vector<size_t>* chosen, std::vector<size_t>* rest)
 {
     Blocker blk, after_wb;
     size_t count = 0;
-    for (size_t i : pending) {
-        const GateOp& op = q[i].op;
-        const uint64_t bits = touched_bits(op), nd = nondiag_bits(op);
-        const bool free = !blk.blocks(bits, nd) && !after_wb.blocks(bits, nd);
+    for (size_t x = 0; x < pending.size(); ++x) {
+        const size_t i = pending[x];
+        const PhaseGate& g = pg[i];
         bool take = false;
-        if (free) {
-            switch (phase_role(op, lm, regs)) {
+        if (!blk.blocks(g.touched, g.nd, g.rnd) && !after_wb.blocks(g.touched, g.nd)) {
+            switch (phase_role(g, regs)) {
             case ROLE_OP: take = true; break;
             case ROLE_WRITEBACK:
                 take = true;
-                after_wb.add(bits, bits);
+                after_wb.add(g.touched, g.touched);
                 break;
             default: break;
             }
@@ -452,9 +516,13 @@ size_t phase_absorb(const std::vector<PendingGate>& q, const std::vector<size_t>
         if (take) {
             ++count;
             if (chosen) chosen->push_back(i);
-        } else {
-            blk.add(bits, nd);
-            if (rest) rest->push_back(i);
+            continue;
+        }
+        blk.add(g.touched, g.nd, g.rnd);
+        if (rest) rest->push_back(i);
+        if ((blk.nd | after_wb.nd) == pg.all) {
+            if (rest) rest->insert(rest->end(), pending.begin() + std::ptrdiff_t(x) + 1, pending.end());
+            break;
         }
     }
     return count;
@@ -492,38 +560,36 @@ static void append_factors(TileFactors& tf, int M, std::vector<SwPhase>& phases,
 // more gates: every phase costs a full LDS round trip of the tile.  Tile
 // factors go to `tf`; a phase left with no op and no write-back map is not
 // emitted.
-std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const std::vector<size_t>& pending,
-                                  const LocalMap& lm, int M, int R, std::vector<SwPhase>& phases,
-                                  std::vector<SwOp>& ops, bool search, std::vector<size_t>* order,
-                                  TileFactors* tf)
+std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const PhaseGates& pg,
+                                  const std::vector<size_t>& pending, const LocalMap& lm, int M, int R,
+                                  std::vector<SwPhase>& phases, std::vector<SwOp>& ops, bool search,
+                                  std::vector<size_t>* order, TileFactors* tf)
 {
     uint32_t regs = 0;
     int nregs = 0;
     Blocker blk;
     for (size_t i : pending) {
-        const GateOp& op = q[i].op;
-        const uint64_t bits = touched_bits(op), nd = nondiag_bits(op);
-        if (blk.blocks(bits, nd) || !sweepable(op, nullptr)) {
-            blk.add(bits, nd);
-            continue;
-        }
-        if (op.kind == OpKind::Dense) {
-            const int lb = lm.local_of[op.targets[0]];
-            if ((regs >> lb) & 1) continue;
-            if (nregs < R) {
-                regs |= 1u << lb;
+        const PhaseGate& g = pg[i];
+        if (blk.blocks(g.touched, g.nd, g.rnd) || !g.ok) {
+            blk.add(g.touched, g.nd, g.rnd);
+        } else if (g.dense && !((regs >> g.target) & 1)) {
+            if (pg.keep && g.wb) {
+                blk.add(g.touched, g.touched);   // left to the write-back map
+            } else if (nregs < R) {
+                regs |= 1u << g.target;
                 ++nregs;
             } else {
-                blk.add(bits, nd);
+                blk.add(g.touched, g.nd, g.rnd);
             }
         }
+        if (blk.nd == pg.all) break;
     }
     for (int b = 0; b < M && nregs < R; ++b)
         if (!((regs >> b) & 1)) {
             regs |= 1u << b;
             ++nregs;
         }
-    size_t best = phase_absorb(q, pending, lm, regs, nullptr, nullptr);
+    size_t best = phase_absorb(pg, pending, regs, nullptr, nullptr);
     for (int iter = 0; search && iter < 4 * M; ++iter) {
         bool improved = false;
         for (int a = 0; a < M && !improved; ++a) {
@@ -531,7 +597,7 @@ std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const std::
             for (int b = 0; b < M; ++b) {
                 if ((regs >> b) & 1) continue;
                 const uint32_t r2 = (regs & ~(1u << a)) | (1u << b);
-                const size_t c = phase_absorb(q, pending, lm, r2, nullptr, nullptr);
+                const size_t c = phase_absorb(pg, pending, r2, nullptr, nullptr);
                 if (c > best) {
                     best = c;
                     regs = r2;
@@ -543,7 +609,7 @@ std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const std::
         if (!improved) break;
     }
     std::vector<size_t> chosen, rest;
-    phase_absorb(q, pending, lm, regs, &chosen, &rest);
+    phase_absorb(pg, pending, regs, &chosen, &rest);
     // Permutation gates taken as register ops (X, CX and SWAP with their
     // target in a register) that no later register op of the phase touches
     // commute with every later op: they join the write-back map (composed
@@ -552,12 +618,11 @@ std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const std::
     {
         uint64_t later = 0;   // bits of the later gates that stay register ops
         for (size_t x = chosen.size(); x-- > 0;) {
-            const GateOp& op = q[chosen[x]].op;
-            if (phase_role(op, lm, regs) != ROLE_OP) continue;
-            const uint64_t bits = touched_bits(op);
-            if (writeback_gate(op, lm) && !(bits & later)) continue;
+            const PhaseGate& g = pg[chosen[x]];
+            if (phase_role(g, regs) != ROLE_OP) continue;
+            if (g.wb && !(g.touched & later)) continue;
             as_op[x] = 1;
-            later |= bits;
+            later |= g.touched;
         }
     }
     SwPhase ph = make_phase(0, regs, M, uint32_t(ops.size()));
@@ -693,9 +758,91 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
     std::vector<size_t> pending = step.gates;
     TileFactors tf;
     TileFactors* tfp = factors ? &tf : nullptr;
-    while (!pending.empty()) pending = one_reg_phase(q, pending, lm, M, R, phases, ops, search, order, tfp);
+    const PhaseGates pg(q, pending, lm, false);
+    while (!pending.empty()) pending = one_reg_phase(q, pg, pending, lm, M, R, phases, ops, search, order, tfp);
     append_factors(tf, M, phases, ops, order);
 }
+
+std::vector<PlanStep> plan_whole(const std::vector<PendingGate>& q, int M)
+{
+    std::vector<PlanStep> steps;
+    PlanStep cur;
+    auto close = [&] {
+        if (cur.gates.empty()) return;
+        cur.sweep = true;
+        for (int b = 0; b < M; ++b) cur.tile.push_back(b);
+        steps.push_back(std::move(cur));
+        cur = PlanStep{};
+    };
+    for (size_t i = 0; i < q.size(); ++i) {
+        if (q[i].op.kind == OpKind::Identity) continue;
+        if (sweepable(q[i].op, nullptr)) {
+            cur.gates.push_back(i);
+            continue;
+        }
+        close();
+        steps.push_back(PlanStep{false, {}, {i}});
+    }
+    close();
+    return steps;
+}
+
+template <typename R>
+void build_whole(const std::vector<PendingGate>& q, const PlanStep& step, int M, int nr, std::vector<WholePhase>& phases,
+                 std::vector<WholeOpT<R>>& ops)
+{
+    const LocalMap lm(step.tile);
+    std::vector<size_t> pending = step.gates;
+    std::vector<SwPhase> ph;
+    std::vector<SwOp> so;
+    const PhaseGates pg(q, pending, lm, true);
+    while (!pending.empty()) pending = one_reg_phase(q, pg, pending, lm, M, nr, ph, so, false, nullptr, nullptr);
+    const int sw = sweep_swizzle_bits(M), nt = M - nr;
+    auto slot = [&](uint32_t l) { return uint16_t(swizzle_slot(sw, M, int(l))); };
+    for (const SwPhase& p : ph) {
+        WholePhase w;
+        std::memset(&w, 0, sizeof(w));
+        w.op_begin = p.op_begin;
+        w.op_end = p.op_end;
+        w.wmap = p.wmap;
+        w.wxor = slot(p.wxor);
+        for (int b = 0; b < nt; ++b) {
+            w.col[b] = uint32_t(slot(1u << p.tbit[b])) | uint32_t(slot(p.wcol[b])) << 16;
+        }
+        for (int k = 0; k < (1 << nr); ++k) {
+            uint32_t l = 0, l2 = 0;
+            for (int b = 0; b < nr; ++b)
+                if ((k >> b) & 1) {
+                    l |= 1u << p.rpos[b];
+                    l2 ^= p.wcol[nt + b];
+                }
+            w.slot[k] = uint32_t(slot(l)) | uint32_t(slot(l2)) << 16;
+        }
+        phases.push_back(w);
+    }
+    for (const SwOp& o : so) {
+        WholeOpT<R> w;
+        std::memset(&w, 0, sizeof(w));
+        w.cr = o.cr;
+        w.ct = o.ct;
+        if (o.type == SW_DENSE1) {
+            w.code = o.aux == SWF_REAL ? uint32_t(SWF_REAL_SEQ) : o.aux == SWF_RX ? uint32_t(SWF_RX_SEQ) : o.aux;
+            w.code |= uint32_t(o.reg) << 8;
+        } else if (o.type == SW_PHASE) {
+            w.code = kWholePhase + o.aux;
+        } else if (o.dreg >= 0) {
+            w.code = kWholeDiagReg | uint32_t(o.dreg) << 8;
+        } else {
+            w.code = kWholeDiagTid | uint32_t(o.dtid) << 16;
+        }
+        for (int k = 0; k < 8; ++k) w.m[k] = R(o.m[k]);
+        ops.push_back(w);
+    }
+}
+template void build_whole<double>(const std::vector<PendingGate>&, const PlanStep&, int, int, std::vector<WholePhase>&,
+                                  std::vector<WholeOpT<double>>&);
+template void build_whole<float>(const std::vector<PendingGate>&, const PlanStep&, int, int, std::vector<WholePhase>&,
+                                 std::vector<WholeOpT<float>>&);
 
 std::vector<size_t> plan_order(const std::vector<PendingGate>& q, int n, const TileGeom& g, bool search)
 {
@@ -720,6 +867,7 @@ void build_fused_program(const std::vector<PendingGate>& q, const PlanStep& step
     std::vector<size_t> pending = step.gates;
     TileFactors tf;
     TileFactors* tfp = factors ? &tf : nullptr;
+    const PhaseGates pg(q, pending, lm, false);
     while (!pending.empty()) {
         // grow one block: gates whose bits are all in the tile, while the
         // union of their local bits stays within K (order kept per bit)
@@ -749,7 +897,7 @@ void build_fused_program(const std::vector<PendingGate>& q, const PlanStep& step
             absorbed.push_back(i);
         }
         if (absorbed.empty()) {
-            pending = one_reg_phase(q, pending, lm, M, R, phases, ops, search, nullptr, tfp);
+            pending = one_reg_phase(q, pg, pending, lm, M, R, phases, ops, search, nullptr, tfp);
             continue;
         }
         if (search && int(B.size()) == K) {

@@ -16,6 +16,7 @@
 #include <atomic>
 #include <chrono>
 #include <exception>
+#include <functional>
 #include <mutex>
 #include <thread>
 #include <cmath>
@@ -163,6 +164,154 @@ static int block_level(const std::vector<SwPhase>& phases)
         if (ph.kind == 1) lv = std::max(lv, ph.reg_mask > 4 ? 2 : 1);
     return lv;
 }
+
+// ------------------------------------------------- whole states in LDS
+
+constexpr int whole_regs(int n) { return n <= 13 ? 3 : 4; }   // register bits: at most 1024 threads
+static int whole_bits(int n) { return std::max(n, whole_regs(n)); }
+
+template <typename V, int NR, int R>
+__device__ __forceinline__ void whole_dense(uint32_t form, int reg, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, V m0,
+                                            V m1, V m2, V m3)
+{
+    switch (form) {
+    case SWF_REAL_SEQ: dense_ctl<V, NR, R, SWF_REAL_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_SWAP: dense_ctl<V, NR, R, SWF_SWAP>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_RX_SEQ: dense_ctl<V, NR, R, SWF_RX_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_Y: dense_ctl<V, NR, R, SWF_Y>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    default: dense_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    }
+}
+
+// One column of up to 2^14 amplitudes per workgroup, in LDS from its load to
+// its store: 2^R amplitudes per thread in registers, the program's register
+// phases as in the tile sweeps, one LDS exchange and barrier per phase.  Bound
+// by latency: a few waves per SIMD, each op a uniform branch; so the next op's
+// record is loaded while the current one runs.  Waves past the column's
+// threads leave at once (barriers count the waves that are left).
+// Before, one launch per gate (single states: 3.2 us per gate at 12 qubits) or
+// one barrier and a full LDS pass per gate (batches: 9 us per gate at 13
+// qubits).  Measured: 12 qubits complex128, 350 gates 1110 -> 138 us; 112
+// columns of 10 to 13 qubits complex64 in a batch 2850 -> 340 us per round.
+template <typename V, int R>
+__global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ items,
+                                                const WholePhase* __restrict__ phases,
+                                                const WholeOpT<typename RealOf<V>::type>* __restrict__ ops)
+{
+    constexpr int NR = 1 << R;
+    extern __shared__ unsigned char smem_whole[];
+    V* s = reinterpret_cast<V*>(smem_whole);
+    const WholeItem it = load_uniform(items, blockIdx.x);
+    const int M = int(it.n) > R ? int(it.n) : R, sw = sweep_swizzle_bits(M);
+    const uint32_t nth = 1u << (M - R), N = 1u << it.n, tid = threadIdx.x;
+    if (tid >= nth) return;
+    V* a = static_cast<V*>(it.amp);
+    {
+        V x[NR];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const uint32_t l = tid + uint32_t(k) * nth;
+            x[k] = mkc<V>(0, 0);
+            if (l < N) x[k] = a[l];
+        }
+#pragma unroll
+        for (int k = 0; k < NR; ++k) s[swizzle_slot(sw, M, int(tid + uint32_t(k) * nth))] = x[k];
+    }
+    __syncthreads();
+    for (uint32_t p = 0; p < it.nphases; ++p) {
+        const WholePhase ph = load_uniform(phases, it.phases + p);
+        uint32_t t = ph.wxor << 16;
+#pragma unroll
+        for (int b = 0; b < 10; ++b) t ^= (0u - ((tid >> b) & 1u)) & ph.col[b];
+        const uint32_t tin = t & 0xffffu, tout = t >> 16;
+        V v[NR];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) v[k] = s[tin ^ (ph.slot[k] & 0xffffu)];
+        const uint32_t o1 = it.ops + ph.op_end;
+        uint32_t oi = it.ops + ph.op_begin;
+        WholeOpT<typename RealOf<V>::type> nxt = load_uniform(ops, oi);   // the table ends with a spare record
+        while (oi < o1) {
+            const WholeOpT<typename RealOf<V>::type> op = nxt;
+            ++oi;
+            nxt = load_uniform(ops, oi);
+            const uint32_t body = op.code & 0xffu, cr = op.cr, ct = op.ct;
+            const int reg = int((op.code >> 8) & 0xffu);
+            const bool tok = (tid & ct) == ct;
+            const V m0 = mkc<V>(op.m[0], op.m[1]), m1 = mkc<V>(op.m[2], op.m[3]);
+            if (body < kWholePhase) {
+                const V m2 = mkc<V>(op.m[4], op.m[5]), m3 = mkc<V>(op.m[6], op.m[7]);
+                whole_dense<V, NR, R>(body, reg, v, cr, ct, tok, m0, m1, m2, m3);
+            } else if (body < kWholeDiagReg) {
+                phase_op<V, NR>(body - kWholePhase, v, cr, ct, tok, m0);
+            } else if (body == kWholeDiagReg) {
+                scale_regs<V, NR>(v, cr, ct, tok, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, m1, m0), x); });
+            } else {
+                const V d = sel(((tid >> (op.code >> 16)) & 1) != 0, m1, m0);
+                scale_regs<V, NR>(v, cr, ct, tok, [&](int, V x) { return cmul(d, x); });
+            }
+        }
+        if (ph.wmap == 0) {
+#pragma unroll
+            for (int k = 0; k < NR; ++k) s[tin ^ (ph.slot[k] & 0xffffu)] = v[k];
+        } else {
+            __syncthreads();   // other threads' slots are overwritten
+#pragma unroll
+            for (int k = 0; k < NR; ++k) s[tout ^ (ph.slot[k] >> 16)] = v[k];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+        const uint32_t l = tid + uint32_t(k) * nth;
+        if (l < N) a[l] = s[swizzle_slot(sw, M, int(l))];
+    }
+}
+
+// `nitems` columns of states of at most n_max qubits (the LDS and threads of
+// the widest).  Tables in device memory; the op table ends with a spare record.
+template <typename V>
+static void launch_whole(int n_max, const WholeItem* items, size_t nitems, const WholePhase* phases,
+                         const WholeOpT<typename RealOf<V>::type>* ops, hipStream_t stream)
+{
+    const int R = whole_regs(n_max), M = whole_bits(n_max);
+    const size_t lds = sizeof(V) << M;
+    const dim3 grid{unsigned(nitems)}, block{unsigned(std::max(64, 1 << (M - R)))};
+    auto go = [&](auto kernel) {
+        if (lds > (size_t(64) << 10))
+            SW_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, items, phases, ops);
+    };
+    if (R == 3) go(&k_whole<V, 3>);
+    else if constexpr (sizeof(V) == 8) go(&k_whole<V, 4>);
+    else throw Error(ERR_INVALID_ARGUMENT, "No whole-state kernel for 2^14 complex128 amplitudes");
+    SW_HIP_OK(hipGetLastError());
+}
+
+// The programs of a small state's whole-state steps, appended to `phases` and
+// `ops` (records of one step: phases [ph0[s], ph0[s] + nph[s]), ops from op0[s]).
+template <typename R> struct WholeTables {
+    std::vector<WholePhase> phases;
+    std::vector<WholeOpT<R>> ops;
+    std::vector<uint32_t> ph0, nph, op0;
+    void build(const std::vector<PendingGate>& q, const std::vector<PlanStep>& steps, int n)
+    {
+        ph0.assign(steps.size(), 0);
+        nph.assign(steps.size(), 0);
+        op0.assign(steps.size(), 0);
+        for (size_t s = 0; s < steps.size(); ++s) {
+            if (!steps[s].sweep) continue;
+            std::vector<WholePhase> p;
+            std::vector<WholeOpT<R>> o;
+            build_whole<R>(q, steps[s], whole_bits(n), whole_regs(n), p, o);
+            ph0[s] = uint32_t(phases.size());
+            nph[s] = uint32_t(p.size());
+            op0[s] = uint32_t(ops.size());
+            phases.insert(phases.end(), p.begin(), p.end());
+            ops.insert(ops.end(), o.begin(), o.end());
+        }
+    }
+};
 
 // One sweep's program: phases, ops and its own block table (block phases
 // index it through op_begin until the table is merged into the flush's).
@@ -432,6 +581,155 @@ std::vector<std::string> plan_jit_sources(const std::vector<PendingGate>& q, int
     return out;
 }
 
+// The single-gate kernels of a step in a launch signature (they hold their
+// matrices by value); false if one cannot be captured.
+static bool put_single_gates(const std::vector<PendingGate>& queue, const PlanStep& step, std::vector<uint64_t>& sig)
+{
+    auto put = [&](uint64_t x) { sig.push_back(x); };
+    bool ok = true;
+    for (size_t i : step.gates) {
+        const GateOp& op = queue[i].op;
+        // a kernel of 3+ targets uploads its matrix and synchronises
+        if (op.kind == OpKind::Dense && op.targets.size() >= 3) ok = false;
+        put(uint64_t(op.kind));
+        put(op.ctrl_mask);
+        put(op.targets.size());
+        for (int t : op.targets) put(uint64_t(t));
+        put(op.m.size());
+        for (const cdouble& c : op.m) {
+            double re = c.real(), im = c.imag();
+            uint64_t u;
+            std::memcpy(&u, &re, 8);
+            put(u);
+            std::memcpy(&u, &im, 8);
+            put(u);
+        }
+    }
+    return ok;
+}
+
+// Uploads a flush's table (`host`: the state's pinned staging memory, which
+// the flush's final synchronisation frees for the next one) and launches its
+// kernels; with a launch signature, as a graph: replayed while the signature
+// repeats, else captured anew.
+static void run_table(GpuVectorState& st, const char* host, size_t total, std::vector<uint64_t>* sig,
+                      const std::function<void(char*)>& launch_all, RunStats& stats)
+{
+    auto upload = [&](char* dst) {
+        upload_table(dst, host, total, st.stream());
+    };
+    if (!sig) {
+        char* dprog = total ? static_cast<char*>(st.scratch(GpuVectorState::SLOT_PROGRAM, total)) : nullptr;
+        upload(dprog);
+        launch_all(dprog);
+        return;
+    }
+    if (GpuVectorState::FlushGraph* hit = st.find_graph(*sig)) {
+        upload(static_cast<char*>(hit->table));
+        SW_HIP_OK(hipGraphLaunch(hit->exec, st.stream()));
+        const RunStats& d = hit->delta;
+        stats.bytes += d.bytes;
+        stats.launches += d.launches;
+        stats.sweeps += d.sweeps;
+        stats.gates += d.gates;
+        stats.blocks += d.blocks;
+        stats.phases += d.phases;
+        stats.mfma_flops += d.mfma_flops;
+        st.note_graph(false);
+        return;
+    }
+    GpuVectorState::FlushGraph& fg = st.new_graph_slot(total);
+    char* table = static_cast<char*>(fg.table);
+    upload(table);
+    const RunStats before = stats;
+    SW_HIP_OK(hipStreamBeginCapture(st.stream(), hipStreamCaptureModeThreadLocal));
+    try {
+        launch_all(table);
+    } catch (...) {
+        hipGraph_t part = nullptr;
+        (void)hipStreamEndCapture(st.stream(), &part);
+        if (part) (void)hipGraphDestroy(part);
+        throw;
+    }
+    hipGraph_t gr = nullptr;
+    SW_HIP_OK(hipStreamEndCapture(st.stream(), &gr));
+    hipGraphExec_t exec = nullptr;
+    const hipError_t ie = hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(gr);
+    SW_HIP_OK(ie);
+    fg.exec = exec;
+    fg.sig = std::move(*sig);
+    fg.delta = RunStats{};
+    fg.delta.bytes = stats.bytes - before.bytes;
+    fg.delta.launches = stats.launches - before.launches;
+    fg.delta.sweeps = stats.sweeps - before.sweeps;
+    fg.delta.gates = stats.gates - before.gates;
+    fg.delta.blocks = stats.blocks - before.blocks;
+    fg.delta.mfma_flops = stats.mfma_flops - before.mfma_flops;
+    fg.delta.phases = stats.phases - before.phases;
+    st.note_graph(true);
+    SW_HIP_OK(hipGraphLaunch(exec, st.stream()));
+}
+
+// A flush of a state that is too small for tiles: whole-state programs
+// (k_whole), one launch for all columns, and single-gate kernels for the gates
+// no register phase takes.
+template <typename V>
+static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
+                      RunStats& stats)
+{
+    using R = typename RealOf<V>::type;
+    const int n = int(st.nr_bits());
+    const size_t ncols = col_end - col_begin;
+    const std::vector<PlanStep> steps = plan_whole(queue, whole_bits(n));
+    WholeTables<R> wt;
+    wt.build(queue, steps, n);
+    wt.ops.push_back(WholeOpT<R>{});   // the spare record
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    const size_t ooff = up(wt.phases.size() * sizeof(WholePhase));
+    const size_t ioff = up(ooff + wt.ops.size() * sizeof(WholeOpT<R>));
+    const size_t total = up(ioff + steps.size() * ncols * sizeof(WholeItem));
+    char* const host = st.stage(total);
+    std::memcpy(host, wt.phases.data(), wt.phases.size() * sizeof(WholePhase));
+    std::memcpy(host + ooff, wt.ops.data(), wt.ops.size() * sizeof(WholeOpT<R>));
+    WholeItem* items = reinterpret_cast<WholeItem*>(host + ioff);   // step-major
+    for (size_t s = 0; s < steps.size(); ++s)
+        for (size_t c = 0; c < ncols; ++c)
+            items[s * ncols + c] = WholeItem{st.col_ptr(col_begin + c), uint32_t(n), wt.nph[s], wt.ph0[s], wt.op0[s]};
+    const double S = double(uint64_t(1) << n) * sizeof(V) * double(ncols);
+    auto launch_all = [&](char* d) {
+        for (size_t s = 0; s < steps.size(); ++s) {
+            if (!steps[s].sweep) {
+                for (size_t i : steps[s].gates) st.apply_op(queue[i].op, col_begin, col_end);
+                continue;
+            }
+            const int ps = st.prof_begin();
+            launch_whole<V>(n, reinterpret_cast<const WholeItem*>(d + ioff) + s * ncols, ncols,
+                            reinterpret_cast<const WholePhase*>(d),
+                            reinterpret_cast<const WholeOpT<R>*>(d + ooff), st.stream());
+            st.prof_end(ps, sizeof(V) == 16 ? "k_whole_c128" : "k_whole_c64", 2.0 * S);
+            stats.launches += 1;
+            stats.sweeps += 1;
+            stats.gates += steps[s].gates.size();
+            stats.bytes += 2.0 * S;
+            stats.phases += wt.nph[s];
+        }
+    };
+    bool graph = st.graph_enabled();
+    std::vector<uint64_t> sig;
+    if (graph) {
+        for (uint64_t x : {uint64_t(n), uint64_t(st.precision()), uint64_t(col_begin), uint64_t(col_end),
+                           uint64_t(total), uint64_t(ooff), uint64_t(ioff),
+                           uint64_t(reinterpret_cast<uintptr_t>(st.col_ptr(col_begin)))})
+            sig.push_back(x);
+        for (const PlanStep& step : steps) {
+            sig.push_back(step.sweep ? 1 : 0);
+            if (!step.sweep) graph = put_single_gates(queue, step, sig) && graph;
+        }
+    }
+    run_table(st, host, total, graph ? &sig : nullptr, launch_all, stats);
+}
+
 void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
                  int fusion_k, bool tiling, RunStats& stats)
 {
@@ -439,6 +737,11 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
     const TileGeom g = st.geometry();
     if (!tiling) {
         for (const PendingGate& pg : queue) st.apply_op(pg.op, col_begin, col_end);
+        return;
+    }
+    if (n < g.M + 2) {
+        if (st.precision() == PREC_C128) run_whole<double2>(st, queue, col_begin, col_end, stats);
+        else run_whole<float2>(st, queue, col_begin, col_end, stats);
         return;
     }
     const double S = double(uint64_t(1) << n) * double(st.elem_bytes()) * double(col_end - col_begin);
@@ -462,17 +765,17 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         nblocks += progs[s].nblocks;
     }
     const size_t boff = total;
-    total += nblk_floats * sizeof(float);
-    std::vector<char> host(total);
+    total += (nblk_floats * sizeof(float) + 15) / 16 * 16;
+    char* const host = st.stage(total);
     for (size_t s = 0; s < steps.size(); ++s) {
         if (!steps[s].sweep) continue;
         // block phases address the merged table
         for (SwPhase& ph : progs[s].phases)
             if (ph.kind == 1) ph.op_begin += uint32_t(boff_s[s]);
-        std::memcpy(host.data() + poff[s], progs[s].phases.data(), progs[s].phases.size() * sizeof(SwPhase));
-        std::memcpy(host.data() + ooff[s], progs[s].ops.data(), progs[s].ops.size() * sizeof(SwOp));
+        std::memcpy(host + poff[s], progs[s].phases.data(), progs[s].phases.size() * sizeof(SwPhase));
+        std::memcpy(host + ooff[s], progs[s].ops.data(), progs[s].ops.size() * sizeof(SwOp));
         if (!progs[s].blocks.empty())
-            std::memcpy(host.data() + boff + boff_s[s] * sizeof(float), progs[s].blocks.data(),
+            std::memcpy(host + boff + boff_s[s] * sizeof(float), progs[s].blocks.data(),
                         progs[s].blocks.size() * sizeof(float));
     }
     // kernels specialised to each sweep's program (compiled on first use)
@@ -491,13 +794,6 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         for (size_t s = 0; s < steps.size(); ++s)
             if (steps[s].sweep) jitfn[s] = jc.function(src[s], false);
     }
-    // ordered after earlier work on this (non-blocking) stream, which may
-    // still read the table; the host copy must outlive the transfer
-    auto upload = [&](char* dst) {
-        if (!total) return;
-        SW_HIP_OK(hipMemcpyAsync(dst, host.data(), total, hipMemcpyHostToDevice, st.stream()));
-        SW_HIP_OK(hipStreamSynchronize(st.stream()));
-    };
     auto launch_all = [&](char* dprog) {
         const float* dblocks = reinterpret_cast<const float*>(dprog + boff);
         for (size_t s = 0; s < steps.size(); ++s) {
@@ -575,79 +871,10 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
                 put(uint64_t(block_level(progs[s].phases)));
                 continue;
             }
-            for (size_t i : steps[s].gates) {
-                const GateOp& op = queue[i].op;
-                // a kernel of 3+ targets uploads its matrix and synchronises
-                if (op.kind == OpKind::Dense && op.targets.size() >= 3) graph = false;
-                put(uint64_t(op.kind));
-                put(op.ctrl_mask);
-                put(op.targets.size());
-                for (int t : op.targets) put(uint64_t(t));
-                put(op.m.size());
-                for (const cdouble& c : op.m) {
-                    double re = c.real(), im = c.imag();
-                    uint64_t u;
-                    std::memcpy(&u, &re, 8);
-                    put(u);
-                    std::memcpy(&u, &im, 8);
-                    put(u);
-                }
-            }
+            graph = put_single_gates(queue, steps[s], sig);
         }
     }
-    if (!graph) {
-        char* dprog = total ? static_cast<char*>(st.scratch(GpuVectorState::SLOT_PROGRAM, total)) : nullptr;
-        upload(dprog);
-        launch_all(dprog);
-        return;
-    }
-
-    // graph path: replay while the signature repeats, else capture anew
-    if (GpuVectorState::FlushGraph* hit = st.find_graph(sig)) {
-        upload(static_cast<char*>(hit->table));
-        SW_HIP_OK(hipGraphLaunch(hit->exec, st.stream()));
-        const RunStats& d = hit->delta;
-        stats.bytes += d.bytes;
-        stats.launches += d.launches;
-        stats.sweeps += d.sweeps;
-        stats.gates += d.gates;
-        stats.blocks += d.blocks;
-        stats.phases += d.phases;
-        stats.mfma_flops += d.mfma_flops;
-        st.note_graph(false);
-        return;
-    }
-    GpuVectorState::FlushGraph& fg = st.new_graph_slot(total);
-    char* table = static_cast<char*>(fg.table);
-    upload(table);
-    const RunStats before = stats;
-    SW_HIP_OK(hipStreamBeginCapture(st.stream(), hipStreamCaptureModeThreadLocal));
-    try {
-        launch_all(table);
-    } catch (...) {
-        hipGraph_t part = nullptr;
-        (void)hipStreamEndCapture(st.stream(), &part);
-        if (part) (void)hipGraphDestroy(part);
-        throw;
-    }
-    hipGraph_t gr = nullptr;
-    SW_HIP_OK(hipStreamEndCapture(st.stream(), &gr));
-    hipGraphExec_t exec = nullptr;
-    const hipError_t ie = hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(gr);
-    SW_HIP_OK(ie);
-    fg.exec = exec;
-    fg.sig = std::move(sig);
-    fg.delta = RunStats{};
-    fg.delta.bytes = stats.bytes - before.bytes;
-    fg.delta.launches = stats.launches - before.launches;
-    fg.delta.sweeps = stats.sweeps - before.sweeps;
-    fg.delta.gates = stats.gates - before.gates;
-    fg.delta.blocks = stats.blocks - before.blocks;
-    fg.delta.mfma_flops = stats.mfma_flops - before.mfma_flops;
-    fg.delta.phases = stats.phases - before.phases;
-    st.note_graph(true);
-    SW_HIP_OK(hipGraphLaunch(exec, st.stream()));
+    run_table(st, host, total, graph ? &sig : nullptr, launch_all, stats);
 }
 
 // ------------------------------------------------------------- batches
@@ -689,174 +916,6 @@ PinnedBuffer::~PinnedBuffer()
     if (ptr) (void)hipHostFree(ptr);
 }
 
-// A gate of a small state, applied in LDS.
-struct SmallOp {
-    int32_t kind;      // 0: dense on nt targets, 1: diagonal on nt targets, 2: phase on cmask, 3: swap t0/t1
-    int32_t nt;
-    int32_t t[3];      // target index bits, t[0] = local MSB
-    int32_t npos;      // deposit positions (targets and controls, ascending)
-    int32_t pos[14];
-    uint64_t cmask;
-    uint32_t moff;     // offset of the matrix / diagonal / phase in the value table
-    uint32_t pad;
-};
-
-struct SmallItem {
-    void* amp;
-    int32_t n;
-    int32_t op_begin, op_end;
-    int32_t pad;
-};
-
-__device__ __forceinline__ uint32_t deposit_small(uint32_t j, const SmallOp& op)
-{
-#pragma unroll
-    for (int k = 0; k < 14; ++k) {
-        if (k < op.npos) {
-            const int s = op.pos[k];
-            j = ((j >> s) << (s + 1)) | (j & ((1u << s) - 1));
-        }
-    }
-    return j;
-}
-
-// Whole states in LDS, one workgroup per (state, column) item; gates one
-// after the other with a barrier in between.
-template <typename V>
-__global__ void __launch_bounds__(256) k_small_batch(const SmallItem* __restrict__ items, int nitems,
-                                                     const SmallOp* __restrict__ ops, const double2* __restrict__ vals)
-{
-    extern __shared__ unsigned char smem_small[];
-    V* s = reinterpret_cast<V*>(smem_small);
-    using Rl = typename RealOf<V>::type;
-    const int tid = threadIdx.x, bd = blockDim.x;
-    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const SmallItem& item = items[it];
-        V* a = static_cast<V*>(item.amp);
-        const uint32_t N = 1u << item.n;
-        for (uint32_t i = tid; i < N; i += bd) s[i] = a[i];
-        __syncthreads();
-        for (int o = item.op_begin; o < item.op_end; ++o) {
-            const SmallOp& op = ops[o];
-            const double2* mv = vals + op.moff;
-            if (op.kind == 0) {
-                const int nt = op.nt, D = 1 << nt;
-                const uint32_t nwork = N >> op.npos;
-                for (uint32_t w = tid; w < nwork; w += bd) {
-                    const uint32_t base = deposit_small(w, op) | uint32_t(op.cmask);
-                    V x[8], y[8];
-                    uint32_t ix[8];
-#pragma unroll
-                    for (int l = 0; l < 8; ++l) {
-                        if (l < D) {
-                            uint32_t i = base;
-#pragma unroll
-                            for (int q = 0; q < 3; ++q)
-                                if (q < nt && ((l >> (nt - 1 - q)) & 1)) i |= 1u << op.t[q];
-                            ix[l] = i;
-                            x[l] = s[i];
-                        }
-                    }
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        if (r < D) {
-                            V acc = mkc<V>(0, 0);
-#pragma unroll
-                            for (int c = 0; c < 8; ++c)
-                                if (c < D) {
-                                    const double2 m = mv[r * D + c];
-                                    acc = cmac(acc, mkc<V>(Rl(m.x), Rl(m.y)), x[c]);
-                                }
-                            y[r] = acc;
-                        }
-                    }
-#pragma unroll
-                    for (int r = 0; r < 8; ++r)
-                        if (r < D) s[ix[r]] = y[r];
-                }
-            } else if (op.kind == 1) {
-                const uint32_t nwork = N >> op.npos;
-                for (uint32_t w = tid; w < nwork; w += bd) {
-                    const uint32_t i = deposit_small(w, op) | uint32_t(op.cmask);
-                    int l = 0;
-#pragma unroll
-                    for (int q = 0; q < 3; ++q)
-                        if (q < op.nt) l = (l << 1) | int((i >> op.t[q]) & 1);
-                    const double2 d = mv[l];
-                    s[i] = cmul(mkc<V>(Rl(d.x), Rl(d.y)), s[i]);
-                }
-            } else if (op.kind == 2) {
-                const uint32_t nwork = N >> op.npos;
-                const double2 d = mv[0];
-                const V ph = mkc<V>(Rl(d.x), Rl(d.y));
-                for (uint32_t w = tid; w < nwork; w += bd) {
-                    const uint32_t i = deposit_small(w, op) | uint32_t(op.cmask);
-                    s[i] = cmul(ph, s[i]);
-                }
-            } else {
-                const uint32_t nwork = N >> op.npos;
-                const uint32_t b0 = 1u << op.t[0], b1 = 1u << op.t[1];
-                for (uint32_t w = tid; w < nwork; w += bd) {
-                    const uint32_t i = deposit_small(w, op) | uint32_t(op.cmask);
-                    const V x = s[i | b1];
-                    s[i | b1] = s[i | b0];
-                    s[i | b0] = x;
-                }
-            }
-            __syncthreads();
-        }
-        for (uint32_t i = tid; i < N; i += bd) a[i] = s[i];
-        __syncthreads();
-    }
-}
-
-static SmallOp make_small_op(const GateOp& g, std::vector<double2>& vals)
-{
-    SmallOp o;
-    std::memset(&o, 0, sizeof(o));
-    std::vector<int> pos;
-    for (int b = 0; b < 64; ++b)
-        if ((g.ctrl_mask >> b) & 1) pos.push_back(b);
-    o.cmask = g.ctrl_mask;
-    o.moff = uint32_t(vals.size());
-    auto push = [&](const cdouble& c) { vals.push_back(double2{c.real(), c.imag()}); };
-    switch (g.kind) {
-    case OpKind::Dense:
-        o.kind = 0;
-        o.nt = int(g.targets.size());
-        for (int q = 0; q < o.nt; ++q) {
-            o.t[q] = g.targets[q];
-            pos.push_back(g.targets[q]);
-        }
-        for (const cdouble& c : g.m) push(c);
-        break;
-    case OpKind::Diag:
-        o.kind = 1;
-        o.nt = int(g.targets.size());
-        for (int q = 0; q < o.nt; ++q) o.t[q] = g.targets[q];
-        for (const cdouble& c : g.m) push(c);
-        break;
-    case OpKind::PhaseOnes:
-        o.kind = 2;
-        push(g.m[0]);
-        break;
-    case OpKind::Swap2:
-        o.kind = 3;
-        o.nt = 2;
-        o.t[0] = g.targets[0];
-        o.t[1] = g.targets[1];
-        pos.push_back(g.targets[0]);
-        pos.push_back(g.targets[1]);
-        break;
-    default:
-        break;
-    }
-    std::sort(pos.begin(), pos.end());
-    o.npos = int(pos.size());
-    for (size_t k = 0; k < pos.size(); ++k) o.pos[k] = pos[k];
-    return o;
-}
-
 void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t stream, DeviceBuffer& prog,
                        PinnedBuffer& stage, ItemQueue& iq, RunStats& agg, unsigned tile_chunk, double* plan_s,
                        double* pack_s)
@@ -878,20 +937,19 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
         if (s->precision() != prec || s->geometry().M != g.M || s->geometry().R != g.R)
             throw Error(ERR_INVALID_ARGUMENT, "A batch needs one precision and tile shape");
 
-    // 1. plans and programs (host), small-state op lists: each state on its
-    // own, in parallel over host threads; then merged into one upload
+    // 1. plans and programs (host): each state on its own, in parallel over
+    // host threads; then merged into one upload
     struct Plan {
         std::vector<PlanStep> steps;
         std::vector<std::vector<SwPhase>> ph;
         std::vector<std::vector<SwOp>> ops;
         std::vector<float> blocks;
-        std::vector<SmallOp> sops;
-        std::vector<double2> svals;
+        WholeTables<double> wd;   // small states: the programs of their precision
+        WholeTables<float> wf;
         std::vector<size_t> poff, ooff;
         std::vector<int> nph;
         std::vector<char> blk;    // per step: block_level of its program
         bool small = false;
-        int sop_begin = 0, sop_end = 0;
         RunStats st;
         std::string error;
     };
@@ -902,17 +960,20 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
         Plan& p = plans[i];
         const int n = int(st.nr_bits());
         const double S = double(uint64_t(1) << n) * double(st.elem_bytes()) * double(st.nr_cols());
-        bool lds_ok = n < g.M + 2;
-        for (const PendingGate& pg : q)
-            if (pg.op.kind == OpKind::Dense && pg.op.targets.size() > 3) lds_ok = false;
-        if (lds_ok) {
+        if (n < g.M + 2) {
             p.small = true;
-            for (const PendingGate& pg : q)
-                if (pg.op.kind != OpKind::Identity) p.sops.push_back(make_small_op(pg.op, p.svals));
-            p.st.sweeps = 1;
-            p.st.launches = 1;
-            p.st.gates = q.size();
-            p.st.bytes = 2.0 * S;
+            p.steps = plan_whole(q, whole_bits(n));
+            if (prec == PREC_C128) p.wd.build(q, p.steps, n);
+            else p.wf.build(q, p.steps, n);
+            const std::vector<uint32_t>& nph = prec == PREC_C128 ? p.wd.nph : p.wf.nph;
+            for (size_t s = 0; s < p.steps.size(); ++s) {
+                if (!p.steps[s].sweep) continue;
+                p.st.sweeps += 1;
+                p.st.launches += 1;
+                p.st.gates += p.steps[s].gates.size();
+                p.st.bytes += 2.0 * S;
+                p.st.phases += nph[s];
+            }
             return;
         }
         const bool search = live[i]->plan_search(S);
@@ -955,23 +1016,22 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
     if (plan_s) *plan_s += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_plan).count();
     const auto t_pack = std::chrono::steady_clock::now();
     // 2. one table in pinned memory, uploaded in one copy: every state's
-    // phases and ops, the block matrices, the small-state ops and items, and
-    // per round one sweep item per state (all its columns).  Offsets first
+    // phases and ops, the block matrices, the small states' programs, and per
+    // round one sweep item per state (all its columns) and one whole-state item
+    // per small state's column.  Offsets first
     // (serial arithmetic), then the states fill their parts in parallel.
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-    size_t off = 0, max_steps = 0, nblock_floats = 0, nsops = 0, nsvals = 0;
-    int max_small_n = 0;
-    std::vector<size_t> bbase(live.size(), 0), sbase(live.size(), 0), vbase(live.size(), 0);
+    const size_t wop_bytes = prec == PREC_C128 ? sizeof(WholeOpT<double>) : sizeof(WholeOpT<float>);
+    size_t off = 0, max_steps = 0, nblock_floats = 0, nwph = 0, nwops = 0;
+    std::vector<size_t> bbase(live.size(), 0), wpbase(live.size(), 0), wobase(live.size(), 0);
     for (size_t i = 0; i < live.size(); ++i) {
         Plan& p = plans[i];
+        max_steps = std::max(max_steps, p.steps.size());
         if (p.small) {
-            sbase[i] = nsops;
-            vbase[i] = nsvals;
-            p.sop_begin = int(nsops);
-            nsops += p.sops.size();
-            nsvals += p.svals.size();
-            p.sop_end = int(nsops);
-            max_small_n = std::max(max_small_n, int(live[i]->nr_bits()));
+            wpbase[i] = nwph;
+            wobase[i] = nwops;
+            nwph += prec == PREC_C128 ? p.wd.phases.size() : p.wf.phases.size();
+            nwops += prec == PREC_C128 ? p.wd.ops.size() : p.wf.ops.size();
             continue;
         }
         bbase[i] = nblock_floats;
@@ -989,19 +1049,51 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             off = up(off + p.ops[s].size() * sizeof(SwOp));
             p.nph[s] = int(p.ph[s].size());
         }
-        max_steps = std::max(max_steps, p.steps.size());
     }
     const size_t boff = off;
     off = up(off + nblock_floats * sizeof(float));
-    const size_t soff = off;
-    off = up(off + nsops * sizeof(SmallOp));
-    const size_t voff = off;
-    off = up(off + nsvals * sizeof(double2));
-    size_t nsitems = 0;
-    for (size_t i = 0; i < live.size(); ++i)
-        if (plans[i].small && plans[i].sop_end != plans[i].sop_begin) nsitems += live[i]->nr_cols();
-    const size_t sioff = off;
-    off = up(off + nsitems * sizeof(SmallItem));
+    const size_t wpoff = off;
+    off = up(off + nwph * sizeof(WholePhase));
+    const size_t wooff = off;
+    off = up(off + (nwops + 1) * wop_bytes);   // and a spare record
+    // whole-state items: round-major, within a round the widest states first;
+    // the columns of state i in round r start at witem[r][i].  A round of up
+    // to 256 items is one launch per register count (every item has a CU of
+    // its own), a longer one a launch per width, so that narrow states do not
+    // take the LDS of the widest.
+    struct WholeGroup {
+        size_t first, count;
+        int n_max;
+    };
+    std::vector<std::vector<WholeGroup>> wgroups(max_steps);
+    std::vector<std::vector<size_t>> witem(max_steps);
+    size_t nwitems = 0;
+    {
+        std::vector<size_t> small;
+        for (size_t i = 0; i < live.size(); ++i)
+            if (plans[i].small) small.push_back(i);
+        std::stable_sort(small.begin(), small.end(),
+                         [&](size_t x, size_t y) { return live[x]->nr_bits() > live[y]->nr_bits(); });
+        for (size_t r = 0; r < max_steps && !small.empty(); ++r) {
+            witem[r].assign(live.size(), 0);
+            size_t round = 0;
+            for (size_t i : small)
+                if (r < plans[i].steps.size() && plans[i].steps[r].sweep) round += live[i]->nr_cols();
+            for (size_t i : small) {
+                if (r >= plans[i].steps.size() || !plans[i].steps[r].sweep) continue;
+                const int n = int(live[i]->nr_bits());
+                std::vector<WholeGroup>& gr = wgroups[r];
+                const bool same = !gr.empty() && whole_regs(gr.back().n_max) == whole_regs(n) &&
+                                  (round <= 256 || gr.back().n_max == n || gr.back().n_max <= 10);
+                if (!same) gr.push_back(WholeGroup{nwitems, 0, n});
+                witem[r][i] = nwitems;
+                nwitems += live[i]->nr_cols();
+                gr.back().count += live[i]->nr_cols();
+            }
+        }
+    }
+    const size_t wioff = off;
+    off = up(off + nwitems * sizeof(WholeItem));
     // sweep items: round-major; item (r, i) at item_at[r][i], tiles from
     // round_first[r][i]
     std::vector<std::pair<size_t, size_t>> round_items(max_steps);   // (first item, count)
@@ -1030,31 +1122,27 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
     char* dbase = static_cast<char*>(prog.get(total, stream));
     char* host = static_cast<char*>(stage.get(total));
     {
-        // small-state items in state order
-        std::vector<size_t> si_first(live.size(), 0);
-        size_t k = 0;
-        for (size_t i = 0; i < live.size(); ++i) {
-            si_first[i] = k;
-            if (plans[i].small && plans[i].sop_end != plans[i].sop_begin) k += live[i]->nr_cols();
-        }
         std::atomic<size_t> next{0};
         auto fill = [&] {
             for (size_t i = next++; i < live.size(); i = next++) {
                 Plan& p = plans[i];
                 GpuVectorState& st = *live[i];
                 if (p.small) {
-                    SmallOp* so = reinterpret_cast<SmallOp*>(host + soff) + sbase[i];
-                    for (size_t j = 0; j < p.sops.size(); ++j) {
-                        so[j] = p.sops[j];
-                        so[j].moff += uint32_t(vbase[i]);
-                    }
-                    std::memcpy(reinterpret_cast<double2*>(host + voff) + vbase[i], p.svals.data(),
-                                p.svals.size() * sizeof(double2));
-                    if (p.sop_end != p.sop_begin) {
-                        SmallItem* it = reinterpret_cast<SmallItem*>(host + sioff) + si_first[i];
-                        for (size_t c = 0; c < st.nr_cols(); ++c)
-                            it[c] = SmallItem{st.col_ptr(c), int(st.nr_bits()), p.sop_begin, p.sop_end, 0};
-                    }
+                    auto copy = [&](const auto& wt) {
+                        std::memcpy(host + wpoff + wpbase[i] * sizeof(WholePhase), wt.phases.data(),
+                                    wt.phases.size() * sizeof(WholePhase));
+                        std::memcpy(host + wooff + wobase[i] * wop_bytes, wt.ops.data(), wt.ops.size() * wop_bytes);
+                        WholeItem* it = reinterpret_cast<WholeItem*>(host + wioff);
+                        for (size_t s = 0; s < p.steps.size(); ++s) {
+                            if (!p.steps[s].sweep) continue;
+                            for (size_t c = 0; c < st.nr_cols(); ++c)
+                                it[witem[s][i] + c] =
+                                    WholeItem{st.col_ptr(c), uint32_t(st.nr_bits()), wt.nph[s],
+                                              uint32_t(wpbase[i]) + wt.ph0[s], uint32_t(wobase[i]) + wt.op0[s]};
+                        }
+                    };
+                    if (prec == PREC_C128) copy(p.wd);
+                    else copy(p.wf);
                     continue;
                 }
                 std::memcpy(reinterpret_cast<float*>(host + boff) + bbase[i], p.blocks.data(),
@@ -1096,37 +1184,28 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
         fill();
         for (std::thread& t : pool) t.join();
     }
-    SW_HIP_OK(hipMemcpyAsync(dbase, host, total, hipMemcpyHostToDevice, stream));
+    std::memset(host + wooff + nwops * wop_bytes, 0, wop_bytes);
+    upload_table(dbase, host, total, stream);
     if (pack_s) *pack_s += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_pack).count();
 
-    // 2. small states: one launch
-    if (nsitems) {
-        const size_t lds = size_t(live[0]->elem_bytes()) << max_small_n;
-        if (prec == PREC_C128) {
-            SW_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_small_batch<double2>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-            hipLaunchKernelGGL(k_small_batch<double2>, dim3(unsigned(std::min<size_t>(nsitems, 65535))),
-                               dim3(256), lds, stream, reinterpret_cast<const SmallItem*>(dbase + sioff),
-                               int(nsitems), reinterpret_cast<const SmallOp*>(dbase + soff),
-                               reinterpret_cast<const double2*>(dbase + voff));
-        } else {
-            SW_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_small_batch<float2>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-            hipLaunchKernelGGL(k_small_batch<float2>, dim3(unsigned(std::min<size_t>(nsitems, 65535))),
-                               dim3(256), lds, stream, reinterpret_cast<const SmallItem*>(dbase + sioff),
-                               int(nsitems), reinterpret_cast<const SmallOp*>(dbase + soff),
-                               reinterpret_cast<const double2*>(dbase + voff));
-        }
-        SW_HIP_OK(hipGetLastError());
-        agg.launches += 1;
-    }
-
-    // 3. rounds: single-gate steps of each state, then one batched sweep launch
+    // 3. rounds: single-gate steps of each state, then the whole-state
+    // launches, then one batched sweep launch
     for (size_t r = 0; r < max_steps; ++r) {
         for (size_t i = 0; i < live.size(); ++i) {
             const Plan& p = plans[i];
             if (r >= p.steps.size() || p.steps[r].sweep) continue;
             for (size_t gi : p.steps[r].gates) live[i]->apply_op(live[i]->pending()[gi].op, 0, live[i]->nr_cols());
+        }
+        for (const WholeGroup& wg : wgroups[r]) {
+            const WholeItem* wi = reinterpret_cast<const WholeItem*>(dbase + wioff) + wg.first;
+            const WholePhase* wp = reinterpret_cast<const WholePhase*>(dbase + wpoff);
+            if (prec == PREC_C128)
+                launch_whole<double2>(wg.n_max, wi, wg.count, wp,
+                                      reinterpret_cast<const WholeOpT<double>*>(dbase + wooff), stream);
+            else
+                launch_whole<float2>(wg.n_max, wi, wg.count, wp,
+                                     reinterpret_cast<const WholeOpT<float>*>(dbase + wooff), stream);
+            agg.launches += 1;
         }
         if (!round_items[r].second) continue;
         const SweepItem* ditems = reinterpret_cast<const SweepItem*>(dbase + items_off) + round_items[r].first;

@@ -134,6 +134,13 @@ __device__ __forceinline__ void dense_pairs(V (&v)[NR], uint32_t cr, bool tok, V
             const auto a = m0.x, b = m1.y;
             nx = mkc<V>(fmad(a, x.x, -(b * y.y)), fmad(a, x.y, b * y.x));
             ny = mkc<V>(fmad(a, y.x, -(b * x.y)), fmad(a, y.y, b * x.x));
+        } else if constexpr (FORM == SWF_REAL_SEQ) {
+            nx = mkc<V>(fmad(m1.x, y.x, m0.x * x.x), fmad(m1.x, y.y, m0.x * x.y));
+            ny = mkc<V>(fmad(m3.x, y.x, m2.x * x.x), fmad(m3.x, y.y, m2.x * x.y));
+        } else if constexpr (FORM == SWF_RX_SEQ) {
+            const auto a = m0.x, b = m1.y;
+            nx = mkc<V>(fmad(-b, y.y, a * x.x), fmad(b, y.x, a * x.y));
+            ny = mkc<V>(fmad(a, y.x, -(b * x.y)), fmad(a, y.y, b * x.x));
         } else {  // SWF_Y
             nx = mkc<V>(y.y, -y.x);
             ny = mkc<V>(-x.y, x.x);

@@ -21,7 +21,12 @@ namespace q1t {
 enum SwOpType : int32_t { SW_DENSE1 = 0, SW_PHASE = 1, SW_DIAG1 = 2, SW_BLOCK = 3 };
 
 // Body of a SW_DENSE1 op, read off its 2x2 matrix (SwOp::aux).
-enum SwDenseForm : uint32_t { SWF_GENERAL = 0, SWF_REAL = 1, SWF_SWAP = 2, SWF_RX = 3, SWF_Y = 4 };
+// The _SEQ forms round as the general body does (its second product fused):
+// whole-state programs use them, which give the bits of the gates applied one
+// by one with the general body.
+enum SwDenseForm : uint32_t {
+    SWF_GENERAL = 0, SWF_REAL = 1, SWF_SWAP = 2, SWF_RX = 3, SWF_Y = 4, SWF_REAL_SEQ = 5, SWF_RX_SEQ = 6
+};
 // Body of a SW_PHASE op (SwOp::aux): general, times i, times -i, times -1.
 enum SwPhaseForm : uint32_t { SWP_GENERAL = 0, SWP_I = 1, SWP_MINUS_I = 2, SWP_NEG = 3 };
 
@@ -79,7 +84,42 @@ constexpr int swizzle_slot(int SW, int M, int l)
     return l ^ (f & ((1 << SW) - 1));
 }
 
-// Swizzle width of the sweep kernels for 2^M tiles (12 -> 4, 13 -> 5).
-constexpr int sweep_swizzle_bits(int M) { return M - 8; }
+// Swizzle width of the sweep kernels for 2^M tiles (13 -> 5, else 4).
+constexpr int sweep_swizzle_bits(int M) { return M == 13 ? 5 : 4; }
+
+// ---- whole-state programs (k_whole): a state of up to 14 qubits in LDS
+
+// One op; its values m follow in the state's precision (WholeOpT).  `code`:
+// bits 0-7 body (SwDenseForm, or kWholePhase + SwPhaseForm, kWholeDiagReg,
+// kWholeDiagTid), bits 8-15 register bit of the target, bits 16-23 thread bit
+// of a diagonal target.
+constexpr uint32_t kWholePhase = 16, kWholeDiagReg = 20, kWholeDiagTid = 21;
+template <typename R> struct WholeOpT {
+    uint32_t code;
+    uint32_t cr;     // controls over register indices
+    uint32_t ct;     // controls over thread-index bits
+    uint32_t pad;
+    R m[8];
+};
+
+// A register phase: R register bits, thread bits the others.  The LDS slot of a
+// thread's element k is tin ^ (slot[k] & 0xffff) when the phase reads the state
+// and tout ^ (slot[k] >> 16) when it writes it back; tin and tout are the low
+// and high halves of the XOR of col over the thread's set bits, tout also of
+// wxor; all swizzled.
+struct WholePhase {
+    uint32_t op_begin, op_end;
+    uint32_t wmap;       // 0: written back where it was read
+    uint32_t wxor;
+    uint32_t col[12];
+    uint32_t slot[16];
+};
+
+struct WholeItem {
+    void* amp;           // the column
+    uint32_t n;          // qubits
+    uint32_t nphases;
+    uint32_t phases, ops;   // first records in the tables
+};
 
 }  // namespace q1t
