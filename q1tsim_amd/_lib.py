@@ -207,7 +207,7 @@ def unpack_result(res):
             return {elems[i].key.decode("utf-8"): elems[i].count for i in range(res.length)}
         if res.restype == RESULT_CSTATE:
             ptr = ctypes.cast(res.data, ctypes.POINTER(ctypes.c_uint64))
-            return [ptr[i] for i in range(res.length)]
+            return ptr[:res.length]
         raise Q1tError(-1, "Unknown data type code: {}".format(res.restype))
     finally:
         L.result_free(res)

@@ -297,11 +297,9 @@ extern "C" int q1t_circuit_jit_compile(const circuit_t* ptr, int precision, int 
             if (op.type != OpType::Gate) throw Error(ERR_INVALID_ARGUMENT, "jit compile: the circuit holds non-gate ops");
             std::vector<double> pv;
             for (const Param& p : op.params) pv.push_back(p.get());
-            const std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+            const GateMatrix m = gate_matrix(*op.gate, pv.data());
             PendingGate pg;
             pg.op = analyze_gate(m.data(), op.bits.size(), op.bits.data(), n);
-            pg.matrix = m;
-            for (size_t b : op.bits) pg.qbits.push_back(int(n - 1 - b));
             q.push_back(std::move(pg));
         }
         const std::vector<std::string> srcs =
@@ -364,9 +362,7 @@ extern "C" int q1t_circuit_set_initial_amplitudes(circuit_t* ptr, const double* 
     NEED(ptr);
     NEED(amps);
     return guard([&] {
-        std::vector<cdouble> a(len);
-        for (size_t i = 0; i < len; ++i) a[i] = cdouble(amps[2 * i], amps[2 * i + 1]);
-        ptr->c.set_initial_amplitudes(std::move(a));
+        ptr->c.set_initial_amplitudes(reinterpret_cast<const cdouble*>(amps), len);
     });
 }
 
@@ -397,7 +393,7 @@ extern "C" int q1t_circuit_plan_order(const circuit_t* ptr, int precision, int s
             if (op.type != OpType::Gate) throw Error(ERR_INVALID_ARGUMENT, "plan order: the circuit holds non-gate ops");
             std::vector<double> pv;
             for (const Param& p : op.params) pv.push_back(p.get());
-            const std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+            const GateMatrix m = gate_matrix(*op.gate, pv.data());
             PendingGate pg;
             pg.op = analyze_gate(m.data(), op.bits.size(), op.bits.data(), n);
             q.push_back(std::move(pg));
@@ -932,7 +928,7 @@ extern "C" int q1t_gate_matrix(const char* name, const double* params, size_t np
         if (!g) throw err_unknown_gate(name);
         if (size_t(g->nparams) != nparams) throw err_invalid_nr_arguments(nparams, size_t(g->nparams), g->desc);
         if (nparams && !params) throw Error(ERR_INVALID_ARGUMENT, "Null parameter array");
-        std::vector<cdouble> m = gate_matrix(*g, params);
+        const GateMatrix m = gate_matrix(*g, params);
         if (cap < 2 * m.size()) throw err_not_enough_space(cap, 2 * m.size());
         for (size_t k = 0; k < m.size(); ++k) {
             out[2 * k] = m[k].real();

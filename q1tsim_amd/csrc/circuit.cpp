@@ -93,11 +93,11 @@ void Circuit::set_backend(Precision prec, int fusion_k, bool tiling)
     tiling_ = tiling;
 }
 
-void Circuit::set_initial_amplitudes(std::vector<cdouble> amps)
+void Circuit::set_initial_amplitudes(const cdouble* amps, size_t len)
 {
-    if (amps.size() != (size_t(1) << nr_qbits_))
+    if (len != (size_t(1) << nr_qbits_))
         throw Error(ERR_INVALID_ARGUMENT, "Initial amplitude vector must have 2^nr_qbits entries");
-    init_amps_ = std::move(amps);
+    init_amps_.assign(amps, amps + len);   // into the memory of the last ones
     init_mode_ = 1;
 }
 
@@ -140,14 +140,14 @@ void Circuit::reexecute()
 void Circuit::apply_named(GpuVectorState& st, const char* name, size_t q)
 {
     const GateSpec* g = find_gate(name);
-    std::vector<cdouble> m = gate_matrix(*g, nullptr);
+    const GateMatrix m = gate_matrix(*g, nullptr);
     st.apply_gate(m.data(), 1, &q, 1, g->desc);
 }
 
 void Circuit::apply_named_all(GpuVectorState& st, const char* name)
 {
     const GateSpec* g = find_gate(name);
-    std::vector<cdouble> m = gate_matrix(*g, nullptr);
+    const GateMatrix m = gate_matrix(*g, nullptr);
     st.apply_unary_gate_all(m.data(), g->desc);
 }
 
@@ -170,7 +170,7 @@ bool Circuit::queue_gates()
         if (op.type != OpType::Gate) return true;
         pv.clear();
         for (const Param& p : op.params) pv.push_back(p.get());
-        std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+        const GateMatrix m = gate_matrix(*op.gate, pv.data());
         st.apply_gate(m.data(), gate_nbits(*op.gate), op.bits.data(), op.bits.size(), op.gate->desc);
     }
     return false;
@@ -275,7 +275,7 @@ bool Circuit::conditional_enqueue(ItemQueue& q)
     const std::vector<uint8_t> apply = condition(op);
     std::vector<double> pv;
     for (const Param& p : op.params) pv.push_back(p.get());
-    std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+    const GateMatrix m = gate_matrix(*op.gate, pv.data());
     if (!state_->conditional_enqueue(q, apply.data(), apply.size(), m.data(), gate_nbits(*op.gate), op.bits.data(),
                                      op.bits.size(), op.gate->desc))
         return false;
@@ -298,7 +298,7 @@ void Circuit::run_op(const CircuitOp& op)
     case OpType::Gate: {
         pv.clear();
         for (const Param& p : op.params) pv.push_back(p.get());
-        std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+        const GateMatrix m = gate_matrix(*op.gate, pv.data());
         st.apply_gate(m.data(), gate_nbits(*op.gate), op.bits.data(), op.bits.size(), op.gate->desc);
         break;
     }
@@ -306,7 +306,7 @@ void Circuit::run_op(const CircuitOp& op)
         const std::vector<uint8_t> apply = condition(op);
         pv.clear();
         for (const Param& p : op.params) pv.push_back(p.get());
-        std::vector<cdouble> m = gate_matrix(*op.gate, pv.data());
+        const GateMatrix m = gate_matrix(*op.gate, pv.data());
         st.apply_conditional_gate(apply.data(), apply.size(), m.data(), gate_nbits(*op.gate), op.bits.data(),
                                   op.bits.size(), op.gate->desc);
         break;

@@ -111,7 +111,7 @@ public:
     void seed(uint64_t s) { rng_.reseed(s); }
     Xoshiro256 rng_state() const { return rng_; }
     void set_rng_state(const Xoshiro256& r) { rng_ = r; }
-    void set_initial_amplitudes(std::vector<cdouble> amps);
+    void set_initial_amplitudes(const cdouble* amps, size_t len);
     void set_initial_random(uint64_t seed);
     GpuVectorState* state() { return state_.get(); }
     const GpuVectorState* state() const { return state_.get(); }

@@ -1,9 +1,11 @@
 // Shared definitions for the q1tsim MI355X statevector backend.
 #pragma once
 
+#include <algorithm>
 #include <complex>
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -11,6 +13,62 @@
 namespace q1t {
 
 using cdouble = std::complex<double>;
+
+// A short list held in place, on the heap above N elements: gates are queued by
+// the ten thousand, and an allocation per list was most of their host time.
+template <typename T, size_t N> class InlineVec {
+public:
+    InlineVec() = default;
+    InlineVec(std::initializer_list<T> l) { assign(l.begin(), l.size()); }
+    size_t size() const { return n_; }
+    bool empty() const { return n_ == 0; }
+    T* data() { return n_ > N ? heap_.data() : in_; }
+    const T* data() const { return n_ > N ? heap_.data() : in_; }
+    T& operator[](size_t i) { return data()[i]; }
+    const T& operator[](size_t i) const { return data()[i]; }
+    T* begin() { return data(); }
+    T* end() { return data() + n_; }
+    const T* begin() const { return data(); }
+    const T* end() const { return data() + n_; }
+    void clear() { n_ = 0; }
+    void assign(const T* p, size_t n)
+    {
+        if (n > N) heap_.assign(p, p + n);
+        else std::copy(p, p + n, in_);
+        n_ = n;
+    }
+    void assign(size_t n, const T& v)
+    {
+        if (n > N) heap_.assign(n, v);
+        else std::fill(in_, in_ + n, v);
+        n_ = n;
+    }
+    void adopt(std::vector<T>&& v)
+    {
+        if (v.size() <= N) {
+            assign(v.data(), v.size());
+            return;
+        }
+        heap_ = std::move(v);
+        n_ = heap_.size();
+    }
+    void push_back(const T& v)
+    {
+        if (n_ < N) {
+            in_[n_] = v;
+        } else {
+            if (n_ == N) heap_.assign(in_, in_ + N);
+            else heap_.resize(n_);
+            heap_.push_back(v);
+        }
+        ++n_;
+    }
+
+private:
+    size_t n_ = 0;
+    T in_[N] = {};
+    std::vector<T> heap_;
+};
 
 // Error kinds; the values are the public Q1T_ERR_* codes of q1tsim_gvs.h and
 // mirror the variants of the reference's Error enum (src/error.rs:135-173).

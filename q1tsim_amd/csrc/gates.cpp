@@ -38,11 +38,11 @@ size_t gate_nbits(const GateSpec& g) { return (g.base == G_SWAP ? 2 : 1) + size_
 
 static cdouble polar(double r, double th) { return cdouble(r * std::cos(th), r * std::sin(th)); }
 
-std::vector<cdouble> gate_matrix(const GateSpec& g, const double* p)
+GateMatrix gate_matrix(const GateSpec& g, const double* p)
 {
     const double hs = 0.70710678118654752440;
     const cdouble z(0, 0), o(1, 0), i(0, 1);
-    std::vector<cdouble> m;
+    GateMatrix m;
     switch (g.base) {
     case G_I: m = {o, z, z, o}; break;
     case G_H: m = {hs, hs, hs, -hs}; break;
@@ -80,7 +80,7 @@ std::vector<cdouble> gate_matrix(const GateSpec& g, const double* p)
     case G_V: m = {cdouble(0.5, 0.5), cdouble(0.5, -0.5), cdouble(0.5, -0.5), cdouble(0.5, 0.5)}; break;
     case G_VDG: m = {cdouble(0.5, -0.5), cdouble(0.5, 0.5), cdouble(0.5, 0.5), cdouble(0.5, -0.5)}; break;
     case G_SWAP:
-        m.assign(16, z);
+        m.assign(size_t(16), z);
         m[0] = o;
         m[1 * 4 + 2] = o;
         m[2 * 4 + 1] = o;
@@ -91,11 +91,12 @@ std::vector<cdouble> gate_matrix(const GateSpec& g, const double* p)
     size_t d = (g.base == G_SWAP) ? 4 : 2;
     for (int c = 0; c < g.nctrl; ++c) {
         size_t nd = 2 * d;
-        std::vector<cdouble> big(nd * nd, z);
+        GateMatrix big;
+        big.assign(nd * nd, z);
         for (size_t k = 0; k < d; ++k) big[k * nd + k] = o;
         for (size_t r = 0; r < d; ++r)
             for (size_t q = 0; q < d; ++q) big[(d + r) * nd + d + q] = m[r * d + q];
-        m.swap(big);
+        m = std::move(big);
         d = nd;
     }
     return m;
@@ -103,7 +104,7 @@ std::vector<cdouble> gate_matrix(const GateSpec& g, const double* p)
 
 // Is local bit `b` a control of the d x d matrix m: no mixing across the bit
 // and identity on its 0-subspace?
-static bool is_control(const std::vector<cdouble>& m, size_t d, int b)
+static bool is_control(const cdouble* m, size_t d, int b)
 {
     for (size_t r = 0; r < d; ++r)
         for (size_t c = 0; c < d; ++c) {
@@ -118,18 +119,16 @@ static bool is_control(const std::vector<cdouble>& m, size_t d, int b)
     return true;
 }
 
-// Keep the bit-b = 1 block of m.
-static std::vector<cdouble> take_one_block(const std::vector<cdouble>& m, size_t d, int b)
+// Keep the bit-b = 1 block of m (in place: every entry moves to a lower index).
+static void take_one_block(cdouble* m, size_t d, int b)
 {
     size_t h = d / 2;
-    std::vector<cdouble> r(h * h);
     auto expand = [b](size_t x) {
         size_t lo = x & ((size_t(1) << b) - 1);
         return ((x >> b) << (b + 1)) | (size_t(1) << b) | lo;
     };
     for (size_t i = 0; i < h; ++i)
-        for (size_t j = 0; j < h; ++j) r[i * h + j] = m[expand(i) * d + expand(j)];
-    return r;
+        for (size_t j = 0; j < h; ++j) m[i * h + j] = m[expand(i) * d + expand(j)];
 }
 
 GateOp analyze_gate(const cdouble* mat, size_t k, const size_t* qbits, size_t nr_bits)
@@ -139,63 +138,80 @@ GateOp analyze_gate(const cdouble* mat, size_t k, const size_t* qbits, size_t nr
         for (size_t b = a + 1; b < k; ++b)
             if (qbits[a] == qbits[b]) throw Error(ERR_INVALID_ARGUMENT, "Repeated qubit index in gate");
     size_t d = size_t(1) << k;
-    std::vector<cdouble> m(mat, mat + d * d);
+    // the table's gates fit the local copy
+    cdouble local[64];
+    std::vector<cdouble> large;
+    cdouble* m = local;
+    if (d * d > 64) {
+        large.assign(mat, mat + d * d);
+        m = large.data();
+    } else {
+        std::copy(mat, mat + d * d, local);
+    }
     // qubit listed j sits at local bit k-1-j and at index bit nr_bits-1-q
-    std::vector<int> tgt;
-    for (size_t j = 0; j < k; ++j) tgt.push_back(int(nr_bits - 1 - qbits[j]));
+    size_t tgt[64], nt = k;
+    for (size_t j = 0; j < k; ++j) tgt[j] = nr_bits - 1 - qbits[j];
     bool changed = true;
-    while (changed && tgt.size() > 1) {
+    while (changed && nt > 1) {
         changed = false;
-        size_t kk = tgt.size();
-        for (size_t j = 0; j < kk && tgt.size() > 1; ++j) {
-            int b = int(kk - 1 - j);
+        for (size_t j = 0; j < nt; ++j) {
+            int b = int(nt - 1 - j);
             if (is_control(m, d, b)) {
                 op.ctrl_mask |= uint64_t(1) << tgt[j];
-                m = take_one_block(m, d, b);
+                take_one_block(m, d, b);
                 d /= 2;
-                tgt.erase(tgt.begin() + j);
+                for (size_t x = j + 1; x < nt; ++x) tgt[x - 1] = tgt[x];
+                --nt;
                 changed = true;
                 break;
             }
         }
     }
-    op.targets = tgt;
-    size_t kt = tgt.size();
+    for (size_t j = 0; j < nt; ++j) op.targets.push_back(int(tgt[j]));
     bool diag = true, ident = true;
-    for (size_t r = 0; r < d; ++r)
+    for (size_t r = 0; r < d && diag; ++r)
         for (size_t c = 0; c < d; ++c) {
             const cdouble& v = m[r * d + c];
-            if (r != c && v != cdouble(0, 0)) diag = false;
-            if (v != (r == c ? cdouble(1, 0) : cdouble(0, 0))) ident = false;
+            if (r != c && v != cdouble(0, 0)) {
+                diag = false;
+                ident = false;
+                break;
+            }
+            if (r == c && v != cdouble(1, 0)) ident = false;
         }
     if (ident) {
         op.kind = OpKind::Identity;
         return op;
     }
     if (diag) {
-        if (kt == 1 && m[0] == cdouble(1, 0)) {
+        if (nt == 1 && m[0] == cdouble(1, 0)) {
             op.kind = OpKind::PhaseOnes;
             op.ctrl_mask |= uint64_t(1) << tgt[0];
             op.targets.clear();
-            op.m = {m[3]};
+            op.m.push_back(m[3]);
             return op;
         }
-        if (kt <= 3) {
+        if (nt <= 3) {
             op.kind = OpKind::Diag;
             for (size_t r = 0; r < d; ++r) op.m.push_back(m[r * d + r]);
             return op;
         }
     }
-    if (kt == 2) {
+    if (nt == 2) {
         const cdouble o(1, 0), z(0, 0);
         const cdouble sw[16] = {o, z, z, z, z, z, o, z, z, o, z, z, z, z, z, o};
-        if (std::equal(m.begin(), m.end(), sw)) {
+        if (std::equal(m, m + 16, sw)) {
             op.kind = OpKind::Swap2;
             return op;
         }
     }
     op.kind = OpKind::Dense;
-    op.m = m;
+    if (d * d > 64 && m == large.data()) {
+        large.resize(d * d);
+        op.m.adopt(std::move(large));
+    } else {
+        op.m.assign(m, d * d);
+    }
     return op;
 }
 

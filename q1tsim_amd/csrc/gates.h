@@ -29,7 +29,8 @@ size_t gate_nbits(const GateSpec& g);
 
 // Gate::matrix() in FP64, row-major 2^k x 2^k, first listed qubit = MSB of
 // the local index (gates.rs:176-183).
-std::vector<cdouble> gate_matrix(const GateSpec& g, const double* params);
+using GateMatrix = InlineVec<cdouble, 16>;
+GateMatrix gate_matrix(const GateSpec& g, const double* params);
 
 // How a gate is applied to the state, found from its matrix alone (the
 // backend only sees Gate::matrix(), as behind the reference's QuState trait).
@@ -37,9 +38,9 @@ enum class OpKind { Identity, Dense, Diag, PhaseOnes, Swap2 };
 
 struct GateOp {
     OpKind kind = OpKind::Dense;
-    std::vector<int> targets;   // index-bit positions p = n-1-q; targets[0] = local MSB
+    InlineVec<int, 4> targets;  // index-bit positions p = n-1-q; targets[0] = local MSB
     uint64_t ctrl_mask = 0;     // index bits that must all be 1 (controls)
-    std::vector<cdouble> m;     // Dense: 2^k x 2^k; Diag: 2^k entries; PhaseOnes: 1 entry
+    InlineVec<cdouble, 4> m;    // Dense: 2^k x 2^k; Diag: 2^k entries; PhaseOnes: 1 entry
     int nctrl() const { return __builtin_popcountll(ctrl_mask); }
 };
 

@@ -68,8 +68,6 @@ struct SweepSample {
 
 struct PendingGate {
     GateOp op;
-    std::vector<cdouble> matrix;  // full FP64 matrix (fused path composes these)
-    std::vector<int> qbits;       // index-bit positions of the listed qubits
 };
 
 // Process-wide cache of freed device blocks.  Requests are rounded up to a
@@ -88,8 +86,9 @@ public:
     // bytes a request of `bytes` takes
     static size_t size_class(size_t bytes);
     void* alloc(size_t bytes, hipStream_t s);
-    // `bytes` as passed to alloc
-    void release(void* p, size_t bytes, hipStream_t s);
+    // `bytes` as passed to alloc; `idle`: no work on the block is in flight
+    // (any stream may take it at once)
+    void release(void* p, size_t bytes, hipStream_t s, bool idle = false);
     void trim();
     // `s` has been synchronised and is about to be destroyed
     void forget_stream(hipStream_t s);
@@ -116,10 +115,25 @@ private:
     std::mutex mu_;
 };
 
-// A HIP stream (default priority, non-blocking) shared by the states of a
-// batch; destroyed with its last user.
+// HIP streams (default priority, non-blocking) kept for reuse, up to
+// kMaxIdle per device: an executed circuit makes a state and drops the last
+// one, and creating and destroying a stream took longer than a small circuit.
+class StreamPool {
+public:
+    static StreamPool& get();
+    hipStream_t take();             // for the current device
+    void give(hipStream_t s, int device);   // synchronises it
+
+private:
+    static constexpr size_t kMaxIdle = 32;
+    std::map<int, std::vector<hipStream_t>> idle_;
+    std::mutex mu_;
+};
+
+// A stream shared by the states of a batch; given back by its last user.
 struct SharedStream {
     hipStream_t s = nullptr;
+    int device = 0;
     SharedStream();
     ~SharedStream();
     SharedStream(const SharedStream&) = delete;

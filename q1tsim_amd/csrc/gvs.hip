@@ -440,7 +440,7 @@ void* DeviceCache::alloc(size_t bytes, hipStream_t s)
     return p;
 }
 
-void DeviceCache::release(void* p, size_t bytes, hipStream_t s)
+void DeviceCache::release(void* p, size_t bytes, hipStream_t s, bool idle)
 {
     if (!p) return;
     const size_t cls = size_class(bytes);
@@ -454,21 +454,67 @@ void DeviceCache::release(void* p, size_t bytes, hipStream_t s)
     // over the cap: free the oldest cached blocks, so the cache follows the
     // sizes in use now (a batch after a large state, c128 after c64)
     evict_to(cap_ - cls);
-    hipEvent_t ev;
-    HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    HIP_OK(hipEventRecord(ev, s));
-    free_[cls].push_back(Entry{p, cls, s, ev, seq_++});
+    hipEvent_t ev = nullptr;
+    if (!idle) {
+        HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        HIP_OK(hipEventRecord(ev, s));
+    }
+    free_[cls].push_back(Entry{p, cls, idle ? nullptr : s, ev, seq_++});
     cached_ += cls;
 }
 
-SharedStream::SharedStream() { HIP_OK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)); }
+// Never destroyed, like the block cache.
+StreamPool& StreamPool::get()
+{
+    static StreamPool* p = new StreamPool();
+    return *p;
+}
+
+hipStream_t StreamPool::take()
+{
+    int dev = 0;
+    HIP_OK(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        std::vector<hipStream_t>& v = idle_[dev];
+        if (!v.empty()) {
+            hipStream_t s = v.back();
+            v.pop_back();
+            return s;
+        }
+    }
+    hipStream_t s = nullptr;
+    HIP_OK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    return s;
+}
+
+void StreamPool::give(hipStream_t s, int device)
+{
+    if (!s) return;
+    // a stream in a failed state is not reused
+    if (hipStreamSynchronize(s) == hipSuccess) {
+        std::lock_guard<std::mutex> lk(mu_);
+        std::vector<hipStream_t>& v = idle_[device];
+        if (v.size() < kMaxIdle) {
+            v.push_back(s);
+            return;
+        }
+    }
+    DeviceCache::get().forget_stream(s);
+    (void)hipStreamDestroy(s);
+}
+
+SharedStream::SharedStream()
+{
+    HIP_OK(hipGetDevice(&device));
+    s = StreamPool::get().take();
+}
 
 SharedStream::~SharedStream()
 {
-    if (s) {
-        (void)hipStreamSynchronize(s);
-        DeviceCache::get().forget_stream(s);
-        (void)hipStreamDestroy(s);
+    try {
+        StreamPool::get().give(s, device);
+    } catch (...) {
     }
 }
 
@@ -485,7 +531,7 @@ GpuVectorState::GpuVectorState(size_t nr_bits, size_t nr_shots, Precision prec, 
         shared_ = std::move(shared);
         stream_ = shared_->s;
     } else {
-        HIP_OK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+        stream_ = StreamPool::get().take();
     }
     geom_ = tile_geometry(prec);
     if (compact_zero) set_zero_state_compact();
@@ -532,9 +578,9 @@ void GpuVectorState::set_jit(int mode)
 
 GpuVectorState::~GpuVectorState()
 {
-    // an own stream is destroyed below, so its work must end first; a shared
-    // stream outlives the state, and the released blocks are event-guarded
-    if (stream_ && !shared_) (void)hipStreamSynchronize(stream_);
+    // the blocks on an own stream are idle once it has ended; a shared stream
+    // outlives the state, and the released blocks are event-guarded
+    const bool idle = stream_ && !shared_ && hipStreamSynchronize(stream_) == hipSuccess;
     try {
         ItemQueuePool::give(std::move(iq_));   // synchronises the queue's last stream
     } catch (...) {
@@ -543,14 +589,14 @@ GpuVectorState::~GpuVectorState()
         DeviceCache& dc = DeviceCache::get();
         for (FlushGraph& fg : fgraphs_) {
             if (fg.exec) (void)hipGraphExecDestroy(fg.exec);
-            dc.release(fg.table, fg.cap, stream_);
+            dc.release(fg.table, fg.cap, stream_, idle);
         }
         fgraphs_.clear();
-        dc.release(amp_, amp_cols_ * dim() * elem_bytes(), stream_);
-        dc.release(d_partial_, partial_cap_ * sizeof(double), stream_);
-        dc.release(d_tree_, tree_cap_ * sizeof(double), stream_);
-        dc.release(d_small_, small_cap_, stream_);
-        for (int s = 0; s < SLOT_COUNT; ++s) dc.release(d_slot_[s], slot_cap_[s], stream_);
+        dc.release(amp_, amp_cols_ * dim() * elem_bytes(), stream_, idle);
+        dc.release(d_partial_, partial_cap_ * sizeof(double), stream_, idle);
+        dc.release(d_tree_, tree_cap_ * sizeof(double), stream_, idle);
+        dc.release(d_small_, small_cap_, stream_, idle);
+        for (int s = 0; s < SLOT_COUNT; ++s) dc.release(d_slot_[s], slot_cap_[s], stream_, idle);
     } catch (...) {
     }
     for (auto& ev : ev_pool_) {
@@ -558,8 +604,10 @@ GpuVectorState::~GpuVectorState()
         (void)hipEventDestroy(ev.second);
     }
     if (stream_ && !shared_) {
-        DeviceCache::get().forget_stream(stream_);
-        (void)hipStreamDestroy(stream_);
+        try {
+            StreamPool::get().give(stream_, device_);
+        } catch (...) {
+        }
     }
 }
 
@@ -766,9 +814,6 @@ void GpuVectorState::apply_gate(const cdouble* mat, size_t nr_affected, const si
     if (nbits > 12) throw Error(ERR_NOT_SUPPORTED, "Gates on more than 12 qubits are not supported");
     PendingGate pg;
     pg.op = analyze_gate(mat, nbits, qbits, nr_bits_);
-    const size_t d = size_t(1) << nbits;
-    pg.matrix.assign(mat, mat + d * d);
-    for (size_t k = 0; k < nbits; ++k) pg.qbits.push_back(int(nr_bits_ - 1 - qbits[k]));
     queue_.push_back(std::move(pg));
 }
 

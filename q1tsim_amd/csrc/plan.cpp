@@ -8,7 +8,6 @@
 //                for the diagonal gates that reach outside the tile.
 #include <algorithm>
 #include <cstring>
-#include <set>
 
 #include "sweep.h"
 
@@ -108,7 +107,7 @@ bool sweepable(const GateOp& op, std::vector<int>* local_targets)
     case OpKind::Swap2:
         // a permutation of two local bits at a phase's write-back
         if (op.ctrl_mask) return false;
-        if (local_targets) *local_targets = op.targets;
+        if (local_targets) local_targets->assign(op.targets.begin(), op.targets.end());
         return true;
     default:
         return false;
@@ -130,9 +129,9 @@ static bool tile_need(const GateOp& op, int fuse_k, uint64_t* need)
         *need = bits;
         return true;
     }
-    std::vector<int> lt;
-    if (!sweepable(op, &lt)) return false;
-    for (int t : lt) *need |= uint64_t(1) << t;
+    if (!sweepable(op, nullptr)) return false;
+    if (op.kind == OpKind::Dense || op.kind == OpKind::Swap2)
+        for (int t : op.targets) *need |= uint64_t(1) << t;
     return true;
 }
 
@@ -192,6 +191,7 @@ std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const
     std::vector<PlanStep> steps;
     std::vector<size_t> rem;
     std::vector<GateBits> gb(q.size());
+    std::vector<char> done(q.size(), 0);
     for (size_t i = 0; i < q.size(); ++i) {
         gb[i].touched = touched_bits(q[i].op);
         gb[i].nd = nondiag_bits(q[i].op);
@@ -213,6 +213,7 @@ std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const
         std::vector<size_t> sel;
         for (size_t i : rem) {
             const GateBits& b = gb[i];
+            if (blk.nd == all) break;   // no later gate can pass
             if (blk.blocks(b.touched, b.nd) || !b.ok) {
                 blk.add(b.touched, b.nd);
                 continue;
@@ -272,11 +273,8 @@ std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const
             steps.push_back(st);
         }
         // drop the consumed gates, keeping the original order of the rest
-        const std::set<size_t> done(steps.back().gates.begin(), steps.back().gates.end());
-        std::vector<size_t> next;
-        for (size_t i : rem)
-            if (!done.count(i)) next.push_back(i);
-        rem.swap(next);
+        for (size_t i : steps.back().gates) done[i] = 1;
+        rem.erase(std::remove_if(rem.begin(), rem.end(), [&](size_t i) { return done[i] != 0; }), rem.end());
     }
     return steps;
 }

@@ -220,7 +220,7 @@ class GpuVectorState:
         return [int(out[i]) for i in range(n)]
 
     def column(self, col):
-        out = np.zeros(1 << self.nr_bits, dtype=np.complex128)
+        out = np.empty(1 << self.nr_bits, dtype=np.complex128)
         check(lib().q1t_gvs_read_amplitudes(self.h, col, _dptr(out), len(out)))
         return out
 

@@ -318,7 +318,7 @@ class Circuit(object):
 
     def amplitudes(self, col=0):
         n = self.nr_qbits()
-        out = np.zeros(1 << n, dtype=np.complex128)
+        out = np.empty(1 << n, dtype=np.complex128)
         _lib.check(self.__sim.q1t_circuit_read_amplitudes(
             self.__ptr, col, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), 1 << n))
         return out
