@@ -146,9 +146,9 @@ int q1t_gvs_flush(q1t_gvs* s);
  * 2..6 composes gate runs into dense k-qubit blocks; tiling = 1 applies
  * runs that fit an LDS tile in one HBM sweep. */
 int q1t_gvs_set_plan(q1t_gvs* s, int fusion_k, int tiling);
-/* Build-added: local search of the sweep tiles and register phases;
- * mode -1 (default) for states of 512 MiB and more, 0 never, 1 always.
- * Changes only the schedule, not the gates applied. */
+/* Build-added: local search of the sweep tiles and register phases; mode -1
+ * (default) tiles always and phases for states of 512 MiB and more, 0 never,
+ * 1 always.  Changes only the schedule, not the gates applied. */
 int q1t_gvs_set_plan_search(q1t_gvs* s, int mode);
 /* Build-added, no counterpart in the reference: flush graphs (on = 1).  The
  * kernel launches of a planned flush are captured into one hipGraph; a later

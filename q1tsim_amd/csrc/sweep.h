@@ -30,8 +30,8 @@ bool sweepable(const GateOp& op, std::vector<int>* local_targets);
 // bits always included); a gate may run before earlier gates it commutes
 // with.  With fuse_k > 0 the non-diagonal gates need all their bits in the
 // tile.  `search`: refine each greedy tile (and, in the programs below, each
-// phase's register bits) by local search -- host time that pays once a
-// sweep moves hundreds of MB (GpuVectorState::plan_search).
+// phase's register bits) by local search (GpuVectorState::tile_search,
+// phase_search).
 std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const TileGeom& g, int fuse_k,
                                  bool search = true);
 

@@ -356,20 +356,19 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
     const int n = int(st.nr_bits());
     const TileGeom g = st.geometry();
     const int prec = int(st.precision());
-    const bool search = st.plan_search(state_bytes);
+    const bool search = st.tile_search(), phase_search = st.phase_search(state_bytes);
     const bool factors = st.tile_factors();   // specialised kernels only
     auto build_all = [&](const std::vector<PlanStep>& ss, int kind) {
         std::vector<SweepProgram> out(ss.size());
         for (size_t s = 0; s < ss.size(); ++s)
-            if (ss[s].sweep) out[s] = build_candidate(queue, ss[s], g, kind, search, factors);
+            if (ss[s].sweep) out[s] = build_candidate(queue, ss[s], g, kind, phase_search, factors);
         return out;
     };
     const bool fused = st.precision() == PREC_C64 && fusion_k > 0;
     // A flush with the previous flush's gate structure (a repeated circuit,
     // new angles allowed) takes that flush's steps and per-sweep program
     // kinds and builds only those programs: the tile searches (and the
-    // learned planner's candidates) are most of the planning time.  Kept for
-    // states the tile search runs on.
+    // learned planner's candidates) are most of the planning time.
     std::vector<uint64_t> key;
     auto cache_hit = [&](std::vector<int>& kind) {
         const std::shared_ptr<void>& cached = st.plan_cache_steps();
@@ -433,7 +432,7 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
         if (cache_hit(kind)) {
             progs.assign(steps.size(), SweepProgram{});
             for (size_t s = 0; s < steps.size(); ++s)
-                if (steps[s].sweep) progs[s] = build_candidate(queue, steps[s], g, kind[s], search, factors);
+                if (steps[s].sweep) progs[s] = build_candidate(queue, steps[s], g, kind[s], phase_search, factors);
             return;
         }
     }
@@ -484,7 +483,7 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
             try {
                 for (size_t i = next++; i < work.size(); i = next++) {
                     const auto& w = work[i];
-                    cand[w[0]][w[1]][w[2]] = build_candidate(queue, tl[w[0]][w[1]], g, kinds[w[2]], search, factors);
+                    cand[w[0]][w[1]][w[2]] = build_candidate(queue, tl[w[0]][w[1]], g, kinds[w[2]], phase_search, factors);
                 }
             } catch (...) {
                 std::lock_guard<std::mutex> lk(err_mu);
@@ -976,8 +975,10 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             }
             return;
         }
-        const bool search = live[i]->plan_search(S);
-        p.steps = plan_gates(q, n, g, K, search);
+        const bool search = live[i]->phase_search(S);
+        // complex64: the greedy tiles, whose order of the gates' rounding a
+        // seeded batch's outcomes depend on
+        p.steps = plan_gates(q, n, g, K, prec == PREC_C128 ? live[i]->tile_search() : search);
         p.ph.resize(p.steps.size());
         p.ops.resize(p.steps.size());
         int nblocks = 0;
