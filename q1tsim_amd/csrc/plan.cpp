@@ -824,7 +824,10 @@ void build_whole(const std::vector<PendingGate>& q, const PlanStep& step, int M,
         w.cr = o.cr;
         w.ct = o.ct;
         if (o.type == SW_DENSE1) {
-            w.code = o.aux == SWF_REAL ? uint32_t(SWF_REAL_SEQ) : o.aux == SWF_RX ? uint32_t(SWF_RX_SEQ) : o.aux;
+            // X, CX and Y by their matrices, as in the interpreted sweeps
+            w.code = o.aux == SWF_REAL || o.aux == SWF_SWAP ? uint32_t(SWF_REAL_SEQ)
+                     : o.aux == SWF_RX                      ? uint32_t(SWF_RX_SEQ)
+                                                            : uint32_t(SWF_GENERAL);
             w.code |= uint32_t(o.reg) << 8;
         } else if (o.type == SW_PHASE) {
             w.code = kWholePhase + o.aux;

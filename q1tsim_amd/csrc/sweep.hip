@@ -155,6 +155,17 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
     return first;
 }
 
+// A program's ops as the interpreter kernels take them: X, CX and Y by their
+// matrices (0, 1 and +-i are exact factors).
+static void interpreter_ops(SwOp* ops, size_t n)
+{
+    for (size_t i = 0; i < n; ++i) {
+        if (ops[i].type != SW_DENSE1) continue;
+        if (ops[i].aux == SWF_SWAP) ops[i].aux = SWF_REAL;
+        else if (ops[i].aux == SWF_Y) ops[i].aux = SWF_GENERAL;
+    }
+}
+
 // The widest fused dense block of a program, as the kernels' BLK: 0 none,
 // 1 blocks of 3 and 4 qubits, 2 wider ones.
 static int block_level(const std::vector<SwPhase>& phases)
@@ -175,11 +186,9 @@ __device__ __forceinline__ void whole_dense(uint32_t form, int reg, V (&v)[NR], 
                                             V m1, V m2, V m3)
 {
     switch (form) {
-    case SWF_REAL_SEQ: dense_ctl<V, NR, R, SWF_REAL_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_SWAP: dense_ctl<V, NR, R, SWF_SWAP>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_RX_SEQ: dense_ctl<V, NR, R, SWF_RX_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_Y: dense_ctl<V, NR, R, SWF_Y>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    default: dense_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_REAL_SEQ: interp_ctl<V, NR, R, SWF_REAL_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_RX_SEQ: interp_ctl<V, NR, R, SWF_RX_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    default: interp_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
     }
 }
 
@@ -242,7 +251,8 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
                 const V m2 = mkc<V>(op.m[4], op.m[5]), m3 = mkc<V>(op.m[6], op.m[7]);
                 whole_dense<V, NR, R>(body, reg, v, cr, ct, tok, m0, m1, m2, m3);
             } else if (body < kWholeDiagReg) {
-                phase_op<V, NR>(body - kWholePhase, v, cr, ct, tok, m0);
+                const V f = sel(tok, m0, mkc<V>(1, 0));
+                scale_regs<V, NR>(v, cr, 0u, tok, [&](int, V x) { return cmul(f, x); });
             } else if (body == kWholeDiagReg) {
                 scale_regs<V, NR>(v, cr, ct, tok, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, m1, m0), x); });
             } else {
@@ -773,6 +783,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             if (ph.kind == 1) ph.op_begin += uint32_t(boff_s[s]);
         std::memcpy(host + poff[s], progs[s].phases.data(), progs[s].phases.size() * sizeof(SwPhase));
         std::memcpy(host + ooff[s], progs[s].ops.data(), progs[s].ops.size() * sizeof(SwOp));
+        if (!st.jit_enabled()) interpreter_ops(reinterpret_cast<SwOp*>(host + ooff[s]), progs[s].ops.size());
         if (!progs[s].blocks.empty())
             std::memcpy(host + boff + boff_s[s] * sizeof(float), progs[s].blocks.data(),
                         progs[s].blocks.size() * sizeof(float));
@@ -1157,6 +1168,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
                         if (ph[j].kind == 1) ph[j].op_begin += uint32_t(bbase[i]);
                     }
                     std::memcpy(host + p.ooff[s], p.ops[s].data(), p.ops[s].size() * sizeof(SwOp));
+                    interpreter_ops(reinterpret_cast<SwOp*>(host + p.ooff[s]), p.ops[s].size());
                     SweepItem it;
                     std::memset(&it, 0, sizeof(it));
                     it.amp = st.col_ptr(0);

@@ -209,16 +209,41 @@ __device__ __forceinline__ void dense_ctl(int reg, V (&v)[NR], uint32_t cr, uint
     }
 }
 
+// The interpreter's dense bodies.  Three forms only (general, real, RX: the
+// planner gives X, CX and Y ops their matrices, interpreter_ops): every body
+// writes its results where its inputs were, so the register array is not
+// copied at the joins of the dispatch.  Thread controls select the
+// coefficients (the identity's where the lane's controls are not set) instead
+// of the results: 4 to 8 selects per op instead of 4 per pair.
+template <typename V, int NR, int R, int FORM, bool RC>
+__device__ __forceinline__ void interp_reg(int reg, V (&v)[NR], uint32_t cr, V m0, V m1, V m2, V m3)
+{
+    dense_reg<V, NR, R, FORM, false, RC>(reg, v, cr, true, m0, m1, m2, m3);
+}
+template <typename V, int NR, int R, int FORM>
+__device__ __forceinline__ void interp_ctl(int reg, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, V m0, V m1, V m2,
+                                           V m3)
+{
+    if (ct) {
+        const V one = mkc<V>(1, 0), zero = mkc<V>(0, 0);
+        m0 = sel(tok, m0, one);
+        m1 = sel(tok, m1, zero);
+        m2 = sel(tok, m2, zero);
+        m3 = sel(tok, m3, one);
+        interp_reg<V, NR, R, FORM, true>(reg, v, cr, m0, m1, m2, m3);
+        return;
+    }
+    if (cr) interp_reg<V, NR, R, FORM, true>(reg, v, cr, m0, m1, m2, m3);
+    else interp_reg<V, NR, R, FORM, false>(reg, v, cr, m0, m1, m2, m3);
+}
 template <typename V, int NR, int R>
 __device__ __forceinline__ void dense_form_dispatch(uint32_t form, int reg, V (&v)[NR], uint32_t cr, uint32_t ct,
                                                     bool tok, V m0, V m1, V m2, V m3)
 {
     switch (form) {
-    case SWF_REAL: dense_ctl<V, NR, R, SWF_REAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_SWAP: dense_ctl<V, NR, R, SWF_SWAP>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_RX: dense_ctl<V, NR, R, SWF_RX>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_Y: dense_ctl<V, NR, R, SWF_Y>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    default: dense_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_REAL: interp_ctl<V, NR, R, SWF_REAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    case SWF_RX: interp_ctl<V, NR, R, SWF_RX>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
+    default: interp_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
     }
 }
 
@@ -593,7 +618,9 @@ __device__ __forceinline__ void tile_phases(V* __restrict__ a, const SweepArgs& 
                     const V m0 = opm<V>(op, 0), m1 = opm<V>(op, 1), m2 = opm<V>(op, 2), m3 = opm<V>(op, 3);
                     dense_form_dispatch<V, NR, R>(op.aux, op.reg, v, cr, ct, tok, m0, m1, m2, m3);
                 } else if (op.type == SW_PHASE) {
-                    phase_op<V, NR>(op.aux, v, cr, ct, tok, opm<V>(op, 0));
+                    // a factor of +-1, +-i is an exact one
+                    const V f = sel(tok, opm<V>(op, 0), mkc<V>(1, 0));
+                    scale_regs<V, NR>(v, cr, 0u, tok, [&](int, V x) { return cmul(f, x); });
                 } else {  // SW_DIAG1
                     const V d0 = opm<V>(op, 0), d1 = opm<V>(op, 1);
                     diag_op<V, NR>(op, v, cr, ct, tok, base, tid, d0, d1);
