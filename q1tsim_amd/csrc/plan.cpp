@@ -761,6 +761,32 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
     append_factors(tf, M, phases, ops, order);
 }
 
+template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq)
+{
+    InterpOpT<R> w;
+    std::memset(&w, 0, sizeof(w));
+    w.ctl = o.cr | o.ct << 16;
+    w.co = o.co;
+    if (o.type == SW_DENSE1) {
+        if (o.aux == SWF_REAL || o.aux == SWF_SWAP) w.code = seq ? SWF_REAL_SEQ : SWF_REAL;
+        else if (o.aux == SWF_RX) w.code = seq ? SWF_RX_SEQ : SWF_RX;
+        else w.code = SWF_GENERAL;
+        w.code |= uint32_t(o.reg) << 8;
+    } else if (o.type == SW_PHASE) {
+        w.code = kInterpPhase;
+    } else if (o.dreg >= 0) {
+        w.code = kInterpDiagReg | uint32_t(o.dreg) << 8;
+    } else if (o.dtid >= 0) {
+        w.code = kInterpDiagTid | uint32_t(o.dtid) << 16;
+    } else {
+        w.code = kInterpDiagOuter | uint32_t(o.dglobal) << 16;
+    }
+    for (int k = 0; k < 8; ++k) w.m[k] = R(o.m[k]);
+    return w;
+}
+template InterpOpT<double> interp_op<double>(const SwOp&, bool);
+template InterpOpT<float> interp_op<float>(const SwOp&, bool);
+
 std::vector<PlanStep> plan_whole(const std::vector<PendingGate>& q, int M)
 {
     std::vector<PlanStep> steps;
@@ -787,7 +813,7 @@ std::vector<PlanStep> plan_whole(const std::vector<PendingGate>& q, int M)
 
 template <typename R>
 void build_whole(const std::vector<PendingGate>& q, const PlanStep& step, int M, int nr, std::vector<WholePhase>& phases,
-                 std::vector<WholeOpT<R>>& ops)
+                 std::vector<InterpOpT<R>>& ops)
 {
     const LocalMap lm(step.tile);
     std::vector<size_t> pending = step.gates;
@@ -818,32 +844,12 @@ void build_whole(const std::vector<PendingGate>& q, const PlanStep& step, int M,
         }
         phases.push_back(w);
     }
-    for (const SwOp& o : so) {
-        WholeOpT<R> w;
-        std::memset(&w, 0, sizeof(w));
-        w.cr = o.cr;
-        w.ct = o.ct;
-        if (o.type == SW_DENSE1) {
-            // X, CX and Y by their matrices, as in the interpreted sweeps
-            w.code = o.aux == SWF_REAL || o.aux == SWF_SWAP ? uint32_t(SWF_REAL_SEQ)
-                     : o.aux == SWF_RX                      ? uint32_t(SWF_RX_SEQ)
-                                                            : uint32_t(SWF_GENERAL);
-            w.code |= uint32_t(o.reg) << 8;
-        } else if (o.type == SW_PHASE) {
-            w.code = kWholePhase + o.aux;
-        } else if (o.dreg >= 0) {
-            w.code = kWholeDiagReg | uint32_t(o.dreg) << 8;
-        } else {
-            w.code = kWholeDiagTid | uint32_t(o.dtid) << 16;
-        }
-        for (int k = 0; k < 8; ++k) w.m[k] = R(o.m[k]);
-        ops.push_back(w);
-    }
+    for (const SwOp& o : so) ops.push_back(interp_op<R>(o, true));
 }
 template void build_whole<double>(const std::vector<PendingGate>&, const PlanStep&, int, int, std::vector<WholePhase>&,
-                                  std::vector<WholeOpT<double>>&);
+                                  std::vector<InterpOpT<double>>&);
 template void build_whole<float>(const std::vector<PendingGate>&, const PlanStep&, int, int, std::vector<WholePhase>&,
-                                 std::vector<WholeOpT<float>>&);
+                                 std::vector<InterpOpT<float>>&);
 
 std::vector<size_t> plan_order(const std::vector<PendingGate>& q, int n, const TileGeom& g, bool search)
 {

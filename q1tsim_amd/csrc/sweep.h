@@ -50,6 +50,9 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
                    std::vector<SwPhase>& phases, std::vector<SwOp>& ops, bool search = true,
                    std::vector<size_t>* order = nullptr, bool factors = false);
 
+// An op as the interpreting kernels take it; `seq`: whole-state programs.
+template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq);
+
 // States too small for tiles (below M+2 qubits) run whole in LDS, one
 // workgroup per column: runs of gates that a register phase takes are one
 // step (its tile: all M bits, M >= 3 bits whatever the state), others run on
@@ -60,7 +63,7 @@ std::vector<PlanStep> plan_whole(const std::vector<PendingGate>& q, int M);
 // from the step's first op.
 template <typename R>
 void build_whole(const std::vector<PendingGate>& q, const PlanStep& step, int M, int nr, std::vector<WholePhase>& phases,
-                 std::vector<WholeOpT<R>>& ops);
+                 std::vector<InterpOpT<R>>& ops);
 
 // The order in which the plain (per-gate) plan of the specialised kernels
 // applies the queue's gates (identity gates, which never run, are left out;

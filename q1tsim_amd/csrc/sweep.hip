@@ -39,6 +39,12 @@ namespace q1t {
                         std::string("HIP error in " #expr ": ") + hipGetErrorString(e_));          \
     } while (0)
 
+template <typename V> __device__ __forceinline__ void warm_sweep(const SweepArgs& sa)
+{
+    warm_program(sa.phases, uint32_t(sa.nphases) * uint32_t(sizeof(SwPhase)));
+    if (sa.nops) warm_program(sa.ops, sa.nops * uint32_t(sizeof(InterpOpT<typename RealOf<V>::type>)));
+}
+
 template <typename V, int M, int R, int SW, int BLK>
 __global__ void __launch_bounds__(1 << (M - R))
 __attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 && M == 12 ? (R == 3 ? 4 : 3) : 2)))
@@ -46,6 +52,7 @@ k_sweep(V* __restrict__ amp, uint64_t col_stride, SweepArgs sa)
 {
     __shared__ V lds[1 << M];
     V* a = amp + uint64_t(blockIdx.y) * col_stride;
+    warm_sweep<V>(sa);
     for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK>(a, sa, tile, lds);
 }
 
@@ -82,6 +89,7 @@ k_sweep_batched(const SweepItem* __restrict__ items, int nitems, uint64_t total_
             if (items[mid].first_tile <= t0) lo = mid;
             else hi = mid - 1;
         }
+        warm_sweep<V>(items[lo].sa);
         for (uint64_t t = t0; t < t1; ++t) {
             while (lo + 1 < nitems && items[lo + 1].first_tile <= t) ++lo;
             const SweepItem& it = items[lo];
@@ -106,7 +114,7 @@ static void launch_batched_c64(int blk, unsigned gx, hipStream_t stream, const S
 
 template <typename V, int M, int R, int SW>
 static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase* dphases, int nphases,
-                         const SwOp* dops, const float* dblocks, size_t cb, size_t ce, int blk,
+                         const SwOp* dops, int nops, const float* dblocks, size_t cb, size_t ce, int blk,
                          hipFunction_t jit = nullptr)
 {
     const int n = int(st.nr_bits());
@@ -121,6 +129,7 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
     sa.ops = dops;
     sa.blocks = dblocks;
     sa.nphases = nphases;
+    sa.nops = uint32_t(nops);
     const uint64_t dim = uint64_t(1) << n;
     const unsigned gx = unsigned(std::min<uint64_t>(sa.ntiles, 2048));
     int first = -1;
@@ -155,14 +164,20 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
     return first;
 }
 
-// A program's ops as the interpreter kernels take them: X, CX and Y by their
-// matrices (0, 1 and +-i are exact factors).
-static void interpreter_ops(SwOp* ops, size_t n)
+// Bytes of a program's ops as its kernel reads them, and the ops written so.
+static size_t op_bytes(Precision prec, bool jit)
 {
-    for (size_t i = 0; i < n; ++i) {
-        if (ops[i].type != SW_DENSE1) continue;
-        if (ops[i].aux == SWF_SWAP) ops[i].aux = SWF_REAL;
-        else if (ops[i].aux == SWF_Y) ops[i].aux = SWF_GENERAL;
+    return jit ? sizeof(SwOp) : prec == PREC_C128 ? sizeof(InterpOpT<double>) : sizeof(InterpOpT<float>);
+}
+static void put_ops(char* to, const std::vector<SwOp>& ops, Precision prec, bool jit)
+{
+    if (jit) {
+        std::memcpy(to, ops.data(), ops.size() * sizeof(SwOp));
+        return;
+    }
+    for (size_t i = 0; i < ops.size(); ++i) {
+        if (prec == PREC_C128) reinterpret_cast<InterpOpT<double>*>(to)[i] = interp_op<double>(ops[i], false);
+        else reinterpret_cast<InterpOpT<float>*>(to)[i] = interp_op<float>(ops[i], false);
     }
 }
 
@@ -181,17 +196,6 @@ static int block_level(const std::vector<SwPhase>& phases)
 constexpr int whole_regs(int n) { return n <= 13 ? 3 : 4; }   // register bits: at most 1024 threads
 static int whole_bits(int n) { return std::max(n, whole_regs(n)); }
 
-template <typename V, int NR, int R>
-__device__ __forceinline__ void whole_dense(uint32_t form, int reg, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, V m0,
-                                            V m1, V m2, V m3)
-{
-    switch (form) {
-    case SWF_REAL_SEQ: interp_ctl<V, NR, R, SWF_REAL_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_RX_SEQ: interp_ctl<V, NR, R, SWF_RX_SEQ>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    default: interp_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    }
-}
-
 // One column of up to 2^14 amplitudes per workgroup, in LDS from its load to
 // its store: 2^R amplitudes per thread in registers, the program's register
 // phases as in the tile sweeps, one LDS exchange and barrier per phase.  Bound
@@ -205,7 +209,7 @@ __device__ __forceinline__ void whole_dense(uint32_t form, int reg, V (&v)[NR], 
 template <typename V, int R>
 __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ items,
                                                 const WholePhase* __restrict__ phases,
-                                                const WholeOpT<typename RealOf<V>::type>* __restrict__ ops)
+                                                const InterpOpT<typename RealOf<V>::type>* __restrict__ ops)
 {
     constexpr int NR = 1 << R;
     extern __shared__ unsigned char smem_whole[];
@@ -213,6 +217,9 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
     const WholeItem it = load_uniform(items, blockIdx.x);
     const int M = int(it.n) > R ? int(it.n) : R, sw = sweep_swizzle_bits(M);
     const uint32_t nth = 1u << (M - R), N = 1u << it.n, tid = threadIdx.x;
+    const uint32_t nops = it.nphases ? load_uniform(phases, it.phases + it.nphases - 1).op_end : 0u;
+    if (it.nphases) warm_program(phases + it.phases, it.nphases * uint32_t(sizeof(WholePhase)));
+    if (nops) warm_program(ops + it.ops, nops * uint32_t(sizeof(InterpOpT<typename RealOf<V>::type>)));
     if (tid >= nth) return;
     V* a = static_cast<V*>(it.amp);
     {
@@ -238,27 +245,12 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
         for (int k = 0; k < NR; ++k) v[k] = s[tin ^ (ph.slot[k] & 0xffffu)];
         const uint32_t o1 = it.ops + ph.op_end;
         uint32_t oi = it.ops + ph.op_begin;
-        WholeOpT<typename RealOf<V>::type> nxt = load_uniform(ops, oi);   // the table ends with a spare record
+        InterpOpT<typename RealOf<V>::type> nxt = load_uniform(ops, oi);   // the table ends with a spare record
         while (oi < o1) {
-            const WholeOpT<typename RealOf<V>::type> op = nxt;
+            const InterpOpT<typename RealOf<V>::type> op = nxt;
             ++oi;
             nxt = load_uniform(ops, oi);
-            const uint32_t body = op.code & 0xffu, cr = op.cr, ct = op.ct;
-            const int reg = int((op.code >> 8) & 0xffu);
-            const bool tok = (tid & ct) == ct;
-            const V m0 = mkc<V>(op.m[0], op.m[1]), m1 = mkc<V>(op.m[2], op.m[3]);
-            if (body < kWholePhase) {
-                const V m2 = mkc<V>(op.m[4], op.m[5]), m3 = mkc<V>(op.m[6], op.m[7]);
-                whole_dense<V, NR, R>(body, reg, v, cr, ct, tok, m0, m1, m2, m3);
-            } else if (body < kWholeDiagReg) {
-                const V f = sel(tok, m0, mkc<V>(1, 0));
-                scale_regs<V, NR>(v, cr, 0u, tok, [&](int, V x) { return cmul(f, x); });
-            } else if (body == kWholeDiagReg) {
-                scale_regs<V, NR>(v, cr, ct, tok, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, m1, m0), x); });
-            } else {
-                const V d = sel(((tid >> (op.code >> 16)) & 1) != 0, m1, m0);
-                scale_regs<V, NR>(v, cr, ct, tok, [&](int, V x) { return cmul(d, x); });
-            }
+            interp_op<V, NR, R, true>(op, v, tid, 0);
         }
         if (ph.wmap == 0) {
 #pragma unroll
@@ -281,7 +273,7 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
 // the widest).  Tables in device memory; the op table ends with a spare record.
 template <typename V>
 static void launch_whole(int n_max, const WholeItem* items, size_t nitems, const WholePhase* phases,
-                         const WholeOpT<typename RealOf<V>::type>* ops, hipStream_t stream)
+                         const InterpOpT<typename RealOf<V>::type>* ops, hipStream_t stream)
 {
     const int R = whole_regs(n_max), M = whole_bits(n_max);
     const size_t lds = sizeof(V) << M;
@@ -302,7 +294,7 @@ static void launch_whole(int n_max, const WholeItem* items, size_t nitems, const
 // `ops` (records of one step: phases [ph0[s], ph0[s] + nph[s]), ops from op0[s]).
 template <typename R> struct WholeTables {
     std::vector<WholePhase> phases;
-    std::vector<WholeOpT<R>> ops;
+    std::vector<InterpOpT<R>> ops;
     std::vector<uint32_t> ph0, nph, op0;
     void build(const std::vector<PendingGate>& q, const std::vector<PlanStep>& steps, int n)
     {
@@ -312,7 +304,7 @@ template <typename R> struct WholeTables {
         for (size_t s = 0; s < steps.size(); ++s) {
             if (!steps[s].sweep) continue;
             std::vector<WholePhase> p;
-            std::vector<WholeOpT<R>> o;
+            std::vector<InterpOpT<R>> o;
             build_whole<R>(q, steps[s], whole_bits(n), whole_regs(n), p, o);
             ph0[s] = uint32_t(phases.size());
             nph[s] = uint32_t(p.size());
@@ -693,14 +685,14 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
     const std::vector<PlanStep> steps = plan_whole(queue, whole_bits(n));
     WholeTables<R> wt;
     wt.build(queue, steps, n);
-    wt.ops.push_back(WholeOpT<R>{});   // the spare record
+    wt.ops.push_back(InterpOpT<R>{});   // the spare record
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
     const size_t ooff = up(wt.phases.size() * sizeof(WholePhase));
-    const size_t ioff = up(ooff + wt.ops.size() * sizeof(WholeOpT<R>));
+    const size_t ioff = up(ooff + wt.ops.size() * sizeof(InterpOpT<R>));
     const size_t total = up(ioff + steps.size() * ncols * sizeof(WholeItem));
     char* const host = st.stage(total);
     std::memcpy(host, wt.phases.data(), wt.phases.size() * sizeof(WholePhase));
-    std::memcpy(host + ooff, wt.ops.data(), wt.ops.size() * sizeof(WholeOpT<R>));
+    std::memcpy(host + ooff, wt.ops.data(), wt.ops.size() * sizeof(InterpOpT<R>));
     WholeItem* items = reinterpret_cast<WholeItem*>(host + ioff);   // step-major
     for (size_t s = 0; s < steps.size(); ++s)
         for (size_t c = 0; c < ncols; ++c)
@@ -715,7 +707,7 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
             const int ps = st.prof_begin();
             launch_whole<V>(n, reinterpret_cast<const WholeItem*>(d + ioff) + s * ncols, ncols,
                             reinterpret_cast<const WholePhase*>(d),
-                            reinterpret_cast<const WholeOpT<R>*>(d + ooff), st.stream());
+                            reinterpret_cast<const InterpOpT<R>*>(d + ooff), st.stream());
             st.prof_end(ps, sizeof(V) == 16 ? "k_whole_c128" : "k_whole_c64", 2.0 * S);
             stats.launches += 1;
             stats.sweeps += 1;
@@ -768,7 +760,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         poff[s] = total;
         total += (progs[s].phases.size() * sizeof(SwPhase) + 255) / 256 * 256;
         ooff[s] = total;
-        total += (progs[s].ops.size() * sizeof(SwOp) + 255) / 256 * 256;
+        total += (progs[s].ops.size() * op_bytes(st.precision(), st.jit_enabled()) + 255) / 256 * 256;
         boff_s[s] = nblk_floats;
         nblk_floats += progs[s].blocks.size();
         nblocks += progs[s].nblocks;
@@ -782,8 +774,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         for (SwPhase& ph : progs[s].phases)
             if (ph.kind == 1) ph.op_begin += uint32_t(boff_s[s]);
         std::memcpy(host + poff[s], progs[s].phases.data(), progs[s].phases.size() * sizeof(SwPhase));
-        std::memcpy(host + ooff[s], progs[s].ops.data(), progs[s].ops.size() * sizeof(SwOp));
-        if (!st.jit_enabled()) interpreter_ops(reinterpret_cast<SwOp*>(host + ooff[s]), progs[s].ops.size());
+        put_ops(host + ooff[s], progs[s].ops, st.precision(), st.jit_enabled());
         if (!progs[s].blocks.empty())
             std::memcpy(host + boff + boff_s[s] * sizeof(float), progs[s].blocks.data(),
                         progs[s].blocks.size() * sizeof(float));
@@ -825,15 +816,15 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             const int shape = g.M * 16 + g.R;
             if (st.precision() == PREC_C128) {
                 switch (shape) {
-                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, dblocks, col_begin, col_end, 0, jf); break;
-                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, dblocks, col_begin, col_end, 0, jf); break;
+                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, jf); break;
+                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, jf); break;
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex128 tile shape");
                 }
             } else {
                 switch (shape) {
-                case 13 * 16 + 4: slot = launch_sweep<float2, 13, 4, 5>(st, step, dp, np, dop, dblocks, col_begin, col_end, blk, jf); break;
-                case 12 * 16 + 3: slot = launch_sweep<float2, 12, 3, 4>(st, step, dp, np, dop, dblocks, col_begin, col_end, blk, jf); break;
-                case 12 * 16 + 4: slot = launch_sweep<float2, 12, 4, 4>(st, step, dp, np, dop, dblocks, col_begin, col_end, blk, jf); break;
+                case 13 * 16 + 4: slot = launch_sweep<float2, 13, 4, 5>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
+                case 12 * 16 + 3: slot = launch_sweep<float2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
+                case 12 * 16 + 4: slot = launch_sweep<float2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex64 tile shape");
                 }
             }
@@ -1033,7 +1024,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
     // per small state's column.  Offsets first
     // (serial arithmetic), then the states fill their parts in parallel.
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-    const size_t wop_bytes = prec == PREC_C128 ? sizeof(WholeOpT<double>) : sizeof(WholeOpT<float>);
+    const size_t wop_bytes = prec == PREC_C128 ? sizeof(InterpOpT<double>) : sizeof(InterpOpT<float>);
     size_t off = 0, max_steps = 0, nblock_floats = 0, nwph = 0, nwops = 0;
     std::vector<size_t> bbase(live.size(), 0), wpbase(live.size(), 0), wobase(live.size(), 0);
     for (size_t i = 0; i < live.size(); ++i) {
@@ -1058,7 +1049,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             p.poff[s] = off;
             off = up(off + p.ph[s].size() * sizeof(SwPhase));
             p.ooff[s] = off;
-            off = up(off + p.ops[s].size() * sizeof(SwOp));
+            off = up(off + p.ops[s].size() * op_bytes(prec, false));
             p.nph[s] = int(p.ph[s].size());
         }
     }
@@ -1167,8 +1158,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
                         ph[j] = p.ph[s][j];
                         if (ph[j].kind == 1) ph[j].op_begin += uint32_t(bbase[i]);
                     }
-                    std::memcpy(host + p.ooff[s], p.ops[s].data(), p.ops[s].size() * sizeof(SwOp));
-                    interpreter_ops(reinterpret_cast<SwOp*>(host + p.ooff[s]), p.ops[s].size());
+                    put_ops(host + p.ooff[s], p.ops[s], prec, false);
                     SweepItem it;
                     std::memset(&it, 0, sizeof(it));
                     it.amp = st.col_ptr(0);
@@ -1186,6 +1176,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
                     it.sa.ops = reinterpret_cast<const SwOp*>(dbase + p.ooff[s]);
                     it.sa.blocks = reinterpret_cast<const float*>(dbase + boff);
                     it.sa.nphases = p.nph[s];
+                    it.sa.nops = uint32_t(p.ops[s].size());
                     std::memcpy(host + items_off + item_idx[s][i] * sizeof(SweepItem), &it, sizeof(it));
                 }
             }
@@ -1214,10 +1205,10 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             const WholePhase* wp = reinterpret_cast<const WholePhase*>(dbase + wpoff);
             if (prec == PREC_C128)
                 launch_whole<double2>(wg.n_max, wi, wg.count, wp,
-                                      reinterpret_cast<const WholeOpT<double>*>(dbase + wooff), stream);
+                                      reinterpret_cast<const InterpOpT<double>*>(dbase + wooff), stream);
             else
                 launch_whole<float2>(wg.n_max, wi, wg.count, wp,
-                                     reinterpret_cast<const WholeOpT<float>*>(dbase + wooff), stream);
+                                     reinterpret_cast<const InterpOpT<float>*>(dbase + wooff), stream);
             agg.launches += 1;
         }
         if (!round_items[r].second) continue;

@@ -17,6 +17,7 @@ struct SweepArgs {
     const SwOp* ops;
     const float* blocks;   // real-embedded block matrices (fused segments)
     int nphases;
+    uint32_t nops;
 };
 
 // p[i] read through the constant address space: wave-uniform scalar loads
@@ -45,16 +46,35 @@ template <> __device__ __forceinline__ float2 opm<float2>(const SwOp& op, int k)
 // Makes every field the op bodies read live at this point, so the op's
 // scalar loads issue together and the op waits once for them (else the mask
 // test's load is waited for first and the rest loaded after the branch).
-template <typename V> __device__ __forceinline__ void pin_op(const SwOp& op)
+template <typename R> __device__ __forceinline__ void pin_op(const InterpOpT<R>& op)
 {
-    asm volatile("" ::"s"(op.type), "s"(op.reg), "s"(op.dreg), "s"(op.dtid), "s"(op.dglobal), "s"(op.cr),
-                 "s"(op.ct), "s"(op.aux), "s"(op.co));
-    if constexpr (sizeof(V) == 8)
-        asm volatile("" ::"s"(op.mf[0]), "s"(op.mf[1]), "s"(op.mf[2]), "s"(op.mf[3]), "s"(op.mf[4]), "s"(op.mf[5]),
-                     "s"(op.mf[6]), "s"(op.mf[7]));
-    else
-        asm volatile("" ::"s"(op.m[0]), "s"(op.m[1]), "s"(op.m[2]), "s"(op.m[3]), "s"(op.m[4]), "s"(op.m[5]),
-                     "s"(op.m[6]), "s"(op.m[7]));
+    asm volatile("" ::"s"(op.code), "s"(op.ctl), "s"(op.co), "s"(op.m[0]), "s"(op.m[1]), "s"(op.m[2]), "s"(op.m[3]),
+                 "s"(op.m[4]), "s"(op.m[5]), "s"(op.m[6]), "s"(op.m[7]));
+}
+
+// Touches `bytes` (at least 4) of a program: by vector loads of the whole
+// workgroup into this XCD's L2, then by scalar loads of each wave's share into
+// the scalar cache.  A workgroup's first tile otherwise waits for memory at
+// every op (no other tile has read the program on this XCD): 17 qubits
+// complex64, 32 tiles, @@ us per sweep without and @@ with.
+__device__ __forceinline__ void warm_program(const void* p, uint32_t bytes)
+{
+    const uint32_t* w = static_cast<const uint32_t*>(p);
+    for (uint32_t o = threadIdx.x * 16u; o < bytes / 4; o += blockDim.x * 16u) {
+        const uint32_t x = w[o];
+        asm volatile("" ::"v"(x));
+    }
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = (blockDim.x + 63u) >> 6;
+    const uint32_t last = bytes / 4 - 1;
+    for (uint32_t o = wave * 128u; o <= last; o += nw * 128u) {
+        uint32_t x = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t i = o + 16u * k;
+            x ^= load_uniform(w, i < last ? i : last);
+        }
+        asm volatile("" ::"s"(x));
+    }
 }
 
 // LDS slot of local element l: XOR-fold higher bits into the low SW bits so
@@ -155,62 +175,8 @@ __device__ __forceinline__ void dense_pairs(V (&v)[NR], uint32_t cr, bool tok, V
     }
 }
 
-template <typename V, int NR, int R, int FORM, bool TC, bool RC, int CB = -1>
-__device__ __forceinline__ void dense_reg(int reg, V (&v)[NR], uint32_t cr, bool tok, V m0, V m1, V m2, V m3)
-{
-    switch (reg) {
-    case 0: dense_pairs<V, NR, 0, FORM, TC, RC, CB>(v, cr, tok, m0, m1, m2, m3); break;
-    case 1: dense_pairs<V, NR, 1, FORM, TC, RC, CB>(v, cr, tok, m0, m1, m2, m3); break;
-    case 2: dense_pairs<V, NR, 2, FORM, TC, RC, CB>(v, cr, tok, m0, m1, m2, m3); break;
-    case 3: dense_pairs<V, NR, 3, FORM, TC, RC, CB>(v, cr, tok, m0, m1, m2, m3); break;
-    default:
-        if constexpr (R > 4) dense_pairs<V, NR, (R > 4 ? 4 : 0), FORM, TC, RC, CB>(v, cr, tok, m0, m1, m2, m3);
-        break;
-    }
-}
-
-// Swap-form ops (X, CX, Toffoli targets) with exactly one register control:
-// the control's register index picked at compile time.
-template <typename V, int NR, int R, bool TC>
-__device__ __forceinline__ void swap_one_rc(int cb, int reg, V (&v)[NR], bool tok)
-{
-    const V z = mkc<V>(0, 0);
-    switch (cb) {
-    case 0: dense_reg<V, NR, R, SWF_SWAP, TC, false, 0>(reg, v, 0u, tok, z, z, z, z); break;
-    case 1: dense_reg<V, NR, R, SWF_SWAP, TC, false, 1>(reg, v, 0u, tok, z, z, z, z); break;
-    case 2: dense_reg<V, NR, R, SWF_SWAP, TC, false, 2>(reg, v, 0u, tok, z, z, z, z); break;
-    default:
-        if constexpr (R > 3) dense_reg<V, NR, R, SWF_SWAP, TC, false, (R > 3 ? 3 : 0)>(reg, v, 0u, tok, z, z, z, z);
-        break;
-    }
-}
-
-// Controls by where they live: thread bits (TC, a per-lane predicate) and
-// register bits (RC, a per-slot predicate); each combination has its own
-// straight-line body, so the common uncontrolled op carries no selects.
-template <typename V, int NR, int R, int FORM>
-__device__ __forceinline__ void dense_ctl(int reg, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, V m0, V m1, V m2,
-                                          V m3)
-{
-    if constexpr (FORM == SWF_SWAP) {
-        if (cr != 0 && (cr & (cr - 1)) == 0) {
-            const int cb = __builtin_ctz(cr);
-            if (ct) swap_one_rc<V, NR, R, true>(cb, reg, v, tok);
-            else swap_one_rc<V, NR, R, false>(cb, reg, v, tok);
-            return;
-        }
-    }
-    if (ct) {
-        if (cr) dense_reg<V, NR, R, FORM, true, true>(reg, v, cr, tok, m0, m1, m2, m3);
-        else dense_reg<V, NR, R, FORM, true, false>(reg, v, cr, tok, m0, m1, m2, m3);
-    } else {
-        if (cr) dense_reg<V, NR, R, FORM, false, true>(reg, v, cr, tok, m0, m1, m2, m3);
-        else dense_reg<V, NR, R, FORM, false, false>(reg, v, cr, tok, m0, m1, m2, m3);
-    }
-}
-
-// The interpreter's dense bodies.  Three forms only (general, real, RX: the
-// planner gives X, CX and Y ops their matrices, interpreter_ops): every body
+// The interpreter's dense bodies.  Three forms only (general, real, RX: X, CX
+// and Y come with their matrices, InterpOpT): every body
 // writes its results where its inputs were, so the register array is not
 // copied at the joins of the dispatch.  Thread controls select the
 // coefficients (the identity's where the lane's controls are not set) instead
@@ -218,7 +184,14 @@ __device__ __forceinline__ void dense_ctl(int reg, V (&v)[NR], uint32_t cr, uint
 template <typename V, int NR, int R, int FORM, bool RC>
 __device__ __forceinline__ void interp_reg(int reg, V (&v)[NR], uint32_t cr, V m0, V m1, V m2, V m3)
 {
-    dense_reg<V, NR, R, FORM, false, RC>(reg, v, cr, true, m0, m1, m2, m3);
+    switch (reg) {
+    case 0: dense_pairs<V, NR, 0, FORM, false, RC>(v, cr, true, m0, m1, m2, m3); break;
+    case 1: dense_pairs<V, NR, 1, FORM, false, RC>(v, cr, true, m0, m1, m2, m3); break;
+    case 2: dense_pairs<V, NR, 2, FORM, false, RC>(v, cr, true, m0, m1, m2, m3); break;
+    default:
+        if constexpr (R > 3) dense_pairs<V, NR, (R > 3 ? 3 : 0), FORM, false, RC>(v, cr, true, m0, m1, m2, m3);
+        break;
+    }
 }
 template <typename V, int NR, int R, int FORM>
 __device__ __forceinline__ void interp_ctl(int reg, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, V m0, V m1, V m2,
@@ -236,17 +209,6 @@ __device__ __forceinline__ void interp_ctl(int reg, V (&v)[NR], uint32_t cr, uin
     if (cr) interp_reg<V, NR, R, FORM, true>(reg, v, cr, m0, m1, m2, m3);
     else interp_reg<V, NR, R, FORM, false>(reg, v, cr, m0, m1, m2, m3);
 }
-template <typename V, int NR, int R>
-__device__ __forceinline__ void dense_form_dispatch(uint32_t form, int reg, V (&v)[NR], uint32_t cr, uint32_t ct,
-                                                    bool tok, V m0, V m1, V m2, V m3)
-{
-    switch (form) {
-    case SWF_REAL: interp_ctl<V, NR, R, SWF_REAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    case SWF_RX: interp_ctl<V, NR, R, SWF_RX>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    default: interp_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3); break;
-    }
-}
-
 // Multiply the registers whose register controls `cr` are set (and, with TC,
 // whose lane passes `tok`) by the value f(k, v[k]) gives.
 template <typename V, int NR, bool TC, bool RC, typename F, int CB = -1>
@@ -316,17 +278,40 @@ __device__ __forceinline__ void phase_op(uint32_t form, V (&v)[NR], uint32_t cr,
     }
 }
 
-template <typename V, int NR>
-__device__ __forceinline__ void diag_op(const SwOp& op, V (&v)[NR], uint32_t cr, uint32_t ct, bool tok, uint64_t base,
-                                        int tid, V d0, V d1)
+// One op on a thread's registers.  SEQ: the whole-state programs' rounding.
+template <typename V, int NR, int R, bool SEQ, typename Op>
+__device__ __forceinline__ void interp_op(const Op& op, V (&v)[NR], uint32_t tid, uint64_t base)
 {
-    if (op.dreg >= 0) {
-        const int dr = op.dreg;
-        scale_regs<V, NR>(v, cr, ct, tok, [&](int k, V x) { return cmul(sel(((k >> dr) & 1) != 0, d1, d0), x); });
+    const uint32_t body = op.code & 0xffu, cr = op.ctl & 0xffffu, ct = op.ctl >> 16;
+    const int reg = int((op.code >> 8) & 0xffu);
+    const bool tok = (tid & ct) == ct;
+    const V m0 = mkc<V>(op.m[0], op.m[1]), m1 = mkc<V>(op.m[2], op.m[3]);
+    if (body < kInterpPhase) {
+        const V m2 = mkc<V>(op.m[4], op.m[5]), m3 = mkc<V>(op.m[6], op.m[7]);
+        if (body == (SEQ ? SWF_REAL_SEQ : SWF_REAL))
+            interp_ctl<V, NR, R, SEQ ? SWF_REAL_SEQ : SWF_REAL>(reg, v, cr, ct, tok, m0, m1, m2, m3);
+        else if (body == (SEQ ? SWF_RX_SEQ : SWF_RX))
+            interp_ctl<V, NR, R, SEQ ? SWF_RX_SEQ : SWF_RX>(reg, v, cr, ct, tok, m0, m1, m2, m3);
+        else
+            interp_ctl<V, NR, R, SWF_GENERAL>(reg, v, cr, ct, tok, m0, m1, m2, m3);
+    } else if (body == kInterpDiagReg) {
+        if (ct) {
+            const V one = mkc<V>(1, 0), d0 = sel(tok, m0, one), d1 = sel(tok, m1, one);
+            scale_regs<V, NR>(v, cr, 0u, true, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, d1, d0), x); });
+        } else {
+            scale_regs<V, NR>(v, cr, 0u, true, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, m1, m0), x); });
+        }
     } else {
-        const bool one = op.dtid >= 0 ? ((tid >> op.dtid) & 1) : ((base >> op.dglobal) & 1);
-        const V d = sel(one, d1, d0);
-        scale_regs<V, NR>(v, cr, ct, tok, [&](int, V x) { return cmul(d, x); });
+        // one factor per lane: a phase (m0 where the controls are set), or a
+        // diagonal entry picked by a thread bit or a bit outside the tile
+        V f = m0;
+        if (body != kInterpPhase) {
+            const uint32_t bit = op.code >> 16;
+            const bool one = body == kInterpDiagTid ? ((tid >> bit) & 1u) != 0 : ((base >> bit) & 1u) != 0;
+            f = sel(one, m1, m0);
+        }
+        if (ct) f = sel(tok, f, mkc<V>(1, 0));
+        scale_regs<V, NR>(v, cr, 0u, true, [&](int, V x) { return cmul(f, x); });
     }
 }
 
@@ -608,23 +593,12 @@ __device__ __forceinline__ void tile_phases(V* __restrict__ a, const SweepArgs& 
             V v[NR];
 #pragma unroll
             for (int k = 0; k < NR; ++k) v[k] = lds[st ^ srp[k]];
+            const InterpOpT<Rl>* ops = reinterpret_cast<const InterpOpT<Rl>*>(sa.ops);
             for (uint32_t oi = ph.op_begin; oi < ph.op_end; ++oi) {
-                const SwOp op = load_uniform(sa.ops, oi);
-                pin_op<V>(op);
+                const InterpOpT<Rl> op = load_uniform(ops, oi);
+                pin_op<Rl>(op);
                 if ((base & op.co) != op.co) continue;
-                const uint32_t cr = op.cr, ct = op.ct;
-                const bool tok = (uint32_t(tid) & ct) == ct;
-                if (op.type == SW_DENSE1) {
-                    const V m0 = opm<V>(op, 0), m1 = opm<V>(op, 1), m2 = opm<V>(op, 2), m3 = opm<V>(op, 3);
-                    dense_form_dispatch<V, NR, R>(op.aux, op.reg, v, cr, ct, tok, m0, m1, m2, m3);
-                } else if (op.type == SW_PHASE) {
-                    // a factor of +-1, +-i is an exact one
-                    const V f = sel(tok, opm<V>(op, 0), mkc<V>(1, 0));
-                    scale_regs<V, NR>(v, cr, 0u, tok, [&](int, V x) { return cmul(f, x); });
-                } else {  // SW_DIAG1
-                    const V d0 = opm<V>(op, 0), d1 = opm<V>(op, 1);
-                    diag_op<V, NR>(op, v, cr, ct, tok, base, tid, d0, d1);
-                }
+                interp_op<V, NR, R, false>(op, v, uint32_t(tid), base);
             }
             if (ph.wmap == 0) {
 #pragma unroll

@@ -87,20 +87,24 @@ constexpr int swizzle_slot(int SW, int M, int l)
 // Swizzle width of the sweep kernels for 2^M tiles (13 -> 5, else 4).
 constexpr int sweep_swizzle_bits(int M) { return M == 13 ? 5 : 4; }
 
-// ---- whole-state programs (k_whole): a state of up to 14 qubits in LDS
+// ---- ops of the interpreting kernels (k_sweep, k_sweep_batched, k_whole)
 
-// One op; its values m follow in the state's precision (WholeOpT).  `code`:
-// bits 0-7 body (SwDenseForm, or kWholePhase + SwPhaseForm, kWholeDiagReg,
-// kWholeDiagTid), bits 8-15 register bit of the target, bits 16-23 thread bit
-// of a diagonal target.
-constexpr uint32_t kWholePhase = 16, kWholeDiagReg = 20, kWholeDiagTid = 21;
-template <typename R> struct WholeOpT {
+// A SwOp in the state's precision: 80 bytes complex128, 48 complex64 (a
+// program of 100 ops then stays in the 16 KiB scalar cache).  X, CX and Y have
+// the body of their matrix, phases of any value the general product (0, 1 and
+// +-i are exact factors).  `code`: bits 0-7 body (SwDenseForm or kInterp*),
+// 8-15 register bit of the target, 16-23 thread bit or outer bit of a
+// diagonal's target; `ctl`: controls over register indices (low half) and
+// thread bits (high half); `co`: controls over bits outside the tile.
+constexpr uint32_t kInterpPhase = 16, kInterpDiagReg = 17, kInterpDiagTid = 18, kInterpDiagOuter = 19;
+template <typename R> struct InterpOpT {
     uint32_t code;
-    uint32_t cr;     // controls over register indices
-    uint32_t ct;     // controls over thread-index bits
-    uint32_t pad;
+    uint32_t ctl;
+    uint64_t co;
     R m[8];
 };
+
+// ---- whole-state programs (k_whole): a state of up to 14 qubits in LDS
 
 // A register phase: R register bits, thread bits the others.  The LDS slot of a
 // thread's element k is tin ^ (slot[k] & 0xffff) when the phase reads the state
