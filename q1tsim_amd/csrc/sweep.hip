@@ -131,7 +131,12 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
     sa.nphases = nphases;
     sa.nops = uint32_t(nops);
     const uint64_t dim = uint64_t(1) << n;
-    const unsigned gx = unsigned(std::min<uint64_t>(sa.ntiles, 2048));
+    // far more workgroups than the chip holds (1024): they start as others
+    // finish, and loads, stores and arithmetic of neighbours spread out in
+    // time.  28 qubits complex64, 10 sweeps: 512 workgroups 27.4 ms, 2048 18.7,
+    // 16384 17.1, one per tile 17.4; specialised kernels, 30 qubits complex128:
+    // 2048 89.0 ms, 16384 85.2.
+    const unsigned gx = unsigned(std::min<uint64_t>(sa.ntiles, 16384));
     int first = -1;
     for (size_t c0 = cb; c0 < ce; c0 += 65535) {
         const unsigned ny = unsigned(std::min<size_t>(65535, ce - c0));
