@@ -240,6 +240,7 @@ public:
     void set_tiling(bool on) { tiling_ = on; }
     void set_geometry(const TileGeom& g);
     const TileGeom& geometry() const { return geom_; }
+    bool geometry_set() const { return geom_set_; }
     hipStream_t stream() const { return stream_; }
     void* device_amplitudes() { return amp_; }
     size_t elem_bytes() const { return prec_ == PREC_C128 ? 16 : 8; }

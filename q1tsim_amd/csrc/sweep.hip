@@ -357,11 +357,11 @@ struct PlanCacheEntry {
     std::vector<int> kind;
 };
 
-static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queue, int fusion_k, double state_bytes,
-                        double tiles, std::vector<PlanStep>& steps, std::vector<SweepProgram>& progs)
+static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queue, const TileGeom& g, int fusion_k,
+                        double state_bytes, double tiles, std::vector<PlanStep>& steps,
+                        std::vector<SweepProgram>& progs)
 {
     const int n = int(st.nr_bits());
-    const TileGeom g = st.geometry();
     const int prec = int(st.precision());
     const bool search = st.tile_search(), phase_search = st.phase_search(state_bytes);
     const bool factors = st.tile_factors();   // specialised kernels only
@@ -740,7 +740,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
                  int fusion_k, bool tiling, RunStats& stats)
 {
     const int n = int(st.nr_bits());
-    const TileGeom g = st.geometry();
+    TileGeom g = st.geometry();
     if (!tiling) {
         for (const PendingGate& pg : queue) st.apply_op(pg.op, col_begin, col_end);
         return;
@@ -752,9 +752,15 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
     }
     const double S = double(uint64_t(1) << n) * double(st.elem_bytes()) * double(col_end - col_begin);
     const double tiles = double(col_end - col_begin) * double(uint64_t(1) << std::max(0, n - g.M));
+    // complex64 interpreter with at most two tiles per CU: a sweep lasts as
+    // long as one tile, so 8 amplitudes per thread and twice the waves win
+    // over fewer phases.  12 layers, kernel time R=3 / R=4: 17 qubits 124 /
+    // 142 us, 20 qubits 152 / 169, 21 qubits 212 / 219, 22 qubits 362 / 304.
+    if (st.precision() == PREC_C64 && !st.geometry_set() && !st.jit_enabled() && fusion_k == 0 && tiles <= 512.0)
+        g.R = 3;
     std::vector<PlanStep> steps;
     std::vector<SweepProgram> progs;
-    choose_plan(st, queue, fusion_k, S, tiles, steps, progs);
+    choose_plan(st, queue, g, fusion_k, S, tiles, steps, progs);
 
     // all sweep programs of this flush in one upload: [phases][ops] per sweep, then the block table
     std::vector<size_t> poff(steps.size()), ooff(steps.size()), boff_s(steps.size());
