@@ -1311,22 +1311,6 @@ void GpuVectorState::measure_into(size_t qbit, size_t cbit, uint64_t* res, size_
     measure_with_n0(qbit, cbit, n0s.data(), w0, res, res_len, collapse, basis);
 }
 
-// Levels of the canonical tree of one column: sizes shrink by 16 until <= 16.
-static TreeDesc tree_shape(uint64_t dim, uint64_t* entries)
-{
-    TreeDesc td{};
-    td.nlev = 1;
-    td.size[0] = dim;
-    uint64_t total = 0;
-    while (td.size[td.nlev - 1] > uint64_t(kTreeFanout)) {
-        td.size[td.nlev] = (td.size[td.nlev - 1] + kTreeFanout - 1) / kTreeFanout;
-        total += td.size[td.nlev];
-        td.nlev += 1;
-    }
-    *entries = total;
-    return td;
-}
-
 // The sampling of measure_all_into_helper (vectorstate.rs:106-161): the
 // tree levels of every column and one walk per run, queued.
 size_t GpuVectorState::sample_enqueue(ItemQueue& q, const double* u)
@@ -1335,8 +1319,7 @@ size_t GpuVectorState::sample_enqueue(ItemQueue& q, const double* u)
     if (basis_ && basis_rot_ != 0) materialize_enqueue(q);   // rotated basis columns are dense in Z
     if (basis_) return SIZE_MAX;
     const size_t nc = counts_.size();
-    uint64_t per_col = 0;
-    TreeDesc td = tree_shape(dim(), &per_col);
+    const uint64_t per_col = tree_offset(int(nr_bits_), tree_top(int(nr_bits_)) + 1);
     const size_t need = std::max<size_t>(per_col * nc, 1);
     if (need > tree_cap_) {
         dev_release(d_tree_, tree_cap_ * sizeof(double));
@@ -1345,20 +1328,6 @@ size_t GpuVectorState::sample_enqueue(ItemQueue& q, const double* u)
         d_tree_ = static_cast<double*>(dev_alloc(need * sizeof(double)));
         tree_cap_ = need;
     }
-    {   // column 0's level pointers; column c's are per_col entries further
-        uint64_t o = 0;
-        for (int l = 1; l < td.nlev; ++l) {
-            td.lev[l] = d_tree_ + o;
-            o += td.size[l];
-        }
-    }
-    std::vector<LevelItem> levels;
-    levels.reserve(size_t(td.nlev - 1) * nc);
-    for (int l = 1; l < td.nlev; ++l)
-        for (size_t c = 0; c < nc; ++c)
-            levels.push_back(LevelItem{l == 1 ? static_cast<const void*>(col_ptr(c))
-                                              : static_cast<const void*>(td.lev[l - 1] + c * per_col),
-                                       const_cast<double*>(td.lev[l]) + c * per_col, td.size[l - 1], 0});
     std::vector<uint64_t> first(nc + 1);
     uint64_t run = 0;
     for (size_t c = 0; c < nc; ++c) {
@@ -1369,10 +1338,11 @@ size_t GpuVectorState::sample_enqueue(ItemQueue& q, const double* u)
     SampleJob job{};
     job.a0 = col_ptr(0);
     job.col_stride = dim();
-    job.td = td;
+    job.tree = d_tree_;
+    job.nbits = int32_t(nr_bits_);
     job.per_col = per_col;
     job.ncols = int32_t(nc);
-    return q.add_sample(job, levels, first.data(), u, size_t(run));
+    return q.add_sample(job, first.data(), u, size_t(run));
 }
 
 // Grouping and bit mapping of measure_all_into_helper (vectorstate.rs:106-161)

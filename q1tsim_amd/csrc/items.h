@@ -4,10 +4,10 @@
 // on whole columns of a state, and a batch of circuits needs the same kind of
 // work on thousands of columns of different states in the same round.  An
 // ItemQueue collects that work as items (one per column, or per state for
-// the sampling walk), uploads every item table in one copy, launches one
-// kernel per kind in dependency order and copies every result back in one
-// copy.  The single-state paths run the same kernels through a queue of
-// their own, so a state gives the same bits alone and in a batch.
+// the sampling walk), uploads the item tables in one copy, launches one
+// kernel per kind in dependency order and has the kernels write the results
+// to host memory.  The single-state paths run the same kernels through a queue
+// of their own, so a state gives the same bits alone and in a batch.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -21,15 +21,18 @@
 
 namespace q1t {
 
-// Sampling tree of one column: level 0 is the column's amplitudes (weights
-// |a|^2), level l > 0 holds the left folds of 16 consecutive entries of
-// level l - 1; lev[l] points at column 0's level l, column c's is per_col
-// entries further.
-struct TreeDesc {
-    int nlev;
-    uint64_t size[16];
-    const double* lev[16];   // lev[0] unused
-};
+// Sampling tree of one column of 2^n amplitudes: level 0 is the column's
+// amplitudes (weights |a|^2), level l > 0 holds the left folds of 16
+// consecutive entries of level l - 1, up to the first level of at most 16
+// entries.  Level l has 2^(n - 4l) entries; levels 1, 2, ... follow each other
+// in memory.
+inline __host__ __device__ int tree_top(int n) { return n <= 4 ? 0 : (n - 1) / 4; }
+inline __host__ __device__ uint64_t tree_offset(int n, int l)   // of level l >= 1
+{
+    uint64_t o = 0;
+    for (int i = 1; i < l; ++i) o += uint64_t(1) << (n - 4 * i);
+    return o;
+}
 
 // One column's outcome-0 weight of one qubit: partial sums of up to
 // kMargBlocks workgroups, added by the one that finishes last.
@@ -85,12 +88,14 @@ struct BasisItem {
     int32_t rot, pad;
 };
 
-// One tree level of one column: out[g] = left fold of in[16g .. 16g+15].
-struct LevelItem {
-    const void* in;   // level 1: amplitudes; higher levels: doubles
+// Up to three tree levels of one column: in[0 .. size) folded by 16, `levels`
+// times; the levels follow each other at `out`.
+struct TreeItem {
+    const void* in;   // levels 1 to 3: amplitudes; higher levels: doubles
     double* out;
     uint64_t size;
     uint64_t chunk0;
+    uint32_t levels, pad;
 };
 
 // The sampling walk of all runs of one state: run r of the state (global
@@ -99,12 +104,13 @@ struct LevelItem {
 struct SampleJob {
     const void* a0;
     uint64_t col_stride;
-    TreeDesc td;
+    const double* tree;   // column 0's level 1; column c's is per_col entries further
     uint64_t per_col;
     uint64_t first_off;
     uint64_t run0;
     uint64_t col0;     // global index of the state's first column (top totals)
-    int32_t ncols, pad;
+    int32_t ncols;
+    int32_t nbits;     // a column has 2^nbits amplitudes
 };
 
 class ItemQueue {
@@ -123,20 +129,19 @@ public:
     uint32_t add_op(const ColOp& op);
     void add_op_item(void* amp, uint64_t nwork, uint32_t op);
     void add_basis(const BasisItem& b);
-    // Sampling of one state: its level items, its job and its uniforms
-    // (nruns = first.back()); returns the job index.  Indices land at
-    // indices(job) and per-column top totals at tops(job) after launch().
-    size_t add_sample(const SampleJob& job, const std::vector<LevelItem>& levels, const uint64_t* first,
-                      const double* u, size_t nruns);
+    // Sampling of one state: the job (its tree is built first) and its
+    // uniforms (nruns = first[ncols]); returns the job index.  Indices land
+    // at indices(job) and per-column top totals at tops(job) after launch().
+    size_t add_sample(const SampleJob& job, const uint64_t* first, const double* u, size_t nruns);
     // device blocks to release (on their stream) once launch() has enqueued
     // the kernels that read them
     void release_after(void* p, size_t bytes, hipStream_t s);
 
     bool empty() const;
     // Upload, launch everything in the order basis columns, collapses,
-    // gates, marginals, tree levels, sampling, then copy the results back;
-    // then perform the deferred releases and clear the inputs (results stay
-    // readable until the next launch()).
+    // gates, marginals, tree levels, sampling; then perform the deferred
+    // releases and clear the inputs (results are readable once `s` has been
+    // synchronised, until the next launch()).
     void launch(hipStream_t s);
     uint64_t launches() const { return launches_; }
     // synchronise and forget the last stream and its upload event (before
@@ -154,16 +159,19 @@ public:
     const double* tops(size_t job) const;
 
 private:
+    void launch_items(hipStream_t s);
+    void clear_inputs();   // and perform the deferred releases
+
     bool c64_;
     std::vector<MargItem> marg_;
     std::vector<CollItem> coll_;
     std::vector<ColOp> ops_;
     std::vector<OpItem> opit_;
     std::vector<BasisItem> basis_;
-    std::vector<LevelItem> levels_[16];
+    static constexpr int kTreeSteps = 6;   // launches of three levels each
+    std::vector<TreeItem> tree_[kTreeSteps];
     std::vector<SampleJob> jobs_;
     std::vector<uint64_t> first_;   // per job: ncols + 1 entries
-    std::vector<uint64_t> run0_;    // per job, plus the total
     std::vector<double> u_;
     uint64_t cols_ = 0;
     struct Release {
@@ -172,19 +180,21 @@ private:
         hipStream_t s;
     };
     std::vector<Release> rel_;
-    uint64_t marg_chunks_ = 0, coll_chunks_ = 0, op_chunks_ = 0, basis_chunks_ = 0, level_chunks_[16] = {};
+    uint64_t marg_chunks_ = 0, coll_chunks_ = 0, op_chunks_ = 0, basis_chunks_ = 0, tree_chunks_[kTreeSteps] = {};
 
     // device and pinned host buffers: inputs, then outputs
     char* dbuf_ = nullptr;
     size_t dcap_ = 0;
     char* hin_ = nullptr;
+    char* hin_dev_ = nullptr;    // the pinned buffers as kernels address them
+    char* hout_dev_ = nullptr;
     size_t hin_cap_ = 0;
     char* hout_ = nullptr;
     size_t hout_cap_ = 0;
     char* stage_ = nullptr;
     size_t stage_cap_ = 0;
     hipStream_t stage_stream_ = nullptr;   // a copy from stage_ may be in flight here
-    hipEvent_t in_done_ = nullptr;   // the last input upload has completed
+    hipEvent_t in_done_ = nullptr;   // the last launch has read its inputs in hin_
     hipStream_t last_stream_ = nullptr;
     size_t out_w0_ = 0, out_idx_ = 0, out_top_ = 0;   // offsets in hout_
     std::vector<uint64_t> res_run0_, res_col0_;         // of the last launch

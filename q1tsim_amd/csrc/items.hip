@@ -20,8 +20,8 @@ namespace q1t {
 
 // work units of one column item per workgroup step
 static constexpr uint64_t kChunk = uint64_t(kBlock) * 4;
-// inputs of one tree-level workgroup step (kBlock outputs)
-static constexpr uint64_t kLevelChunk = uint64_t(kBlock) * kTreeFanout;
+// inputs of one tree workgroup step (kBlock outputs of the first level)
+static constexpr uint64_t kTreeChunk = uint64_t(kBlock) * kTreeFanout;
 static constexpr unsigned kMaxGrid = 8192;
 
 // The item whose chunk range holds chunk c: the last with chunk0 <= c.
@@ -35,6 +35,14 @@ __device__ __forceinline__ uint32_t find_item(const I* items, uint32_t n, uint64
         else hi = mid - 1;
     }
     return lo;
+}
+
+// Item of chunk c: a launch with one item has it in its arguments (items is
+// null), so that nothing is uploaded.
+template <typename I>
+__device__ __forceinline__ I item_at(const I& one, const I* items, uint32_t n, uint64_t c)
+{
+    return items ? items[find_item(items, n, c)] : one;
 }
 
 __device__ __forceinline__ uint64_t insert_zero(uint64_t j, int p)
@@ -203,13 +211,13 @@ __device__ __forceinline__ void marginal_block(const V* a, uint64_t nwork, int p
 
 // Chunk c: share c - chunk0 of its item; partial sums at partial[c].
 template <typename V>
-__global__ void __launch_bounds__(kMargThreads) k_marginal_items(const MargItem* __restrict__ items, uint32_t n,
-                                                                 uint64_t nchunks, double* partial, uint32_t* done,
-                                                                 double* w0)
+__global__ void __launch_bounds__(kMargThreads) k_marginal_items(MargItem one, const MargItem* __restrict__ items,
+                                                                 uint32_t n, uint64_t nchunks, double* partial,
+                                                                 uint32_t* done, double* w0)
 {
     for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const uint32_t it = find_item(items, n, c);
-        const MargItem m = items[it];
+        const uint32_t it = items ? find_item(items, n, c) : 0;
+        const MargItem m = items ? items[it] : one;
         marginal_block<V>(static_cast<const V*>(m.amp), m.nwork, m.p, m.basis, uint32_t(c - m.chunk0), m.blocks,
                           2 * m.nwork * sizeof(V) >= kStreamBytes, partial + m.chunk0, done + it, w0 + it);
         __syncthreads();   // the shared sums and flag are reused by the next chunk
@@ -298,11 +306,11 @@ __device__ __forceinline__ void collapse_pair(const CollItem& m, uint64_t j)
 }
 
 template <typename V>
-__global__ void __launch_bounds__(kBlock) k_collapse_items(const CollItem* __restrict__ items, uint32_t n,
-                                                           uint64_t nchunks)
+__global__ void __launch_bounds__(kBlock) k_collapse_items(CollItem one, const CollItem* __restrict__ items,
+                                                           uint32_t n, uint64_t nchunks)
 {
     for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const CollItem m = items[find_item(items, n, c)];
+        const CollItem m = item_at(one, items, n, c);
         const uint64_t j0 = (c - m.chunk0) * kChunk;
         const uint64_t j1 = j0 + kChunk < m.nwork ? j0 + kChunk : m.nwork;
         for (uint64_t j = j0 + threadIdx.x; j < j1; j += kBlock) collapse_pair<V>(m, j);
@@ -388,12 +396,12 @@ __global__ void __launch_bounds__(kBlock) k_op_items(const OpItem* __restrict__ 
 // Column of |k> (rot 0), H^n|k> (rot 1) or S^n H^n|k> (rot 2): amplitude j =
 // (-1)^popcount(j&k) i^popcount(j) (the i factor for rot 2 only) times mag.
 template <typename V>
-__global__ void __launch_bounds__(kBlock) k_basis_items(const BasisItem* __restrict__ items, uint32_t n,
-                                                        uint64_t nchunks)
+__global__ void __launch_bounds__(kBlock) k_basis_items(BasisItem one, const BasisItem* __restrict__ items,
+                                                        uint32_t n, uint64_t nchunks)
 {
     using Rl = typename RealOf<V>::type;
     for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const BasisItem b = items[find_item(items, n, c)];
+        const BasisItem b = item_at(one, items, n, c);
         V* a = static_cast<V*>(b.amp);
         const Rl mag = Rl(b.mag);
         const uint64_t j0 = (c - b.chunk0) * kChunk;
@@ -414,93 +422,161 @@ __global__ void __launch_bounds__(kBlock) k_basis_items(const BasisItem* __restr
 
 // ------------------------------------------------------------- sampling
 
-template <typename T> __device__ __forceinline__ double leaf(const T* in, uint64_t k);
-template <> __device__ __forceinline__ double leaf<double2>(const double2* in, uint64_t k) { return weight(in[k]); }
-template <> __device__ __forceinline__ double leaf<float2>(const float2* in, uint64_t k) { return weight(in[k]); }
-template <> __device__ __forceinline__ double leaf<double>(const double* in, uint64_t k) { return in[k]; }
+__device__ __forceinline__ double leaf(double2 a) { return weight(a); }
+__device__ __forceinline__ double leaf(float2 a) { return weight(a); }
+__device__ __forceinline__ double leaf(double w) { return w; }
 
-// One tree level of many columns: out[g] = left fold of in[16g .. 16g+15].
-// A workgroup step folds 4096 inputs; loads are coalesced into LDS in a
-// transposed, padded layout so each thread reads its 16 values bank-conflict
-// free.
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_level_items(const LevelItem* __restrict__ items, uint32_t n,
-                                                        uint64_t nchunks)
+template <bool NT, typename V> __device__ __forceinline__ double load_leaf(const V* p) { return leaf(load_amp<NT>(p)); }
+template <bool NT> __device__ __forceinline__ double load_leaf(const double* p) { return *p; }
+
+// The weights of the kTreeChunk entries from `base` on, into LDS, 16 loads per
+// thread in flight; entry e in a transposed, padded place, so that thread t
+// reads entries 16t .. 16t+15 without bank conflicts.
+template <typename T, bool NT>
+__device__ __forceinline__ void load_leaves(const T* in, uint64_t size, uint64_t base, double* w)
 {
-    __shared__ double w[kTreeFanout * (kBlock + 1)];
-    for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const LevelItem it = items[find_item(items, n, c)];
-        const T* in = static_cast<const T*>(it.in);
-        const uint64_t size = it.size;
-        const uint64_t nout = (size + kTreeFanout - 1) / kTreeFanout;
-        const uint64_t base = (c - it.chunk0) * kLevelChunk;
+    double v[kTreeFanout];
+    if (base + kTreeChunk <= size) {
+#pragma unroll
+        for (int r = 0; r < kTreeFanout; ++r) v[r] = load_leaf<NT>(in + base + r * kBlock + threadIdx.x);
+    } else {
 #pragma unroll
         for (int r = 0; r < kTreeFanout; ++r) {
-            const int e = r * kBlock + threadIdx.x;
-            const uint64_t k = base + e;
-            const double v = k < size ? leaf<T>(in, k) : 0.0;
-            w[(e & (kTreeFanout - 1)) * (kBlock + 1) + (e >> 4)] = v;
+            const uint64_t k = base + r * kBlock + threadIdx.x;
+            v[r] = k < size ? load_leaf<NT>(in + k) : 0.0;
         }
+    }
+#pragma unroll
+    for (int r = 0; r < kTreeFanout; ++r) {
+        const int e = r * kBlock + threadIdx.x;
+        w[(e & (kTreeFanout - 1)) * (kBlock + 1) + (e >> 4)] = v[r];
+    }
+}
+
+// Up to three levels of the sampling tree, a workgroup per 4096 inputs: bound
+// by the read of the column at the first levels (the higher ones hold 1/16 of
+// it and less) and by launches for small columns, so one launch makes three
+// levels: 256 threads fold 16 entries each, 16 threads the 256 folds, one
+// thread the 16 folds of those.  Sizes are powers of two above 16: every group
+// that exists is full.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_tree_items(TreeItem one, const TreeItem* __restrict__ items, uint32_t n,
+                                                       uint64_t nchunks)
+{
+    __shared__ double w[kTreeFanout * (kBlock + 1)];
+    __shared__ double w2[kTreeFanout * (kTreeFanout + 1)];
+    const uint32_t t = threadIdx.x;
+    for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+        const TreeItem it = item_at(one, items, n, c);
+        const T* in = static_cast<const T*>(it.in);
+        const uint64_t base = (c - it.chunk0) * kTreeChunk;
+        const uint64_t n1 = it.size / kTreeFanout, n2 = n1 / kTreeFanout;
+        if (it.size * sizeof(T) >= kStreamBytes) load_leaves<T, true>(in, it.size, base, w);
+        else load_leaves<T, false>(in, it.size, base, w);
         __syncthreads();
-        const uint64_t g = base / kTreeFanout + threadIdx.x;
-        if (g < nout) {
-            double acc = w[threadIdx.x];
-            for (int jj = 1; jj < kTreeFanout; ++jj)
-                if (g * kTreeFanout + jj < size) acc += w[jj * (kBlock + 1) + threadIdx.x];
+        double acc = 0.0;
+        const uint64_t g = base / kTreeFanout + t;
+        if (g < n1) {
+            acc = w[t];
+#pragma unroll
+            for (int j = 1; j < kTreeFanout; ++j) acc += w[j * (kBlock + 1) + t];
             it.out[g] = acc;
+        }
+        if (it.levels > 1) {
+            w2[(t & (kTreeFanout - 1)) * (kTreeFanout + 1) + (t >> 4)] = acc;
+            __syncthreads();
+            if (t < 64) {
+                const uint64_t g2 = base / (kTreeFanout * kTreeFanout) + t;
+                double a2 = 0.0;
+                if (t < kTreeFanout && g2 < n2) {
+                    a2 = w2[t];
+#pragma unroll
+                    for (int j = 1; j < kTreeFanout; ++j) a2 += w2[j * (kTreeFanout + 1) + t];
+                    it.out[n1 + g2] = a2;
+                }
+                if (it.levels > 2) {
+                    double a3 = __shfl(a2, 0, 64);
+#pragma unroll
+                    for (int j = 1; j < kTreeFanout; ++j) a3 += __shfl(a2, j, 64);
+                    if (t == 0) it.out[n1 + n2 + base / kTreeChunk] = a3;
+                }
+            }
         }
         __syncthreads();
     }
 }
 
+// Entry k of a tree level of a column (level 0: its amplitudes).
 template <typename V>
-__device__ __forceinline__ double tree_at(const V* a, const TreeDesc& td, int l, uint64_t k, uint64_t coff)
+__device__ __forceinline__ double tree_at(const V* a, const double* lev, int l, uint64_t k)
 {
-    return l == 0 ? weight(a[k]) : td.lev[l][coff + k];
+    return l == 0 ? weight(a[k]) : lev[k];
+}
+
+// The last job whose key (run0 or col0) is at most x.
+__device__ __forceinline__ SampleJob job_at(const SampleJob& one, const SampleJob* jobs, uint32_t njobs,
+                                            uint64_t SampleJob::*key, uint64_t x)
+{
+    if (!jobs) return one;
+    uint32_t lo = 0, hi = njobs - 1;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].*key <= x) lo = mid;
+        else hi = mid - 1;
+    }
+    return jobs[lo];
 }
 
 // Inverse-CDF sampling of one run per thread by the canonical tree walk:
 // t = u * T; within each group keep offset += S_j while offset + S_j <= t,
 // descend into the first child where that fails, or the last positive one.
+// The workgroups past the runs' write the total weight of each column (its
+// top tree level summed in order), one thread per column of all jobs: the
+// norm check of measure_all.
 template <typename V>
-__global__ void __launch_bounds__(kBlock) k_sample_items(const SampleJob* __restrict__ jobs, uint32_t njobs,
-                                                         const uint64_t* __restrict__ run0,
-                                                         const uint64_t* __restrict__ first,
+__global__ void __launch_bounds__(kBlock) k_sample_items(SampleJob one, const SampleJob* __restrict__ jobs,
+                                                         uint32_t njobs, const uint64_t* __restrict__ first,
                                                          const double* __restrict__ u01, uint64_t nruns,
-                                                         uint64_t* __restrict__ out)
+                                                         uint64_t* __restrict__ out, uint64_t ncols,
+                                                         double* __restrict__ tops)
 {
-    const uint64_t r = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (r >= nruns) return;
-    uint32_t lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (run0[mid] <= r) lo = mid;
-        else hi = mid - 1;
+    const uint64_t run_blocks = (nruns + kBlock - 1) / kBlock;
+    const bool is_top = blockIdx.x >= run_blocks;
+    const uint64_t r = (uint64_t(blockIdx.x) - (is_top ? run_blocks : 0)) * kBlock + threadIdx.x;
+    if (r >= (is_top ? ncols : nruns)) return;
+    const SampleJob jb = job_at(one, jobs, njobs, is_top ? &SampleJob::col0 : &SampleJob::run0, r);
+    uint64_t col;
+    if (is_top) {
+        col = r - jb.col0;
+    } else {
+        const uint64_t rl = r - jb.run0;
+        const uint64_t* fr = first + jb.first_off;
+        int clo = 0, chi = jb.ncols - 1;
+        while (clo < chi) {
+            const int mid = (clo + chi + 1) >> 1;
+            if (fr[mid] <= rl) clo = mid;
+            else chi = mid - 1;
+        }
+        col = uint64_t(clo);
     }
-    const SampleJob& jb = jobs[lo];
-    const uint64_t rl = r - jb.run0;
-    const uint64_t* fr = first + jb.first_off;
-    int clo = 0, chi = jb.ncols - 1;
-    while (clo < chi) {
-        const int mid = (clo + chi + 1) >> 1;
-        if (fr[mid] <= rl) clo = mid;
-        else chi = mid - 1;
+    const V* a = static_cast<const V*>(jb.a0) + col * jb.col_stride;
+    const int nb = jb.nbits, top = tree_top(nb);
+    const double* lev = jb.tree + col * jb.per_col + tree_offset(nb, top);
+    uint64_t gstart = 0, glen = uint64_t(1) << (nb - 4 * top), idx = 0;
+    double total = tree_at(a, lev, top, 0);
+    for (uint64_t k = 1; k < glen; ++k) total += tree_at(a, lev, top, k);
+    if (is_top) {
+        tops[r] = total;
+        return;
     }
-    const V* a = static_cast<const V*>(jb.a0) + uint64_t(clo) * jb.col_stride;
-    const uint64_t coff = uint64_t(clo) * jb.per_col;
-    const TreeDesc& td = jb.td;
-    const int top = td.nlev - 1;
-    double total = tree_at(a, td, top, 0, coff);
-    for (uint64_t k = 1; k < td.size[top]; ++k) total += tree_at(a, td, top, k, coff);
     const double t = u01[r] * total;
     double offset = 0.0;
-    uint64_t gstart = 0, glen = td.size[top], idx = 0;
     for (int l = top; l >= 0; --l) {
         double v[kTreeFanout];
         int last = 0;
 #pragma unroll
         for (int j = 0; j < kTreeFanout; ++j) {
-            v[j] = (uint64_t(j) < glen) ? tree_at(a, td, l, gstart + j, coff) : 0.0;
+            v[j] = (uint64_t(j) < glen) ? tree_at(a, lev, l, gstart + j) : 0.0;
             if (v[j] > 0.0) last = j;
         }
         int chosen = last;
@@ -514,35 +590,11 @@ __global__ void __launch_bounds__(kBlock) k_sample_items(const SampleJob* __rest
             }
         }
         idx = gstart + uint64_t(chosen);
-        if (l == 0) break;
         gstart = idx * kTreeFanout;
-        const uint64_t rem = td.size[l - 1] - gstart;
-        glen = rem < uint64_t(kTreeFanout) ? rem : uint64_t(kTreeFanout);
+        glen = kTreeFanout;
+        if (l > 1) lev -= uint64_t(1) << (nb - 4 * (l - 1));
     }
     out[r] = idx;
-}
-
-// Total weight of each column (its top tree level summed in order), one
-// thread per column of all jobs: the norm check of measure_all.
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_top_items(const SampleJob* __restrict__ jobs, uint32_t njobs,
-                                                      uint64_t ncols, double* __restrict__ tops)
-{
-    const uint64_t cg = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (cg >= ncols) return;
-    uint32_t lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (jobs[mid].col0 <= cg) lo = mid;
-        else hi = mid - 1;
-    }
-    const SampleJob& jb = jobs[lo];
-    const uint64_t c = cg - jb.col0;
-    const V* a = static_cast<const V*>(jb.a0) + c * jb.col_stride;
-    const int top = jb.td.nlev - 1;
-    double total = 0.0;
-    for (uint64_t k = 0; k < jb.td.size[top]; ++k) total += tree_at(a, jb.td, top, k, c * jb.per_col);
-    tops[cg] = total;
 }
 
 // ------------------------------------------------------------- the queue
@@ -601,18 +653,24 @@ void ItemQueue::add_basis(const BasisItem& b)
     basis_.push_back(x);
 }
 
-size_t ItemQueue::add_sample(const SampleJob& job, const std::vector<LevelItem>& levels, const uint64_t* first,
-                             const double* u, size_t nruns)
+size_t ItemQueue::add_sample(const SampleJob& job, const uint64_t* first, const double* u, size_t nruns)
 {
-    if (job.td.nlev < 1 || job.td.nlev > 16 || levels.size() != size_t(job.td.nlev - 1) * size_t(job.ncols) ||
-        job.ncols < 1)
+    const int top = tree_top(job.nbits);
+    if (job.ncols < 1 || job.nbits < 0 || top > 3 * kTreeSteps)
         throw Error(ERR_INVALID_ARGUMENT, "sampling job: inconsistent tree");
-    for (size_t i = 0; i < levels.size(); ++i) {
-        const int l = int(i / size_t(job.ncols)) + 1;
-        LevelItem it = levels[i];
-        it.chunk0 = level_chunks_[l];
-        level_chunks_[l] += (it.size + kLevelChunk - 1) / kLevelChunk;
-        levels_[l].push_back(it);
+    for (int c = 0; c < job.ncols; ++c) {
+        double* const tree = const_cast<double*>(job.tree) + uint64_t(c) * job.per_col;
+        const char* a = static_cast<const char*>(job.a0) + uint64_t(c) * job.col_stride * (c64_ ? 8 : 16);
+        for (int l = 0, k = 0; l < top; l += 3, ++k) {
+            TreeItem it{};
+            it.in = l == 0 ? static_cast<const void*>(a) : tree + tree_offset(job.nbits, l);
+            it.out = tree + tree_offset(job.nbits, l + 1);
+            it.size = uint64_t(1) << (job.nbits - 4 * l);
+            it.levels = uint32_t(std::min(3, top - l));
+            it.chunk0 = tree_chunks_[k];
+            tree_chunks_[k] += (it.size + kTreeChunk - 1) / kTreeChunk;
+            tree_[k].push_back(it);
+        }
     }
     SampleJob j = job;
     j.first_off = first_.size();
@@ -633,7 +691,7 @@ void ItemQueue::release_after(void* p, size_t bytes, hipStream_t s)
 bool ItemQueue::empty() const
 {
     bool lv = false;
-    for (const auto& v : levels_) lv = lv || !v.empty();
+    for (const auto& v : tree_) lv = lv || !v.empty();
     return marg_.empty() && coll_.empty() && opit_.empty() && basis_.empty() && jobs_.empty() && !lv &&
            rel_.empty();
 }
@@ -642,30 +700,68 @@ static size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 
 void ItemQueue::launch(hipStream_t s)
 {
-    // layout: inputs, then outputs (partials, indices, tops)
-    size_t in = 0;
+    if (!marg_.empty() || !coll_.empty() || !opit_.empty() || !basis_.empty() || !jobs_.empty()) launch_items(s);
+    clear_inputs();
+}
+
+void ItemQueue::clear_inputs()
+{
+    // the kernels that read the released blocks are enqueued: stream order
+    // keeps later users of those blocks behind them
+    for (const Release& r : rel_) DeviceCache::get().release(r.p, r.bytes, r.s);
+    rel_.clear();
+    marg_.clear();
+    coll_.clear();
+    ops_.clear();
+    opit_.clear();
+    basis_.clear();
+    for (auto& v : tree_) v.clear();
+    jobs_.clear();
+    first_.clear();
+    u_.clear();
+    cols_ = 0;
+    marg_chunks_ = coll_chunks_ = op_chunks_ = basis_chunks_ = 0;
+    for (uint64_t& c : tree_chunks_) c = 0;
+}
+
+// What a launch moves besides the columns is small, and its cost is launches
+// and copies: a kernel of one item has it in its arguments, and up to
+// kHostBytes the kernels read the uniforms from pinned host memory and write
+// the results there, where a copy would be a launch of its own at either end.
+// A marginal of a 16-qubit state then is one launch, not three, and sampling it
+// two, not seven: 16 marginals or peeks and one sampling of 4096 runs of 16
+// complex64 qubits take 577 us, 845 us before; 21 marginals of 21 qubits 166 us
+// less.
+static constexpr size_t kHostBytes = size_t(1) << 20;
+
+void ItemQueue::launch_items(hipStream_t s)
+{
+    // the device buffer: the count of finished workgroups of a single
+    // marginal (zero between launches), inputs, partial sums, results
+    size_t in = 256;
     auto take = [&](size_t bytes) {
         const size_t o = in;
         in = up256(in + bytes);
         return o;
     };
-    const size_t o_marg = take(marg_.size() * sizeof(MargItem));
-    const size_t o_coll = take(coll_.size() * sizeof(CollItem));
+    auto many = [&](const auto& v) { return v.size() > 1 ? v.size() * sizeof(v[0]) : 0; };   // one: by argument
+    const size_t o_marg = take(many(marg_));
+    const size_t o_coll = take(many(coll_));
     const size_t o_ops = take(ops_.size() * sizeof(ColOp));
     const size_t o_opit = take(opit_.size() * sizeof(OpItem));
-    const size_t o_basis = take(basis_.size() * sizeof(BasisItem));
-    size_t o_lev[16] = {};
-    for (int l = 1; l < 16; ++l) o_lev[l] = take(levels_[l].size() * sizeof(LevelItem));
-    const size_t o_jobs = take(jobs_.size() * sizeof(SampleJob));
-    run0_.clear();
-    for (const SampleJob& j : jobs_) run0_.push_back(j.run0);
-    run0_.push_back(u_.size());
-    const size_t o_run0 = take(run0_.size() * sizeof(uint64_t));
-    const size_t o_first = take(first_.size() * sizeof(uint64_t));
-    const size_t o_u = take(u_.size() * sizeof(double));
-    const size_t o_done = take(marg_.size() * sizeof(uint32_t));       // zeros: finished workgroups per marginal
+    const size_t o_basis = take(many(basis_));
+    size_t o_tree[kTreeSteps];
+    for (int k = 0; k < kTreeSteps; ++k) o_tree[k] = take(many(tree_[k]));
+    const size_t o_jobs = take(many(jobs_));
+    const size_t o_done = take(marg_.size() > 1 ? marg_.size() * sizeof(uint32_t) : 0);   // zeros
+    const size_t u_bytes = up256(u_.size() * sizeof(double));
+    const bool u_host = u_bytes <= kHostBytes;
+    const size_t o_first = take(cols_ > jobs_.size() ? first_.size() * sizeof(uint64_t) : 0);   // not read for one column
+    const size_t o_u = u_host ? in : take(u_bytes);
+    const size_t up_bytes = in - 256;                                  // uploaded
+    const size_t in_bytes = o_u + u_bytes - 256;                       // of hin_
     const size_t o_part = take(marg_chunks_ * sizeof(double));         // device only
-    const size_t in_bytes = o_part, dev_bytes = in;
+    const size_t dev_bytes = in;
     size_t out = 0;
     const size_t p_w0 = out;
     out = up256(out + marg_.size() * sizeof(double));
@@ -674,9 +770,10 @@ void ItemQueue::launch(hipStream_t s)
     const size_t p_top = out;
     out = up256(out + cols_ * sizeof(double));
     const size_t out_bytes = out;
+    const bool out_host = out_bytes <= kHostBytes;
 
-    // buffers: wait for the previous upload before the host inputs are
-    // rewritten; grow the device buffer after the stream has drained
+    // buffers: wait for the previous launch's reads before the host inputs
+    // are rewritten; grow the device buffer after the stream has drained
     if (in_done_) IQ_OK(hipEventSynchronize(in_done_));
     else IQ_OK(hipEventCreateWithFlags(&in_done_, hipEventDisableTiming));
     if (dev_bytes + out_bytes > dcap_) {
@@ -687,126 +784,83 @@ void ItemQueue::launch(hipStream_t s)
         dcap_ = 0;
         const size_t cap = std::max<size_t>(dev_bytes + out_bytes, size_t(1) << 20) * 3 / 2;
         IQ_OK(hipMalloc(reinterpret_cast<void**>(&dbuf_), cap));
+        IQ_OK(hipMemsetAsync(dbuf_, 0, 256, s));
         dcap_ = cap;
     }
-    if (in_bytes > hin_cap_) {
-        if (hin_) IQ_OK(hipHostFree(hin_));
-        hin_ = nullptr;
-        hin_cap_ = 0;
-        const size_t cap = std::max<size_t>(in_bytes, size_t(1) << 20) * 3 / 2;
-        IQ_OK(hipHostMalloc(reinterpret_cast<void**>(&hin_), cap, hipHostMallocDefault));
-        hin_cap_ = cap;
-    }
-    if (out_bytes > hout_cap_) {
+    auto grow = [&](char*& host, char*& dev, size_t& have, size_t bytes) {
+        if (bytes <= have) return;
         if (last_stream_) IQ_OK(hipStreamSynchronize(last_stream_));
-        if (hout_) IQ_OK(hipHostFree(hout_));
-        hout_ = nullptr;
-        hout_cap_ = 0;
-        const size_t cap = std::max<size_t>(out_bytes, size_t(1) << 20) * 3 / 2;
-        IQ_OK(hipHostMalloc(reinterpret_cast<void**>(&hout_), cap, hipHostMallocDefault));
-        hout_cap_ = cap;
-    }
+        if (host) IQ_OK(hipHostFree(host));
+        host = dev = nullptr;
+        have = 0;
+        const size_t cap = std::max<size_t>(bytes, size_t(1) << 20) * 3 / 2;
+        IQ_OK(hipHostMalloc(reinterpret_cast<void**>(&host), cap, hipHostMallocDefault));
+        IQ_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&dev), host, 0));
+        have = cap;
+    };
+    grow(hin_, hin_dev_, hin_cap_, in_bytes);
+    grow(hout_, hout_dev_, hout_cap_, out_bytes);
     last_stream_ = s;
     auto put = [&](size_t off, const void* src, size_t bytes) {
-        if (bytes) std::memcpy(hin_ + off, src, bytes);
+        if (bytes) std::memcpy(hin_ + off - 256, src, bytes);
     };
-    put(o_marg, marg_.data(), marg_.size() * sizeof(MargItem));
-    put(o_coll, coll_.data(), coll_.size() * sizeof(CollItem));
+    put(o_marg, marg_.data(), many(marg_));
+    put(o_coll, coll_.data(), many(coll_));
     put(o_ops, ops_.data(), ops_.size() * sizeof(ColOp));
     put(o_opit, opit_.data(), opit_.size() * sizeof(OpItem));
-    put(o_basis, basis_.data(), basis_.size() * sizeof(BasisItem));
-    for (int l = 1; l < 16; ++l) put(o_lev[l], levels_[l].data(), levels_[l].size() * sizeof(LevelItem));
-    put(o_jobs, jobs_.data(), jobs_.size() * sizeof(SampleJob));
-    put(o_run0, run0_.data(), run0_.size() * sizeof(uint64_t));
-    put(o_first, first_.data(), first_.size() * sizeof(uint64_t));
+    put(o_basis, basis_.data(), many(basis_));
+    for (int k = 0; k < kTreeSteps; ++k) put(o_tree[k], tree_[k].data(), many(tree_[k]));
+    put(o_jobs, jobs_.data(), many(jobs_));
+    if (marg_.size() > 1) std::memset(hin_ + o_done - 256, 0, marg_.size() * sizeof(uint32_t));
+    if (cols_ > jobs_.size()) put(o_first, first_.data(), first_.size() * sizeof(uint64_t));
     put(o_u, u_.data(), u_.size() * sizeof(double));
-    if (!marg_.empty()) std::memset(hin_ + o_done, 0, marg_.size() * sizeof(uint32_t));
-    if (in_bytes) {
-        upload_table(dbuf_, hin_, in_bytes, s);
+    if (up_bytes) {
+        upload_table(dbuf_ + 256, hin_, up_bytes, s);
         launches_ += 1;
     }
-    IQ_OK(hipEventRecord(in_done_, s));
     char* d = dbuf_;
-    char* dout = dbuf_ + dev_bytes;
-    auto grid = [](uint64_t chunks) { return dim3(unsigned(std::min<uint64_t>(chunks, kMaxGrid))); };
-    if (!basis_.empty()) {
-        if (c64_) hipLaunchKernelGGL(k_basis_items<float2>, grid(basis_chunks_), dim3(kBlock), 0, s,
-                                     reinterpret_cast<const BasisItem*>(d + o_basis), uint32_t(basis_.size()), basis_chunks_);
-        else hipLaunchKernelGGL(k_basis_items<double2>, grid(basis_chunks_), dim3(kBlock), 0, s,
-                                reinterpret_cast<const BasisItem*>(d + o_basis), uint32_t(basis_.size()), basis_chunks_);
+    char* dout = out_host ? hout_dev_ : dbuf_ + dev_bytes;
+    auto table = [&](const auto& v, size_t off) {
+        using I = typename std::decay<decltype(v[0])>::type;
+        return v.size() > 1 ? reinterpret_cast<const I*>(d + off) : nullptr;
+    };
+    auto grid = [](uint64_t chunks, uint64_t cap) { return dim3(unsigned(std::min<uint64_t>(chunks, cap))); };
+    auto run = [&](auto kernel, dim3 g, int threads, auto... args) {
+        hipLaunchKernelGGL(kernel, g, dim3(unsigned(threads)), 0, s, args...);
         IQ_OK(hipGetLastError());
         launches_ += 1;
-    }
-    if (!coll_.empty()) {
-        if (c64_) hipLaunchKernelGGL(k_collapse_items<float2>, grid(coll_chunks_), dim3(kBlock), 0, s,
-                                     reinterpret_cast<const CollItem*>(d + o_coll), uint32_t(coll_.size()), coll_chunks_);
-        else hipLaunchKernelGGL(k_collapse_items<double2>, grid(coll_chunks_), dim3(kBlock), 0, s,
-                                reinterpret_cast<const CollItem*>(d + o_coll), uint32_t(coll_.size()), coll_chunks_);
-        IQ_OK(hipGetLastError());
-        launches_ += 1;
-    }
-    if (!opit_.empty()) {
-        const ColOp* dops = reinterpret_cast<const ColOp*>(d + o_ops);
-        if (c64_) hipLaunchKernelGGL(k_op_items<float2>, grid(op_chunks_), dim3(kBlock), 0, s,
-                                     reinterpret_cast<const OpItem*>(d + o_opit), uint32_t(opit_.size()), op_chunks_, dops);
-        else hipLaunchKernelGGL(k_op_items<double2>, grid(op_chunks_), dim3(kBlock), 0, s,
-                                reinterpret_cast<const OpItem*>(d + o_opit), uint32_t(opit_.size()), op_chunks_, dops);
-        IQ_OK(hipGetLastError());
-        launches_ += 1;
-    }
-    if (!marg_.empty()) {
-        // a workgroup per chunk, up to 2^20 of them (2^30 threads)
-        const dim3 g{unsigned(std::min<uint64_t>(marg_chunks_, uint64_t(1) << 20))};
-        const MargItem* mi = reinterpret_cast<const MargItem*>(d + o_marg);
-        double* part = reinterpret_cast<double*>(d + o_part);
-        uint32_t* done = reinterpret_cast<uint32_t*>(d + o_done);
-        double* w = reinterpret_cast<double*>(dout + p_w0);
-        if (c64_) hipLaunchKernelGGL(k_marginal_items<float2>, g, dim3(kMargThreads), 0, s, mi, uint32_t(marg_.size()),
-                                     marg_chunks_, part, done, w);
-        else hipLaunchKernelGGL(k_marginal_items<double2>, g, dim3(kMargThreads), 0, s, mi, uint32_t(marg_.size()),
-                                marg_chunks_, part, done, w);
-        IQ_OK(hipGetLastError());
-        launches_ += 1;
-    }
-    for (int l = 1; l < 16; ++l) {
-        if (levels_[l].empty()) continue;
-        const LevelItem* li = reinterpret_cast<const LevelItem*>(d + o_lev[l]);
-        const uint32_t nl = uint32_t(levels_[l].size());
-        if (l > 1) hipLaunchKernelGGL(k_level_items<double>, grid(level_chunks_[l]), dim3(kBlock), 0, s, li, nl,
-                                      level_chunks_[l]);
-        else if (c64_) hipLaunchKernelGGL(k_level_items<float2>, grid(level_chunks_[l]), dim3(kBlock), 0, s, li, nl,
-                                          level_chunks_[l]);
-        else hipLaunchKernelGGL(k_level_items<double2>, grid(level_chunks_[l]), dim3(kBlock), 0, s, li, nl,
-                                level_chunks_[l]);
-        IQ_OK(hipGetLastError());
-        launches_ += 1;
-    }
+    };
+    if (!basis_.empty())
+        run(c64_ ? k_basis_items<float2> : k_basis_items<double2>, grid(basis_chunks_, kMaxGrid), kBlock, basis_[0],
+            table(basis_, o_basis), uint32_t(basis_.size()), basis_chunks_);
+    if (!coll_.empty())
+        run(c64_ ? k_collapse_items<float2> : k_collapse_items<double2>, grid(coll_chunks_, kMaxGrid), kBlock, coll_[0],
+            table(coll_, o_coll), uint32_t(coll_.size()), coll_chunks_);
+    if (!opit_.empty())
+        run(c64_ ? k_op_items<float2> : k_op_items<double2>, grid(op_chunks_, kMaxGrid), kBlock,
+            reinterpret_cast<const OpItem*>(d + o_opit), uint32_t(opit_.size()), op_chunks_,
+            reinterpret_cast<const ColOp*>(d + o_ops));
+    // marginals and trees: a workgroup per chunk, up to 2^20 of them
+    if (!marg_.empty())
+        run(c64_ ? k_marginal_items<float2> : k_marginal_items<double2>, grid(marg_chunks_, uint64_t(1) << 20),
+            kMargThreads, marg_[0], table(marg_, o_marg), uint32_t(marg_.size()), marg_chunks_,
+            reinterpret_cast<double*>(d + o_part), reinterpret_cast<uint32_t*>(marg_.size() > 1 ? d + o_done : d),
+            reinterpret_cast<double*>(dout + p_w0));
+    for (int k = 0; k < kTreeSteps; ++k)
+        if (!tree_[k].empty())
+            run(k > 0 ? k_tree_items<double> : c64_ ? k_tree_items<float2> : k_tree_items<double2>,
+                grid(tree_chunks_[k], uint64_t(1) << 20), kBlock, tree_[k][0], table(tree_[k], o_tree[k]),
+                uint32_t(tree_[k].size()), tree_chunks_[k]);
     if (!jobs_.empty()) {
-        const SampleJob* dj = reinterpret_cast<const SampleJob*>(d + o_jobs);
-        const uint32_t nj = uint32_t(jobs_.size());
         const uint64_t nruns = u_.size();
-        uint64_t* idx = reinterpret_cast<uint64_t*>(dout + p_idx);
-        double* tops = reinterpret_cast<double*>(dout + p_top);
-        if (nruns) {
-            const dim3 g(unsigned((nruns + kBlock - 1) / kBlock));
-            if (c64_) hipLaunchKernelGGL(k_sample_items<float2>, g, dim3(kBlock), 0, s, dj, nj,
-                                         reinterpret_cast<const uint64_t*>(d + o_run0),
-                                         reinterpret_cast<const uint64_t*>(d + o_first),
-                                         reinterpret_cast<const double*>(d + o_u), nruns, idx);
-            else hipLaunchKernelGGL(k_sample_items<double2>, g, dim3(kBlock), 0, s, dj, nj,
-                                    reinterpret_cast<const uint64_t*>(d + o_run0),
-                                    reinterpret_cast<const uint64_t*>(d + o_first),
-                                    reinterpret_cast<const double*>(d + o_u), nruns, idx);
-            IQ_OK(hipGetLastError());
-            launches_ += 1;
-        }
-        const dim3 gt(unsigned((cols_ + kBlock - 1) / kBlock));
-        if (c64_) hipLaunchKernelGGL(k_top_items<float2>, gt, dim3(kBlock), 0, s, dj, nj, cols_, tops);
-        else hipLaunchKernelGGL(k_top_items<double2>, gt, dim3(kBlock), 0, s, dj, nj, cols_, tops);
-        IQ_OK(hipGetLastError());
-        launches_ += 1;
+        run(c64_ ? k_sample_items<float2> : k_sample_items<double2>,
+            dim3(unsigned((nruns + kBlock - 1) / kBlock + (cols_ + kBlock - 1) / kBlock)), kBlock, jobs_[0],
+            table(jobs_, o_jobs), uint32_t(jobs_.size()), reinterpret_cast<const uint64_t*>(d + o_first),
+            reinterpret_cast<const double*>(u_host ? hin_dev_ + o_u - 256 : d + o_u), nruns,
+            reinterpret_cast<uint64_t*>(dout + p_idx), cols_, reinterpret_cast<double*>(dout + p_top));
     }
-    if (out_bytes) {
+    if (in_bytes) IQ_OK(hipEventRecord(in_done_, s));
+    if (out_bytes && !out_host) {
         IQ_OK(hipMemcpyAsync(hout_, dout, out_bytes, hipMemcpyDeviceToHost, s));
         launches_ += 1;
     }
@@ -819,22 +873,6 @@ void ItemQueue::launch(hipStream_t s)
         res_run0_.push_back(j.run0);
         res_col0_.push_back(j.col0);
     }
-    // the kernels that read the released blocks are enqueued: stream order
-    // keeps later users of those blocks behind them
-    for (const Release& r : rel_) DeviceCache::get().release(r.p, r.bytes, r.s);
-    rel_.clear();
-    marg_.clear();
-    coll_.clear();
-    ops_.clear();
-    opit_.clear();
-    basis_.clear();
-    for (auto& v : levels_) v.clear();
-    jobs_.clear();
-    first_.clear();
-    u_.clear();
-    cols_ = 0;
-    marg_chunks_ = coll_chunks_ = op_chunks_ = basis_chunks_ = 0;
-    for (uint64_t& c : level_chunks_) c = 0;
 }
 
 char* ItemQueue::stage(size_t bytes, hipStream_t s)
@@ -875,20 +913,7 @@ void ItemQueue::detach()
     // destroyed and its handle reused: the next owner records a fresh one
     if (in_done_) (void)hipEventDestroy(in_done_);
     in_done_ = nullptr;
-    for (const Release& r : rel_) DeviceCache::get().release(r.p, r.bytes, r.s);
-    rel_.clear();
-    marg_.clear();
-    coll_.clear();
-    ops_.clear();
-    opit_.clear();
-    basis_.clear();
-    for (auto& v : levels_) v.clear();
-    jobs_.clear();
-    first_.clear();
-    u_.clear();
-    cols_ = 0;
-    marg_chunks_ = coll_chunks_ = op_chunks_ = basis_chunks_ = 0;
-    for (uint64_t& c : level_chunks_) c = 0;
+    clear_inputs();
 }
 
 namespace {
