@@ -223,6 +223,8 @@ public:
     // the state starts as the compact basis column |0..0> (no device memory
     // until gates need it)
     void set_zero_state_compact();
+    // a compact state written out in the middle of a flush
+    void write_zero_state() { materialize(); }
 
     // build-added
     void read_amplitudes(size_t col, cdouble* out);
@@ -425,6 +427,7 @@ private:
     void* small_buf(size_t bytes);
     double* partial_buf(size_t n);
     void materialize();
+    void forget_basis();   // the columns are dense from here on
     void apply_queue_plain(size_t col_begin, size_t col_end);
 };
 

@@ -667,17 +667,10 @@ void GpuVectorState::synchronize() { HIP_OK(hipStreamSynchronize(stream_)); }
 
 void GpuVectorState::set_zero_state()
 {
-    queue_.clear();
-    basis_ = false;
-    counts_.assign(1, nr_shots_);
+    // the column's memory is taken here and written by the first flush, or
+    // by what needs it written (materialize): sweeps start from |0..0> itself
+    set_zero_state_compact();
     alloc_cols(1);
-    HIP_OK(hipMemsetAsync(amp_, 0, dim() * elem_bytes(), stream_));
-    // static sources: the copies may run after this returns (same stream
-    // order for everything that follows, no wait needed)
-    static const double one64[2] = {1.0, 0.0};
-    static const float one32[2] = {1.0f, 0.0f};
-    if (prec_ == PREC_C128) HIP_OK(hipMemcpyAsync(amp_, one64, sizeof(one64), hipMemcpyHostToDevice, stream_));
-    else HIP_OK(hipMemcpyAsync(amp_, one32, sizeof(one32), hipMemcpyHostToDevice, stream_));
 }
 
 void GpuVectorState::set_product_state(const cdouble* coefs)
@@ -799,6 +792,11 @@ void GpuVectorState::materialize_enqueue(ItemQueue& q)
     const double mag = (nr_bits_ & 1) ? std::ldexp(0.70710678118654752440, -int(nr_bits_ / 2))
                                       : std::ldexp(1.0, -int(nr_bits_ / 2));
     for (size_t c = 0; c < nc; ++c) q.add_basis(BasisItem{col_ptr(c), dim(), basis_idx_[c], 0, mag, basis_rot_, 0});
+    forget_basis();
+}
+
+void GpuVectorState::forget_basis()
+{
     basis_ = false;
     basis_rot_ = 0;
     basis_idx_.clear();
@@ -825,13 +823,19 @@ void GpuVectorState::apply_unary_gate_all(const cdouble* mat2, const std::string
 void GpuVectorState::flush()
 {
     if (queue_.empty()) return;
-    materialize();
+    // a column |0..0> that nothing has written yet goes into the sweeps as it
+    // is; a captured or recorded flush, and the kernels that prefetch, have it
+    // written first
+    const bool fresh = basis_ && basis_rot_ == 0 && basis_idx_.size() == 1 && basis_idx_[0] == 0 && amp_ &&
+                       tiling_ && !graph_on_ && !recording_ && !jit_prefetch();
+    if (!fresh) materialize();
     auto t0 = std::chrono::steady_clock::now();
     stats_ = RunStats{};
     if (fusion_k_ > 0 || tiling_)
-        run_planned(*this, queue_, 0, counts_.size(), fusion_k_, tiling_, stats_);
+        run_planned(*this, queue_, 0, counts_.size(), fusion_k_, tiling_, fresh, stats_);
     else
         apply_queue_plain(0, counts_.size());
+    if (fresh) forget_basis();
     HIP_OK(hipStreamSynchronize(stream_));
     staged_done();
     stats_.gate_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

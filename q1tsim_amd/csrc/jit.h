@@ -30,8 +30,9 @@ const char* jit_kernel_name(bool c64);
 // op_begin.
 // `prefetch`: software-pipelined tiles -- a thread's share of the next tile
 // is loaded into registers while the phases of the current one run.
+// `unset`: for launches with SweepArgs::unset bits (without prefetch).
 std::string jit_sweep_source(const std::vector<SwPhase>& phases, const std::vector<SwOp>& ops, bool c64, int M,
-                             int R, int SW, bool prefetch = false);
+                             int R, int SW, bool prefetch = false, bool unset = false);
 
 // Compile a source with hipRTC for gfx950 (no device needed); returns the
 // code object, or throws with the compiler log.

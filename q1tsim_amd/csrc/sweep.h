@@ -129,8 +129,9 @@ std::vector<std::string> plan_jit_sources(const std::vector<PendingGate>& q, int
 // Apply the pending gates to columns [col_begin, col_end) of the state with
 // the planned schedule: runs of gates whose qubits fit one tile are applied
 // in one HBM sweep; `fusion_k` > 0 composes runs into dense blocks of at most
-// that many qubits first (complex64 path).
+// that many qubits first (complex64 path).  `fresh`: the state is one column
+// |0..0> that is not in memory (tiling only).
 void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
-                 int fusion_k, bool tiling, RunStats& stats);
+                 int fusion_k, bool tiling, bool fresh, RunStats& stats);
 
 }  // namespace q1t

@@ -45,7 +45,9 @@ template <typename V> __device__ __forceinline__ void warm_sweep(const SweepArgs
     if (sa.nops) warm_program(sa.ops, sa.nops * uint32_t(sizeof(InterpOpT<typename RealOf<V>::type>)));
 }
 
-template <typename V, int M, int R, int SW, int BLK>
+// UNSET: launches with SweepArgs::unset bits, in a kernel of their own (the
+// load that takes them costs the sweeps without).
+template <typename V, int M, int R, int SW, int BLK, bool UNSET>
 __global__ void __launch_bounds__(1 << (M - R))
 __attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 && M == 12 ? (R == 3 ? 4 : 3) : 2)))
 k_sweep(V* __restrict__ amp, uint64_t col_stride, SweepArgs sa)
@@ -53,7 +55,7 @@ k_sweep(V* __restrict__ amp, uint64_t col_stride, SweepArgs sa)
     __shared__ V lds[1 << M];
     V* a = amp + uint64_t(blockIdx.y) * col_stride;
     warm_sweep<V>(sa);
-    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK>(a, sa, tile, lds);
+    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK, UNSET>(a, sa, tile, lds);
 }
 
 // Sweeps of many states in one launch: item i covers flattened tiles
@@ -95,7 +97,7 @@ k_sweep_batched(const SweepItem* __restrict__ items, int nitems, uint64_t total_
             const SweepItem& it = items[lo];
             const uint64_t lt = t - it.first_tile;
             V* a = static_cast<V*>(it.amp) + (lt >> it.log_ntiles) * it.col_stride;
-            sweep_tile<V, M, R, SW, BLK>(a, it.sa, lt & ((uint64_t(1) << it.log_ntiles) - 1), lds);
+            sweep_tile<V, M, R, SW, BLK, false>(a, it.sa, lt & ((uint64_t(1) << it.log_ntiles) - 1), lds);
         }
     }
 }
@@ -115,7 +117,7 @@ static void launch_batched_c64(int blk, unsigned gx, hipStream_t stream, const S
 template <typename V, int M, int R, int SW>
 static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase* dphases, int nphases,
                          const SwOp* dops, int nops, const float* dblocks, size_t cb, size_t ce, int blk,
-                         hipFunction_t jit = nullptr)
+                         uint64_t unset, double bytes, hipFunction_t jit = nullptr)
 {
     const int n = int(st.nr_bits());
     SweepArgs sa{};
@@ -130,12 +132,15 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
     sa.blocks = dblocks;
     sa.nphases = nphases;
     sa.nops = uint32_t(nops);
+    sa.unset = unset;
     const uint64_t dim = uint64_t(1) << n;
     // far more workgroups than the chip holds (1024): they start as others
     // finish, and loads, stores and arithmetic of neighbours spread out in
     // time.  28 qubits complex64, 10 sweeps: 512 workgroups 27.4 ms, 2048 18.7,
     // 16384 17.1, one per tile 17.4; specialised kernels, 30 qubits complex128:
     // 2048 89.0 ms, 16384 85.2.
+    // Sweeps that skip tiles too: one workgroup per tile costs them 0.9 ms at
+    // 2^18 tiles.
     const unsigned gx = unsigned(std::min<uint64_t>(sa.ntiles, 16384));
     int first = -1;
     for (size_t c0 = cb; c0 < ce; c0 += 65535) {
@@ -149,22 +154,18 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
             void* args[] = {&amp, &stride, &sa};
             SW_HIP_OK(hipModuleLaunchKernel(jit, gx, ny, 1, 1u << (M - R), 1, 1, 0, st.stream(), args, nullptr));
             st.prof_end(ps, sizeof(V) == 16 ? "q1t_jit_sweep_c128" : "q1t_jit_sweep_c64",
-                        2.0 * double(dim) * sizeof(V) * ny);
+                        bytes * ny);
             continue;
         }
         V* amp = static_cast<V*>(st.col_ptr(c0));
+        auto k = unset ? k_sweep<V, M, R, SW, 0, true> : k_sweep<V, M, R, SW, 0, false>;
         if constexpr (sizeof(V) == 8) {
-            if (blk == 2)
-                hipLaunchKernelGGL((k_sweep<V, M, R, SW, 2>), dim3(gx, ny), dim3(1 << (M - R)), 0, st.stream(), amp, dim, sa);
-            else if (blk == 1)
-                hipLaunchKernelGGL((k_sweep<V, M, R, SW, 1>), dim3(gx, ny), dim3(1 << (M - R)), 0, st.stream(), amp, dim, sa);
-            else
-                hipLaunchKernelGGL((k_sweep<V, M, R, SW, 0>), dim3(gx, ny), dim3(1 << (M - R)), 0, st.stream(), amp, dim, sa);
-        } else {
-            hipLaunchKernelGGL((k_sweep<V, M, R, SW, 0>), dim3(gx, ny), dim3(1 << (M - R)), 0, st.stream(), amp, dim, sa);
+            if (blk == 2) k = unset ? k_sweep<V, M, R, SW, 2, true> : k_sweep<V, M, R, SW, 2, false>;
+            else if (blk == 1) k = unset ? k_sweep<V, M, R, SW, 1, true> : k_sweep<V, M, R, SW, 1, false>;
         }
+        hipLaunchKernelGGL(k, dim3(gx, ny), dim3(1 << (M - R)), 0, st.stream(), amp, dim, sa);
         SW_HIP_OK(hipGetLastError());
-        st.prof_end(ps, sizeof(V) == 16 ? "k_sweep_c128" : "k_sweep_c64", 2.0 * double(dim) * sizeof(V) * ny);
+        st.prof_end(ps, sizeof(V) == 16 ? "k_sweep_c128" : "k_sweep_c64", bytes * ny);
     }
     return first;
 }
@@ -232,8 +233,8 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
 #pragma unroll
         for (int k = 0; k < NR; ++k) {
             const uint32_t l = tid + uint32_t(k) * nth;
-            x[k] = mkc<V>(0, 0);
-            if (l < N) x[k] = a[l];
+            x[k] = mkc<V>(it.fresh && l == 0 ? 1 : 0, 0);
+            if (l < N && !it.fresh) x[k] = a[l];
         }
 #pragma unroll
         for (int k = 0; k < NR; ++k) s[swizzle_slot(sw, M, int(tid + uint32_t(k) * nth))] = x[k];
@@ -682,7 +683,7 @@ static void run_table(GpuVectorState& st, const char* host, size_t total, std::v
 // no register phase takes.
 template <typename V>
 static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
-                      RunStats& stats)
+                      bool fresh, RunStats& stats)
 {
     using R = typename RealOf<V>::type;
     const int n = int(st.nr_bits());
@@ -701,7 +702,9 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
     WholeItem* items = reinterpret_cast<WholeItem*>(host + ioff);   // step-major
     for (size_t s = 0; s < steps.size(); ++s)
         for (size_t c = 0; c < ncols; ++c)
-            items[s * ncols + c] = WholeItem{st.col_ptr(col_begin + c), uint32_t(n), wt.nph[s], wt.ph0[s], wt.op0[s]};
+            items[s * ncols + c] = WholeItem{st.col_ptr(col_begin + c), uint32_t(n), wt.nph[s], wt.ph0[s], wt.op0[s],
+                                             fresh && s == 0, 0};
+    if (fresh && (steps.empty() || !steps[0].sweep)) st.write_zero_state();
     const double S = double(uint64_t(1) << n) * sizeof(V) * double(ncols);
     auto launch_all = [&](char* d) {
         for (size_t s = 0; s < steps.size(); ++s) {
@@ -737,7 +740,7 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
 }
 
 void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
-                 int fusion_k, bool tiling, RunStats& stats)
+                 int fusion_k, bool tiling, bool fresh, RunStats& stats)
 {
     const int n = int(st.nr_bits());
     TileGeom g = st.geometry();
@@ -746,8 +749,8 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         return;
     }
     if (n < g.M + 2) {
-        if (st.precision() == PREC_C128) run_whole<double2>(st, queue, col_begin, col_end, stats);
-        else run_whole<float2>(st, queue, col_begin, col_end, stats);
+        if (st.precision() == PREC_C128) run_whole<double2>(st, queue, col_begin, col_end, fresh, stats);
+        else run_whole<float2>(st, queue, col_begin, col_end, fresh, stats);
         return;
     }
     const double S = double(uint64_t(1) << n) * double(st.elem_bytes()) * double(col_end - col_begin);
@@ -790,6 +793,28 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             std::memcpy(host + boff + boff_s[s] * sizeof(float), progs[s].blocks.data(),
                         progs[s].blocks.size() * sizeof(float));
     }
+    // A state still |0..0> (`fresh`, one column, none of it in memory): each
+    // sweep's unset bits, and the bytes a column moves.  Gates between sweeps
+    // and bits that no sweep reaches need the zeros in memory.
+    std::vector<uint64_t> unset(steps.size(), 0);
+    std::vector<double> col_bytes(steps.size(), 2.0 * std::ldexp(double(st.elem_bytes()), n));
+    if (fresh) {
+        const uint64_t all = (uint64_t(1) << n) - 1;
+        uint64_t un = ~uint64_t(0);
+        bool zeros = false;
+        for (size_t s = 0; s < steps.size(); ++s) {
+            if (!steps[s].sweep) {
+                zeros = zeros || un != 0;
+                un = 0;
+                continue;
+            }
+            unset[s] = un & all ? un : 0;
+            const double read = un == ~uint64_t(0) ? 0.0 : std::ldexp(1.0, __builtin_popcountll(~un & all));
+            for (int b : steps[s].tile) un &= ~(uint64_t(1) << b);
+            col_bytes[s] = (read + std::ldexp(1.0, __builtin_popcountll(~un & all))) * double(st.elem_bytes());
+        }
+        if (zeros || (un & all)) st.write_zero_state();
+    }
     // kernels specialised to each sweep's program (compiled on first use)
     std::vector<hipFunction_t> jitfn(steps.size(), nullptr);
     if (st.jit_enabled()) {
@@ -798,7 +823,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
         for (size_t s = 0; s < steps.size(); ++s)
             if (steps[s].sweep) {
                 src[s] = jit_sweep_source(progs[s].phases, progs[s].ops, st.precision() == PREC_C64, g.M, g.R,
-                                          sweep_swizzle_bits(g.M), st.jit_prefetch());
+                                          sweep_swizzle_bits(g.M), st.jit_prefetch(), unset[s] != 0);
                 all.push_back(src[s]);
             }
         JitCache& jc = JitCache::get();
@@ -827,15 +852,15 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             const int shape = g.M * 16 + g.R;
             if (st.precision() == PREC_C128) {
                 switch (shape) {
-                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, jf); break;
-                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, jf); break;
+                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, unset[s], col_bytes[s], jf); break;
+                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, unset[s], col_bytes[s], jf); break;
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex128 tile shape");
                 }
             } else {
                 switch (shape) {
-                case 13 * 16 + 4: slot = launch_sweep<float2, 13, 4, 5>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
-                case 12 * 16 + 3: slot = launch_sweep<float2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
-                case 12 * 16 + 4: slot = launch_sweep<float2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, jf); break;
+                case 13 * 16 + 4: slot = launch_sweep<float2, 13, 4, 5>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, unset[s], col_bytes[s], jf); break;
+                case 12 * 16 + 3: slot = launch_sweep<float2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, unset[s], col_bytes[s], jf); break;
+                case 12 * 16 + 4: slot = launch_sweep<float2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, unset[s], col_bytes[s], jf); break;
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex64 tile shape");
                 }
             }
@@ -847,7 +872,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             stats.launches += 1;
             stats.sweeps += 1;
             stats.gates += step.gates.size();
-            stats.bytes += 2.0 * S;
+            stats.bytes += col_bytes[s] * double(col_end - col_begin);
             stats.phases += progs[s].phases.size();
             for (const SwPhase& ph : progs[s].phases)
                 if (ph.kind == 1)
@@ -1152,7 +1177,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
                             for (size_t c = 0; c < st.nr_cols(); ++c)
                                 it[witem[s][i] + c] =
                                     WholeItem{st.col_ptr(c), uint32_t(st.nr_bits()), wt.nph[s],
-                                              uint32_t(wpbase[i]) + wt.ph0[s], uint32_t(wobase[i]) + wt.op0[s]};
+                                              uint32_t(wpbase[i]) + wt.ph0[s], uint32_t(wobase[i]) + wt.op0[s], 0, 0};
                         }
                     };
                     if (prec == PREC_C128) copy(p.wd);

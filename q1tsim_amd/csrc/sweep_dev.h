@@ -18,6 +18,7 @@ struct SweepArgs {
     const float* blocks;   // real-embedded block matrices (fused segments)
     int nphases;
     uint32_t nops;
+    uint64_t unset;        // see sweep_tile
 };
 
 // p[i] read through the constant address space: wave-uniform scalar loads
@@ -637,8 +638,26 @@ __device__ __forceinline__ void tile_phases(V* __restrict__ a, const SweepArgs& 
     }
 }
 
+// A sweep of a state that started as |0..0> and has not reached every index
+// bit yet: amplitudes with a bit of `unset` in their index are zero and not
+// in memory.  Tiles at such an index are skipped, such amplitudes of the other
+// tiles are taken as zero, and the tile is written whole, which makes its bits
+// set.  unset = ~0 is |0..0> itself, of which nothing is in memory.  The first
+// sweeps of a circuit then cost what they reach: 12 bits and a tile's bits
+// more per sweep (about 8), so that a 28-qubit state pays two sweeps less and
+// writes no zeros first (20 layers, specialised kernels: 30 qubits complex128
+// with 4096 shots 147.9 -> 133.3 ms, 28 qubits complex64 with 28 marginals
+// 24.1 -> 21.3 ms; 23 qubits complex128 with shots 2.21 -> 2.10 ms).  Every lane loads, from the amplitude without the
+// unset bits where its own is zero: a branch around each load would serialise
+// them.
+template <typename V> __device__ __forceinline__ V load_set(const V* a, uint64_t base, uint64_t off, uint64_t unset)
+{
+    const V x = load_stream(a + (base | (off & ~unset)));
+    return off & unset ? mkc<V>(0, 0) : unset == ~uint64_t(0) ? mkc<V>(1, 0) : x;
+}
+
 // One tile of a sweep: HBM -> LDS, the program's phases, LDS -> HBM.
-template <typename V, int M, int R, int SW, int BLK>
+template <typename V, int M, int R, int SW, int BLK, bool UNSET>
 __device__ __forceinline__ void sweep_tile(V* __restrict__ a, const SweepArgs& sa, uint64_t tile, V* lds)
 {
     constexpr int NT = 1 << (M - R), NR = 1 << R;
@@ -646,8 +665,15 @@ __device__ __forceinline__ void sweep_tile(V* __restrict__ a, const SweepArgs& s
     tile_addr<M, R>(sa, ta);
     const uint64_t base = deposit(tile, sa.tset);
     const int s0 = tile_slot_base<SW, M>();
+    if constexpr (UNSET) {
+        if (base & sa.unset) return;
 #pragma unroll
-    for (int k = 0; k < NR; ++k) lds[s0 ^ swz<SW, M>(k * NT)] = load_stream(a + (base | ta.g_tid | ta.g_k[k]));
+        for (int k = 0; k < NR; ++k)
+            lds[s0 ^ swz<SW, M>(k * NT)] = load_set(a, base, ta.g_tid | ta.g_k[k], sa.unset);
+    } else {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) lds[s0 ^ swz<SW, M>(k * NT)] = load_stream(a + (base | ta.g_tid | ta.g_k[k]));
+    }
     __syncthreads();
     tile_phases<V, M, R, SW, BLK>(a, sa, base, lds, ta);
 }

@@ -124,6 +124,7 @@ struct WholeItem {
     uint32_t n;          // qubits
     uint32_t nphases;
     uint32_t phases, ops;   // first records in the tables
+    uint32_t fresh, pad;    // 1: the column is |0..0> and not in memory yet
 };
 
 }  // namespace q1t
