@@ -55,6 +55,8 @@ static void emit_register_phase(std::ostringstream& o, const SwPhase& ph, const 
         o << "        " << (noops ? "const V " : "") << vname << k << vend << " = lds[st ^ " << srp[k] << "];\n";
     }
     o << "        __builtin_amdgcn_s_setprio(0);\n";
+    for (uint32_t oi = ph.op_begin; oi < ph.op_end; ++oi)
+        if (ops[oi].type == SW_APPLY) o << "        V lane = mkc<V>(1, 0);\n";   // one per phase at most
     for (uint32_t oi = ph.op_begin; oi < ph.op_end; ++oi) {
         const SwOp& op = ops[oi];
         o << "        {\n";
@@ -65,12 +67,25 @@ static void emit_register_phase(std::ostringstream& o, const SwPhase& ph, const 
         }
         if (op.ct) o << ind << "const bool tok = (uint32_t(tid) & " << op.ct << "u) == " << op.ct << "u;\n";
         else o << ind << "const bool tok = true;\n";
+        if (op.type == SW_APPLY) {
+            o << ind << "scale_regs_t<V, NR, false, false>(v, 0u, true, [&](int, V x) { return cmul(lane, x); });\n";
+            o << "        }\n";
+            continue;
+        }
         o << ind << "const SwOp op = load_uniform(ops, " << oi << "u);\n";
         const std::string TC = op.ct ? "true" : "false";
         if (op.type == SW_DENSE1) {
             const uint32_t form = op.aux;
             const bool single_rc = op.cr != 0 && (op.cr & (op.cr - 1)) == 0;
-            if (form == SWF_SWAP && single_rc) {
+            if (form >= SWF_ROT_D) {
+                // which entry was divided out depends on the angle: both bodies
+                const uint32_t d = form - uint32_t(op.dreg);
+                o << ind << "const V t = mkc<V>(opm<V>(op, 0).x, 0);\n";
+                o << ind << "if (op.dreg) dense_pairs<V, NR, " << op.reg << ", " << d + 1
+                  << ", false, false>(v, 0u, true, t, t, t, t);\n";
+                o << ind << "else dense_pairs<V, NR, " << op.reg << ", " << d
+                  << ", false, false>(v, 0u, true, t, t, t, t);\n";
+            } else if (form == SWF_SWAP && single_rc) {
                 const int cb = __builtin_ctz(op.cr);
                 o << ind << "const V z = mkc<V>(0, 0);\n";
                 o << ind << "dense_pairs<V, NR, " << op.reg << ", SWF_SWAP, " << TC << ", false, " << cb
@@ -84,6 +99,15 @@ static void emit_register_phase(std::ostringstream& o, const SwPhase& ph, const 
                 o << ind << "dense_pairs<V, NR, " << op.reg << ", " << form << ", " << TC << ", " << RC << ">(v, "
                   << op.cr << "u, tok, m0, m1, m2, m3);\n";
             }
+        } else if (op.reg) {   // a factor of the thread's product
+            std::string f = "opm<V>(op, 0)";
+            if (op.type == SW_DIAG1) {
+                if (op.dtid >= 0) o << ind << "const bool one = ((tid >> " << op.dtid << ") & 1) != 0;\n";
+                else o << ind << "const bool one = ((base >> " << op.dglobal << ") & 1) != 0;\n";
+                f = "sel(one, opm<V>(op, 1), opm<V>(op, 0))";
+            }
+            if (op.ct) f = "sel(tok, " + f + ", mkc<V>(1, 0))";
+            o << ind << "lane = cmul(" << f << ", lane);\n";
         } else if (op.type == SW_PHASE) {
             o << ind << "phase_op<V, NR>(" << op.aux << "u, v, " << op.cr << "u, " << op.ct
               << "u, tok, opm<V>(op, 0));\n";

@@ -762,6 +762,95 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
     append_factors(tf, M, phases, ops, order);
 }
 
+// A gate's largest entry is at least 2^-1/2 for what reduce_op takes: after
+// this many gates the amplitudes have grown by at most 2^40 (complex64), 2^400.
+static int reduction_limit(Precision prec) { return prec == PREC_C128 ? 800 : 80; }
+
+static void set_coefs(SwOp& o, cdouble a)
+{
+    for (int k = 0; k < 8; ++k) o.m[k] = 0;
+    o.m[0] = a.real();
+    o.m[1] = a.imag();
+    for (int k = 0; k < 8; ++k) o.mf[k] = float(o.m[k]);
+}
+
+static void reduce_op(SwOp& o, Reduction& red)
+{
+    if (o.cr || o.ct || o.co) return;
+    auto unit = [](double x) { return x > 0.75 && x < 1.5; };   // squared norm of a unitary's row, with room
+    if (o.type == SW_DIAG1 && o.dreg >= 0) {
+        const cdouble d0(o.m[0], o.m[1]), d1(o.m[2], o.m[3]);
+        if (!unit(std::norm(d0))) return;
+        red.factor *= std::complex<long double>(d0.real(), d0.imag());
+        red.gates += 1;
+        o.type = SW_PHASE;
+        o.aux = SWP_GENERAL;
+        o.cr = 1u << o.dreg;
+        o.dreg = -1;
+        set_coefs(o, d1 / d0);
+        return;
+    }
+    if (o.type != SW_DENSE1 || (o.aux != SWF_REAL && o.aux != SWF_RX)) return;
+    const bool rx = o.aux == SWF_RX;
+    const double a = o.m[0], b = rx ? o.m[3] : o.m[4];   // m00; m01 / i or m10
+    const bool rot = !rx && o.m[6] == a && o.m[2] == -b, refl = !rx && o.m[6] == -a && o.m[2] == b;
+    if ((!rx && !rot && !refl) || !unit(a * a + b * b)) return;
+    const bool off = std::fabs(b) > std::fabs(a);
+    o.aux = (rx ? SWF_RX_D : rot ? SWF_ROT_D : SWF_REFL_D) + (off ? 1 : 0);
+    o.dreg = off ? 1 : 0;
+    if (off) red.factor *= rx ? std::complex<long double>(0, b) : std::complex<long double>(b, 0);
+    else red.factor *= std::complex<long double>(a, 0);
+    red.gates += 1;
+    set_coefs(o, off ? a / b : b / a);
+}
+
+void reduce_program(std::vector<SwPhase>& phases, std::vector<SwOp>& ops, Precision prec, Reduction& red, bool last)
+{
+    std::vector<SwOp> out;
+    out.reserve(ops.size() + 2 * phases.size());
+    auto put_factor = [&] {
+        SwOp o;
+        std::memset(&o, 0, sizeof(o));
+        o.type = SW_PHASE;
+        o.dreg = o.dtid = o.dglobal = -1;
+        set_coefs(o, cdouble(double(red.factor.real()), double(red.factor.imag())));
+        out.push_back(o);
+        red = Reduction();
+    };
+    size_t last_phase = phases.size();
+    for (size_t p = 0; p < phases.size(); ++p)
+        if (phases[p].kind == 0) last_phase = p;
+    for (size_t p = 0; p < phases.size(); ++p) {
+        SwPhase& ph = phases[p];
+        const size_t begin = out.size();
+        for (uint32_t i = ph.op_begin; i < ph.op_end; ++i) {
+            out.push_back(ops[i]);
+            if (ph.kind != 0) continue;
+            reduce_op(out.back(), red);
+            if (red.gates >= reduction_limit(prec)) put_factor();
+        }
+        if (ph.kind == 0) {
+            if (last && p == last_phase && red.gates) put_factor();
+            auto lane = [](const SwOp& o) {
+                return o.cr == 0 && (o.type == SW_PHASE || (o.type == SW_DIAG1 && o.dreg < 0));
+            };
+            size_t n = 0;
+            for (size_t i = begin; i < out.size(); ++i) n += lane(out[i]);
+            if (n > 1) {
+                for (size_t i = begin; i < out.size(); ++i)
+                    if (lane(out[i])) out[i].reg = 1;
+                SwOp o;
+                std::memset(&o, 0, sizeof(o));
+                o.type = SW_APPLY;
+                out.push_back(o);
+            }
+        }
+        ph.op_begin = uint32_t(begin);
+        ph.op_end = uint32_t(out.size());
+    }
+    ops.swap(out);
+}
+
 template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq)
 {
     InterpOpT<R> w;
@@ -771,10 +860,13 @@ template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq)
     if (o.type == SW_DENSE1) {
         if (o.aux == SWF_REAL || o.aux == SWF_SWAP) w.code = seq ? SWF_REAL_SEQ : SWF_REAL;
         else if (o.aux == SWF_RX) w.code = seq ? SWF_RX_SEQ : SWF_RX;
+        else if (o.aux >= SWF_ROT_D) w.code = o.aux;
         else w.code = SWF_GENERAL;
         w.code |= uint32_t(o.reg) << 8;
     } else if (o.type == SW_PHASE) {
         w.code = kInterpPhase;
+    } else if (o.type == SW_APPLY) {
+        w.code = kInterpApply;
     } else if (o.dreg >= 0) {
         w.code = kInterpDiagReg | uint32_t(o.dreg) << 8;
     } else if (o.dtid >= 0) {
@@ -782,6 +874,7 @@ template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq)
     } else {
         w.code = kInterpDiagOuter | uint32_t(o.dglobal) << 16;
     }
+    if ((o.type == SW_PHASE || o.type == SW_DIAG1) && o.reg) w.code |= kInterpLane;
     for (int k = 0; k < 8; ++k) w.m[k] = R(o.m[k]);
     return w;
 }

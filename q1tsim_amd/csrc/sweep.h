@@ -1,6 +1,7 @@
 // Gate-stream planner and multi-gate sweeps (LDS/register tiles, fused blocks).
 #pragma once
 
+#include <complex>
 #include <string>
 #include <vector>
 
@@ -49,6 +50,27 @@ std::vector<uint64_t> plan_key(const std::vector<PendingGate>& q, int n, const T
 void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int M, int R,
                    std::vector<SwPhase>& phases, std::vector<SwOp>& ops, bool search = true,
                    std::vector<size_t>* order = nullptr, bool factors = false);
+
+// The factor that reduce_program has taken out of a flush's gates so far, and
+// the number of gates it comes from.
+struct Reduction {
+    std::complex<long double> factor{1, 0};
+    int gates = 0;
+};
+// The same sweep in fewer operations per amplitude, for kernels bound by them:
+// uncontrolled rotations, reflections (H) and RX gates without their larger
+// entry, uncontrolled diagonal gates on a register bit as the phase of its ones,
+// and the factors that depend only on thread and outer bits multiplied per
+// thread and applied once per phase.  The common factor is applied at the end
+// of the program if `last`, and before it could leave the precision's range.
+// The structure does not depend on the gates' angles.
+// Measured: specialised kernels, 20 layers, 30 qubits complex128 133.3 -> 115.9
+// ms, 28 qubits complex64 21.3 -> 19.0 ms (the sweeps of many gates are bound by
+// FP64 issue: 154 ops on 2^18 tiles 15 ms); interpreted, 12 layers of 24 qubits
+// 1866 -> 1695 us complex128, 1033 -> 979 us complex64.  Errors against 64-bit
+// arithmetic fall with the roundings: 28 qubits complex64 4.3e-6 -> 1.5e-6.
+// Batches keep the gates' own forms.
+void reduce_program(std::vector<SwPhase>& phases, std::vector<SwOp>& ops, Precision prec, Reduction& red, bool last);
 
 // An op as the interpreting kernels take it; `seq`: whole-state programs.
 template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq);

@@ -47,15 +47,17 @@ template <typename V> __device__ __forceinline__ void warm_sweep(const SweepArgs
 
 // UNSET: launches with SweepArgs::unset bits, in a kernel of their own (the
 // load that takes them costs the sweeps without).
+// complex64 with 16 amplitudes per thread is held to 4 waves per SIMD, at the
+// price of 44 bytes of scratch: 24 qubits 979 us, at 3 waves 1092 us.
 template <typename V, int M, int R, int SW, int BLK, bool UNSET>
 __global__ void __launch_bounds__(1 << (M - R))
-__attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 && M == 12 ? (R == 3 ? 4 : 3) : 2)))
+__attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 && M == 12 ? (R == 3 || BLK == 0 ? 4 : 3) : 2)))
 k_sweep(V* __restrict__ amp, uint64_t col_stride, SweepArgs sa)
 {
     __shared__ V lds[1 << M];
     V* a = amp + uint64_t(blockIdx.y) * col_stride;
     warm_sweep<V>(sa);
-    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK, UNSET>(a, sa, tile, lds);
+    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK, BLK == 0, UNSET>(a, sa, tile, lds);
 }
 
 // Sweeps of many states in one launch: item i covers flattened tiles
@@ -97,7 +99,7 @@ k_sweep_batched(const SweepItem* __restrict__ items, int nitems, uint64_t total_
             const SweepItem& it = items[lo];
             const uint64_t lt = t - it.first_tile;
             V* a = static_cast<V*>(it.amp) + (lt >> it.log_ntiles) * it.col_stride;
-            sweep_tile<V, M, R, SW, BLK, false>(a, it.sa, lt & ((uint64_t(1) << it.log_ntiles) - 1), lds);
+            sweep_tile<V, M, R, SW, BLK, false, false>(a, it.sa, lt & ((uint64_t(1) << it.log_ntiles) - 1), lds);
         }
     }
 }
@@ -251,12 +253,13 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
         for (int k = 0; k < NR; ++k) v[k] = s[tin ^ (ph.slot[k] & 0xffffu)];
         const uint32_t o1 = it.ops + ph.op_end;
         uint32_t oi = it.ops + ph.op_begin;
+        V lane = mkc<V>(1, 0);
         InterpOpT<typename RealOf<V>::type> nxt = load_uniform(ops, oi);   // the table ends with a spare record
         while (oi < o1) {
             const InterpOpT<typename RealOf<V>::type> op = nxt;
             ++oi;
             nxt = load_uniform(ops, oi);
-            interp_op<V, NR, R, true>(op, v, tid, 0);
+            interp_op<V, NR, R, true, false>(op, v, tid, 0, lane);
         }
         if (ph.wmap == 0) {
 #pragma unroll
@@ -338,6 +341,21 @@ static SweepProgram build_candidate(const std::vector<PendingGate>& q, const Pla
     if (kind == 0) build_program(q, step, g.M, g.R, p.phases, p.ops, search, nullptr, factors);
     else build_fused_program(q, step, g.M, g.R, kind, p.phases, p.ops, p.blocks, &p.nblocks, search, factors);
     return p;
+}
+
+// The reduced programs of a flush (sweeps with dense blocks stay as they are):
+// the factor taken out of the gates goes back in with the last of them that
+// has a register phase.
+static void reduce_programs(std::vector<SweepProgram>& progs, Precision prec)
+{
+    size_t last = progs.size();
+    for (size_t s = 0; s < progs.size(); ++s)
+        if (block_level(progs[s].phases) == 0)
+            for (const SwPhase& ph : progs[s].phases)
+                if (ph.kind == 0) last = s;
+    Reduction red;
+    for (size_t s = 0; s < progs.size(); ++s)
+        if (block_level(progs[s].phases) == 0) reduce_program(progs[s].phases, progs[s].ops, prec, red, s == last);
 }
 
 // Wall-time estimate of a gate applied on its own: one read and one write
@@ -575,11 +593,15 @@ std::vector<std::string> plan_jit_sources(const std::vector<PendingGate>& q, int
     const TileGeom g = tile_geometry_specialised(prec);
     const int K = prec == PREC_C64 && fusion_k > 0 ? std::min(6, std::max(3, fusion_k)) : 0;
     const std::vector<PlanStep> steps = plan_gates(q, n, g, K, search);
+    std::vector<SweepProgram> progs(steps.size());
+    for (size_t s = 0; s < steps.size(); ++s)
+        if (steps[s].sweep) progs[s] = build_candidate(q, steps[s], g, K, search, factors);
+    reduce_programs(progs, prec);
     std::vector<std::string> out;
     size_t nblk_floats = 0;
-    for (const PlanStep& step : steps) {
-        if (!step.sweep) continue;
-        SweepProgram p = build_candidate(q, step, g, K, search, factors);
+    for (size_t s = 0; s < steps.size(); ++s) {
+        if (!steps[s].sweep) continue;
+        SweepProgram& p = progs[s];
         for (SwPhase& ph : p.phases)
             if (ph.kind == 1) ph.op_begin += uint32_t(nblk_floats);
         nblk_floats += p.blocks.size();
@@ -757,13 +779,14 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
     const double tiles = double(col_end - col_begin) * double(uint64_t(1) << std::max(0, n - g.M));
     // complex64 interpreter with at most two tiles per CU: a sweep lasts as
     // long as one tile, so 8 amplitudes per thread and twice the waves win
-    // over fewer phases.  12 layers, kernel time R=3 / R=4: 17 qubits 124 /
-    // 142 us, 20 qubits 152 / 169, 21 qubits 212 / 219, 22 qubits 362 / 304.
+    // over fewer phases.  12 layers, kernel time R=3 / R=4: 16 qubits 108 /
+    // 128 us, 20 qubits 141 / 168, 22 qubits 332 / 295, 24 qubits 1082 / 979.
     if (st.precision() == PREC_C64 && !st.geometry_set() && !st.jit_enabled() && fusion_k == 0 && tiles <= 512.0)
         g.R = 3;
     std::vector<PlanStep> steps;
     std::vector<SweepProgram> progs;
     choose_plan(st, queue, g, fusion_k, S, tiles, steps, progs);
+    reduce_programs(progs, st.precision());
 
     // all sweep programs of this flush in one upload: [phases][ops] per sweep, then the block table
     std::vector<size_t> poff(steps.size()), ooff(steps.size()), boff_s(steps.size());

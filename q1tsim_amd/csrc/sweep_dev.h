@@ -162,6 +162,30 @@ __device__ __forceinline__ void dense_pairs(V (&v)[NR], uint32_t cr, bool tok, V
             const auto a = m0.x, b = m1.y;
             nx = mkc<V>(fmad(-b, y.y, a * x.x), fmad(b, y.x, a * x.y));
             ny = mkc<V>(fmad(a, y.x, -(b * x.y)), fmad(a, y.y, b * x.x));
+        } else if constexpr (FORM == SWF_ROT_D) {   // x - t y, y + t x
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(-t, y.x, x.x), fmad(-t, y.y, x.y));
+            ny = mkc<V>(fmad(t, x.x, y.x), fmad(t, x.y, y.y));
+        } else if constexpr (FORM == SWF_ROT_O) {   // t x - y, x + t y
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(t, x.x, -y.x), fmad(t, x.y, -y.y));
+            ny = mkc<V>(fmad(t, y.x, x.x), fmad(t, y.y, x.y));
+        } else if constexpr (FORM == SWF_REFL_D) {   // x + t y, t x - y
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(t, y.x, x.x), fmad(t, y.y, x.y));
+            ny = mkc<V>(fmad(t, x.x, -y.x), fmad(t, x.y, -y.y));
+        } else if constexpr (FORM == SWF_REFL_O) {   // t x + y, x - t y
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(t, x.x, y.x), fmad(t, x.y, y.y));
+            ny = mkc<V>(fmad(-t, y.x, x.x), fmad(-t, y.y, x.y));
+        } else if constexpr (FORM == SWF_RX_D) {   // x + i t y, y + i t x
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(-t, y.y, x.x), fmad(t, y.x, x.y));
+            ny = mkc<V>(fmad(-t, x.y, y.x), fmad(t, x.x, y.y));
+        } else if constexpr (FORM == SWF_RX_O) {   // y - i t x, x - i t y
+            const auto t = m0.x;
+            nx = mkc<V>(fmad(t, x.y, y.x), fmad(-t, x.x, y.y));
+            ny = mkc<V>(fmad(t, y.y, x.x), fmad(-t, y.x, x.y));
         } else {  // SWF_Y
             nx = mkc<V>(y.y, -y.x);
             ny = mkc<V>(-x.y, x.x);
@@ -280,14 +304,28 @@ __device__ __forceinline__ void phase_op(uint32_t form, V (&v)[NR], uint32_t cr,
 }
 
 // One op on a thread's registers.  SEQ: the whole-state programs' rounding.
-template <typename V, int NR, int R, bool SEQ, typename Op>
-__device__ __forceinline__ void interp_op(const Op& op, V (&v)[NR], uint32_t tid, uint64_t base)
+// RED: programs of reduce_program, `lane` the thread's product of factors.
+template <typename V, int NR, int R, bool SEQ, bool RED, typename Op>
+__device__ __forceinline__ void interp_op(const Op& op, V (&v)[NR], uint32_t tid, uint64_t base, V& lane)
 {
     const uint32_t body = op.code & 0xffu, cr = op.ctl & 0xffffu, ct = op.ctl >> 16;
     const int reg = int((op.code >> 8) & 0xffu);
     const bool tok = (tid & ct) == ct;
     const V m0 = mkc<V>(op.m[0], op.m[1]), m1 = mkc<V>(op.m[2], op.m[3]);
     if (body < kInterpPhase) {
+        if constexpr (RED) {
+            if (body >= SWF_ROT_D) {
+                switch (body) {
+                case SWF_ROT_D: interp_reg<V, NR, R, SWF_ROT_D, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                case SWF_ROT_O: interp_reg<V, NR, R, SWF_ROT_O, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                case SWF_REFL_D: interp_reg<V, NR, R, SWF_REFL_D, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                case SWF_REFL_O: interp_reg<V, NR, R, SWF_REFL_O, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                case SWF_RX_D: interp_reg<V, NR, R, SWF_RX_D, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                default: interp_reg<V, NR, R, SWF_RX_O, false>(reg, v, 0u, m0, m0, m0, m0); break;
+                }
+                return;
+            }
+        }
         const V m2 = mkc<V>(op.m[4], op.m[5]), m3 = mkc<V>(op.m[6], op.m[7]);
         if (body == (SEQ ? SWF_REAL_SEQ : SWF_REAL))
             interp_ctl<V, NR, R, SEQ ? SWF_REAL_SEQ : SWF_REAL>(reg, v, cr, ct, tok, m0, m1, m2, m3);
@@ -303,15 +341,27 @@ __device__ __forceinline__ void interp_op(const Op& op, V (&v)[NR], uint32_t tid
             scale_regs<V, NR>(v, cr, 0u, true, [&](int k, V x) { return cmul(sel(((k >> reg) & 1) != 0, m1, m0), x); });
         }
     } else {
+        if constexpr (RED) {
+            if (body == kInterpApply) {
+                scale_regs_t<V, NR, false, false>(v, 0u, true, [&](int, V x) { return cmul(lane, x); });
+                return;
+            }
+        }
         // one factor per lane: a phase (m0 where the controls are set), or a
         // diagonal entry picked by a thread bit or a bit outside the tile
         V f = m0;
         if (body != kInterpPhase) {
-            const uint32_t bit = op.code >> 16;
+            const uint32_t bit = (op.code >> 16) & 0xffu;
             const bool one = body == kInterpDiagTid ? ((tid >> bit) & 1u) != 0 : ((base >> bit) & 1u) != 0;
             f = sel(one, m1, m0);
         }
         if (ct) f = sel(tok, f, mkc<V>(1, 0));
+        if constexpr (RED) {
+            if (op.code & kInterpLane) {
+                lane = cmul(f, lane);
+                return;
+            }
+        }
         scale_regs<V, NR>(v, cr, 0u, true, [&](int, V x) { return cmul(f, x); });
     }
 }
@@ -540,8 +590,9 @@ __device__ __forceinline__ V tile_factor(const SwOp* ops, uint32_t begin, uint32
 // The program's phases on a tile already in LDS, then LDS -> HBM.  BLK is
 // the widest fused dense block the kernel holds: 0 none (programs without
 // blocks: the MFMA code's registers would halve the kernel's occupancy),
-// 1 the 3- and 4-qubit blocks, 2 also the 5- and 6-qubit ones.
-template <typename V, int M, int R, int SW, int BLK>
+// 1 the 3- and 4-qubit blocks, 2 also the 5- and 6-qubit ones.  RED: the
+// program went through reduce_program.
+template <typename V, int M, int R, int SW, int BLK, bool RED>
 __device__ __forceinline__ void tile_phases(V* __restrict__ a, const SweepArgs& sa, uint64_t base, V* lds,
                                             const TileAddr<M, R>& ta)
 {
@@ -595,11 +646,12 @@ __device__ __forceinline__ void tile_phases(V* __restrict__ a, const SweepArgs& 
 #pragma unroll
             for (int k = 0; k < NR; ++k) v[k] = lds[st ^ srp[k]];
             const InterpOpT<Rl>* ops = reinterpret_cast<const InterpOpT<Rl>*>(sa.ops);
+            V lane = mkc<V>(1, 0);
             for (uint32_t oi = ph.op_begin; oi < ph.op_end; ++oi) {
                 const InterpOpT<Rl> op = load_uniform(ops, oi);
                 pin_op<Rl>(op);
                 if ((base & op.co) != op.co) continue;
-                interp_op<V, NR, R, false>(op, v, uint32_t(tid), base);
+                interp_op<V, NR, R, false, RED>(op, v, uint32_t(tid), base, lane);
             }
             if (ph.wmap == 0) {
 #pragma unroll
@@ -657,7 +709,7 @@ template <typename V> __device__ __forceinline__ V load_set(const V* a, uint64_t
 }
 
 // One tile of a sweep: HBM -> LDS, the program's phases, LDS -> HBM.
-template <typename V, int M, int R, int SW, int BLK, bool UNSET>
+template <typename V, int M, int R, int SW, int BLK, bool RED, bool UNSET>
 __device__ __forceinline__ void sweep_tile(V* __restrict__ a, const SweepArgs& sa, uint64_t tile, V* lds)
 {
     constexpr int NT = 1 << (M - R), NR = 1 << R;
@@ -675,7 +727,7 @@ __device__ __forceinline__ void sweep_tile(V* __restrict__ a, const SweepArgs& s
         for (int k = 0; k < NR; ++k) lds[s0 ^ swz<SW, M>(k * NT)] = load_stream(a + (base | ta.g_tid | ta.g_k[k]));
     }
     __syncthreads();
-    tile_phases<V, M, R, SW, BLK>(a, sa, base, lds, ta);
+    tile_phases<V, M, R, SW, BLK, RED>(a, sa, base, lds, ta);
 }
 
 }  // namespace q1t

@@ -18,14 +18,20 @@ namespace q1t {
 
 // One in-tile operation of a sweep program (read by every thread of a
 // workgroup; uniform).
-enum SwOpType : int32_t { SW_DENSE1 = 0, SW_PHASE = 1, SW_DIAG1 = 2, SW_BLOCK = 3 };
+enum SwOpType : int32_t { SW_DENSE1 = 0, SW_PHASE = 1, SW_DIAG1 = 2, SW_BLOCK = 3, SW_APPLY = 4 };
 
 // Body of a SW_DENSE1 op, read off its 2x2 matrix (SwOp::aux).
 // The _SEQ forms round as the general body does (its second product fused):
 // whole-state programs use them, which give the bits of the gates applied one
 // by one with the general body.
+// The last six are reduced forms (reduce_program): the matrix without a factor
+// that the flush applies once, rotations [[a, -b], [b, a]], reflections
+// [[a, b], [b, -a]] and RX [[a, ib], [ib, a]] divided by their diagonal entry
+// (_D, one coefficient m[0] = b / a) or their off-diagonal one (_O, m[0] = a / b):
+// four fused multiply-adds per pair instead of eight operations.
 enum SwDenseForm : uint32_t {
-    SWF_GENERAL = 0, SWF_REAL = 1, SWF_SWAP = 2, SWF_RX = 3, SWF_Y = 4, SWF_REAL_SEQ = 5, SWF_RX_SEQ = 6
+    SWF_GENERAL = 0, SWF_REAL = 1, SWF_SWAP = 2, SWF_RX = 3, SWF_Y = 4, SWF_REAL_SEQ = 5, SWF_RX_SEQ = 6,
+    SWF_ROT_D = 7, SWF_ROT_O = 8, SWF_REFL_D = 9, SWF_REFL_O = 10, SWF_RX_D = 11, SWF_RX_O = 12
 };
 // Body of a SW_PHASE op (SwOp::aux): general, times i, times -i, times -1.
 enum SwPhaseForm : uint32_t { SWP_GENERAL = 0, SWP_I = 1, SWP_MINUS_I = 2, SWP_NEG = 3 };
@@ -36,8 +42,10 @@ enum SwPhaseForm : uint32_t { SWP_GENERAL = 0, SWP_I = 1, SWP_MINUS_I = 2, SWP_N
 // bits outside the tile (uniform per tile).
 struct SwOp {
     int32_t type;
-    int32_t reg;       // SW_DENSE1: index of the target among the phase's register bits
-    int32_t dreg;      // SW_DIAG1: register index of the target, or -1
+    int32_t reg;       // SW_DENSE1: index of the target among the phase's register bits; SW_PHASE and
+                       // SW_DIAG1 without register bits: 1 if the factor goes to the thread's product,
+                       // which a SW_APPLY at the phase's end multiplies into its registers
+    int32_t dreg;      // SW_DIAG1: register index of the target, or -1; reduced dense forms: 1 for the _O one
     int32_t dtid;      // SW_DIAG1: thread-index bit of the target, or -1
     int32_t dglobal;   // SW_DIAG1: global bit of the target when it is outside the tile, or -1
     uint32_t cr;       // control (or phase) mask over register indices
@@ -94,9 +102,10 @@ constexpr int sweep_swizzle_bits(int M) { return M == 13 ? 5 : 4; }
 // the body of their matrix, phases of any value the general product (0, 1 and
 // +-i are exact factors).  `code`: bits 0-7 body (SwDenseForm or kInterp*),
 // 8-15 register bit of the target, 16-23 thread bit or outer bit of a
-// diagonal's target; `ctl`: controls over register indices (low half) and
+// diagonal's target, 24 a factor that goes to the thread's product; `ctl`: controls over register indices (low half) and
 // thread bits (high half); `co`: controls over bits outside the tile.
-constexpr uint32_t kInterpPhase = 16, kInterpDiagReg = 17, kInterpDiagTid = 18, kInterpDiagOuter = 19;
+constexpr uint32_t kInterpPhase = 16, kInterpDiagReg = 17, kInterpDiagTid = 18, kInterpDiagOuter = 19,
+                   kInterpApply = 20, kInterpLane = 1u << 24;
 template <typename R> struct InterpOpT {
     uint32_t code;
     uint32_t ctl;
