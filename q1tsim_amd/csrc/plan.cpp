@@ -313,13 +313,6 @@ SwPhase make_phase(uint32_t kind, uint32_t regs, int M, uint32_t op_begin)
         if ((regs >> b) & 1) ph.rpos[nr++] = uint8_t(b);
         else ph.tbit[nt++] = uint8_t(b);
     }
-    if (kind == 0 && nr <= 4)
-        for (int k = 0; k < (1 << nr); ++k) {
-            int l = 0;
-            for (int b = 0; b < nr; ++b)
-                if ((k >> b) & 1) l |= 1 << ph.rpos[b];
-            ph.rslot[k] = uint32_t(swizzle_slot(sweep_swizzle_bits(M), M, l));
-        }
     return ph;
 }
 
@@ -802,6 +795,28 @@ static void reduce_op(SwOp& o, Reduction& red)
     else red.factor *= std::complex<long double>(a, 0);
     red.gates += 1;
     set_coefs(o, off ? a / b : b / a);
+}
+
+void place_phases(std::vector<SwPhase>& phases, int M, int R, size_t elem_bytes)
+{
+    const int nt = M - R;
+    auto at = [&](uint32_t l) {
+        return uint32_t(swizzle_slot(sweep_swizzle_bits(M), M, int(l))) * uint32_t(elem_bytes);
+    };
+    for (SwPhase& ph : phases) {
+        if (ph.kind != 0) continue;
+        for (int b = 0; b < nt; ++b) ph.col[b] = at(1u << ph.tbit[b]) | at(ph.wcol[b]) << 16;
+        for (int k = 0; k < (1 << R); ++k) {
+            uint32_t l = 0, l2 = ph.wxor;
+            for (int b = 0; b < R; ++b)
+                if ((k >> b) & 1) {
+                    l |= 1u << ph.rpos[b];
+                    l2 ^= ph.wcol[nt + b];
+                }
+            ph.slot_in[k] = at(l);
+            ph.slot_out[k] = at(l2);
+        }
+    }
 }
 
 void reduce_program(std::vector<SwPhase>& phases, std::vector<SwOp>& ops, Precision prec, Reduction& red, bool last)

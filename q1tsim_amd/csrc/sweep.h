@@ -72,6 +72,9 @@ struct Reduction {
 // Batches keep the gates' own forms.
 void reduce_program(std::vector<SwPhase>& phases, std::vector<SwOp>& ops, Precision prec, Reduction& red, bool last);
 
+// The LDS places of the register phases for amplitudes of elem_bytes.
+void place_phases(std::vector<SwPhase>& phases, int M, int R, size_t elem_bytes);
+
 // An op as the interpreting kernels take it; `seq`: whole-state programs.
 template <typename R> InterpOpT<R> interp_op(const SwOp& o, bool seq);
 

@@ -47,8 +47,8 @@ template <typename V> __device__ __forceinline__ void warm_sweep(const SweepArgs
 
 // UNSET: launches with SweepArgs::unset bits, in a kernel of their own (the
 // load that takes them costs the sweeps without).
-// complex64 with 16 amplitudes per thread is held to 4 waves per SIMD, at the
-// price of 44 bytes of scratch: 24 qubits 979 us, at 3 waves 1092 us.
+// complex64 with 16 amplitudes per thread is held to 4 waves per SIMD (24 qubits
+// 979 us when it took 44 bytes of scratch to get there, at 3 waves 1092 us).
 template <typename V, int M, int R, int SW, int BLK, bool UNSET>
 __global__ void __launch_bounds__(1 << (M - R))
 __attribute__((amdgpu_waves_per_eu(sizeof(V) == 8 && M == 12 ? (R == 3 || BLK == 0 ? 4 : 3) : 2)))
@@ -779,14 +779,15 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
     const double tiles = double(col_end - col_begin) * double(uint64_t(1) << std::max(0, n - g.M));
     // complex64 interpreter with at most two tiles per CU: a sweep lasts as
     // long as one tile, so 8 amplitudes per thread and twice the waves win
-    // over fewer phases.  12 layers, kernel time R=3 / R=4: 16 qubits 108 /
-    // 128 us, 20 qubits 141 / 168, 22 qubits 332 / 295, 24 qubits 1082 / 979.
+    // over fewer phases.  12 layers, kernel time R=3 / R=4: 16 qubits 106 /
+    // 119 us, 20 qubits 140 / 157, 21 qubits 188 / 199, 22 qubits 328 / 261.
     if (st.precision() == PREC_C64 && !st.geometry_set() && !st.jit_enabled() && fusion_k == 0 && tiles <= 512.0)
         g.R = 3;
     std::vector<PlanStep> steps;
     std::vector<SweepProgram> progs;
     choose_plan(st, queue, g, fusion_k, S, tiles, steps, progs);
     reduce_programs(progs, st.precision());
+    for (SweepProgram& p : progs) place_phases(p.phases, g.M, g.R, st.elem_bytes());
 
     // all sweep programs of this flush in one upload: [phases][ops] per sweep, then the block table
     std::vector<size_t> poff(steps.size()), ooff(steps.size()), boff_s(steps.size());
@@ -1047,6 +1048,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             if (!p.steps[s].sweep) continue;
             if (K) build_fused_program(q, p.steps[s], g.M, g.R, K, p.ph[s], p.ops[s], p.blocks, &nblocks, search);
             else build_program(q, p.steps[s], g.M, g.R, p.ph[s], p.ops[s], search);
+            place_phases(p.ph[s], g.M, g.R, st.elem_bytes());
             p.st.sweeps += 1;
             p.st.launches += 1;
             p.st.gates += p.steps[s].gates.size();

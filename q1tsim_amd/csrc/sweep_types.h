@@ -76,11 +76,12 @@ struct SwPhase {
     uint32_t wmap;       // 0: identity (plain write-back)
     uint32_t wxor;
     uint16_t wcol[16];
-    // register phases: LDS slot term of register slot k, swz of the local
-    // index made of k's bits at the register positions (the slot of a
-    // thread's element k is swz(thread part) ^ rslot[k]); set by the planner
-    // for the kernel's swizzle (sweep_swizzle_bits)
-    uint32_t rslot[16];
+    // register phases, for the interpreting kernels (place_phases): byte offsets
+    // in LDS, swizzled.  A thread reads its element k at tin ^ slot_in[k] and
+    // writes it back at tout ^ slot_out[k]; tin and tout are the low and high
+    // halves of the XOR of col over the thread's set bits, wxor is in slot_out.
+    uint32_t col[12];
+    uint32_t slot_in[16], slot_out[16];
 };
 
 // LDS swizzle of local element l in a 2^M tile: XOR-fold of the bits above
