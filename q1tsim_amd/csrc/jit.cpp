@@ -248,6 +248,10 @@ std::string jit_sweep_source(const std::vector<SwPhase>& phases, const std::vect
                 if (op.co) o << "    }\n";
                 o << "    }\n";
             }
+        } else if (ph.kind == 4) {
+            o << "    pair_phase<V, M, R, SW>(lds, ops, " << ph.op_begin << "u, " << int(ph.rpos[0]) << ", "
+              << int(ph.rpos[1]) << ", tid, [](const SwOp& op, int k) { return opm<V>(op, k); });\n";
+            o << "    __syncthreads();\n";
         } else {
             emit_register_phase(o, ph, ops, M, R, SW);
         }

@@ -115,12 +115,19 @@ bool sweepable(const GateOp& op, std::vector<int>* local_targets)
     }
 }
 
+// A dense gate on two qubits without controls: a phase of its own in a sweep of
+// unfused programs.
+static bool pair_gate(const GateOp& op)
+{
+    return op.kind == OpKind::Dense && op.targets.size() == 2 && op.ctrl_mask == 0;
+}
+
 // Which bits a gate needs inside the tile, or false if it cannot join a sweep.
 // Plain: non-diagonal targets (controls and diagonal factors outside the tile
 // are per-tile predicates / constants).  Fused (fuse_k > 0): every bit of a
 // non-diagonal gate, so it can be absorbed into a block; diagonal one-target
 // gates and phases may still reach outside.
-static bool tile_need(const GateOp& op, int fuse_k, uint64_t* need)
+static bool tile_need(const GateOp& op, int fuse_k, bool pairs, uint64_t* need)
 {
     *need = 0;
     if (fuse_k > 0) {
@@ -130,7 +137,7 @@ static bool tile_need(const GateOp& op, int fuse_k, uint64_t* need)
         *need = bits;
         return true;
     }
-    if (!sweepable(op, nullptr)) return false;
+    if (!sweepable(op, nullptr) && !(pairs && pair_gate(op))) return false;
     if (op.kind == OpKind::Dense || op.kind == OpKind::Swap2)
         for (int t : op.targets) *need |= uint64_t(1) << t;
     return true;
@@ -178,7 +185,7 @@ std::vector<uint64_t> plan_key(const std::vector<PendingGate>& q, int n, const T
     k.push_back(search ? 1 : 0);
     for (const PendingGate& pg : q) {
         uint64_t need = 0;
-        const bool ok = tile_need(pg.op, fuse_k, &need);
+        const bool ok = tile_need(pg.op, fuse_k, false, &need);
         k.push_back(touched_bits(pg.op));
         k.push_back(nondiag_bits(pg.op));
         k.push_back(need);
@@ -187,7 +194,8 @@ std::vector<uint64_t> plan_key(const std::vector<PendingGate>& q, int n, const T
     return k;
 }
 
-std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const TileGeom& g, int fuse_k, bool search)
+std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const TileGeom& g, int fuse_k, bool search,
+                                 bool pairs)
 {
     std::vector<PlanStep> steps;
     std::vector<size_t> rem;
@@ -196,7 +204,7 @@ std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const
     for (size_t i = 0; i < q.size(); ++i) {
         gb[i].touched = touched_bits(q[i].op);
         gb[i].nd = nondiag_bits(q[i].op);
-        gb[i].ok = tile_need(q[i].op, fuse_k, &gb[i].need);
+        gb[i].ok = tile_need(q[i].op, fuse_k, pairs, &gb[i].need);
         if (q[i].op.kind != OpKind::Identity) rem.push_back(i);
     }
     const bool tiles_ok = n >= g.M + 2;
@@ -232,8 +240,10 @@ std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const
         if (sel.empty()) {
             // the first remaining gate cannot run inside a tile
             steps.push_back(PlanStep{false, {}, {rem.front()}});
-        } else if (sel.size() == 1 && (is_diagonal(q[sel[0]].op) || q[sel[0]].op.kind == OpKind::Swap2)) {
-            // a lone diagonal or swap gate touches only part of the state: its own kernel is cheaper
+        } else if (sel.size() == 1 && (is_diagonal(q[sel[0]].op) || q[sel[0]].op.kind == OpKind::Swap2 ||
+                                       pair_gate(q[sel[0]].op))) {
+            // a lone diagonal or swap gate touches only part of the state: its
+            // own kernel is cheaper; a lone dense pair gains nothing in a sweep
             steps.push_back(PlanStep{false, {}, sel});
         } else {
             // fill the tile up to M bits with the lowest unused bits
@@ -674,6 +684,45 @@ std::vector<size_t> one_reg_phase(const std::vector<PendingGate>& q, const Phase
     return rest;
 }
 
+// The dense two-qubit gates of `pending` that no earlier gate holds back, a
+// phase each; returns the other gates.  Register phases come after them, so
+// that the gates they free share as few phases as possible.
+std::vector<size_t> pair_phases(const std::vector<PendingGate>& q, const PhaseGates& pg,
+                                const std::vector<size_t>& pending, const LocalMap& lm, int M,
+                                std::vector<SwPhase>& phases, std::vector<SwOp>& ops, std::vector<size_t>* order)
+{
+    std::vector<size_t> rest;
+    Blocker blk;
+    for (size_t i : pending) {
+        const PhaseGate& g = pg[i];
+        const GateOp& op = q[i].op;
+        if (!pair_gate(op) || blk.blocks(g.touched, g.nd)) {
+            blk.add(g.touched, g.nd);
+            rest.push_back(i);
+            continue;
+        }
+        SwPhase ph = make_phase(4, 0, M, uint32_t(ops.size()));
+        ph.rpos[0] = uint8_t(lm.local_of[op.targets[0]]);
+        ph.rpos[1] = uint8_t(lm.local_of[op.targets[1]]);
+        for (int r = 0; r < 4; ++r) {
+            SwOp o;
+            std::memset(&o, 0, sizeof(o));
+            o.type = SW_PAIR;
+            o.dreg = o.dtid = o.dglobal = -1;
+            for (int c = 0; c < 4; ++c) {
+                o.m[2 * c] = op.m[size_t(4 * r + c)].real();
+                o.m[2 * c + 1] = op.m[size_t(4 * r + c)].imag();
+            }
+            for (int k = 0; k < 8; ++k) o.mf[k] = float(o.m[k]);
+            ops.push_back(o);
+        }
+        ph.op_end = uint32_t(ops.size());
+        phases.push_back(ph);
+        if (order) order->push_back(i);
+    }
+    return rest;
+}
+
 // Apply a gate to every column of the block matrix U (dimension 2^|B|);
 // pos[b] = block-index bit of global bit b.
 void compose(std::vector<cdouble>& U, int nb, const GateOp& op, const int* pos)
@@ -751,7 +800,10 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
     TileFactors tf;
     TileFactors* tfp = factors ? &tf : nullptr;
     const PhaseGates pg(q, pending, lm, false);
-    while (!pending.empty()) pending = one_reg_phase(q, pg, pending, lm, M, R, phases, ops, search, order, tfp);
+    while (!pending.empty()) {
+        pending = pair_phases(q, pg, pending, lm, M, phases, ops, order);
+        if (!pending.empty()) pending = one_reg_phase(q, pg, pending, lm, M, R, phases, ops, search, order, tfp);
+    }
     append_factors(tf, M, phases, ops, order);
 }
 
@@ -1119,6 +1171,9 @@ void sweep_features(const std::vector<SwPhase>& phases, const std::vector<SwOp>&
             if (nb == 3) f[1] += 1.0f;
             else f[2] += float(1 << (2 * (nb - 4)));
             f[16] = std::max(f[16], float(nb));
+        } else if (ph.kind == 4) {   // as a block of 3 qubits
+            nb = 2;
+            f[1] += 1.0f;
         } else if (ph.kind == 0) {
             nb = g.R;
             f[0] += 1.0f;

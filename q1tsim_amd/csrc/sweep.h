@@ -33,8 +33,10 @@ bool sweepable(const GateOp& op, std::vector<int>* local_targets);
 // tile.  `search`: refine each greedy tile (and, in the programs below, each
 // phase's register bits) by local search (GpuVectorState::tile_search,
 // phase_search).
+// `pairs`: dense two-qubit gates without controls join the sweeps (unfused
+// programs; batches and fused plans apply them on their own).
 std::vector<PlanStep> plan_gates(const std::vector<PendingGate>& q, int n, const TileGeom& g, int fuse_k,
-                                 bool search = true);
+                                 bool search = true, bool pairs = false);
 
 // Everything plan_gates reads of the queue and its settings: equal keys give
 // equal plans (a flush repeating the previous flush's gate structure, with

@@ -57,7 +57,7 @@ k_sweep(V* __restrict__ amp, uint64_t col_stride, SweepArgs sa)
     __shared__ V lds[1 << M];
     V* a = amp + uint64_t(blockIdx.y) * col_stride;
     warm_sweep<V>(sa);
-    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK, BLK == 0, UNSET>(a, sa, tile, lds);
+    for (uint64_t tile = blockIdx.x; tile < sa.ntiles; tile += gridDim.x) sweep_tile<V, M, R, SW, BLK, BLK == 0 || BLK == 3, UNSET>(a, sa, tile, lds);
 }
 
 // Sweeps of many states in one launch: item i covers flattened tiles
@@ -161,6 +161,7 @@ static int launch_sweep(GpuVectorState& st, const PlanStep& step, const SwPhase*
         }
         V* amp = static_cast<V*>(st.col_ptr(c0));
         auto k = unset ? k_sweep<V, M, R, SW, 0, true> : k_sweep<V, M, R, SW, 0, false>;
+        if (blk == 3) k = unset ? k_sweep<V, M, R, SW, 3, true> : k_sweep<V, M, R, SW, 3, false>;
         if constexpr (sizeof(V) == 8) {
             if (blk == 2) k = unset ? k_sweep<V, M, R, SW, 2, true> : k_sweep<V, M, R, SW, 2, false>;
             else if (blk == 1) k = unset ? k_sweep<V, M, R, SW, 1, true> : k_sweep<V, M, R, SW, 1, false>;
@@ -190,12 +191,16 @@ static void put_ops(char* to, const std::vector<SwOp>& ops, Precision prec, bool
 }
 
 // The widest fused dense block of a program, as the kernels' BLK: 0 none,
-// 1 blocks of 3 and 4 qubits, 2 wider ones.
+// 1 blocks of 3 and 4 qubits, 2 wider ones; 3 dense pairs, which no program with
+// blocks has (kernels of their own too: the pairs' registers would spill in the
+// complex64 kernel of the others).
 static int block_level(const std::vector<SwPhase>& phases)
 {
     int lv = 0;
-    for (const SwPhase& ph : phases)
+    for (const SwPhase& ph : phases) {
         if (ph.kind == 1) lv = std::max(lv, ph.reg_mask > 4 ? 2 : 1);
+        if (ph.kind == 4) lv = 3;
+    }
     return lv;
 }
 
@@ -348,14 +353,18 @@ static SweepProgram build_candidate(const std::vector<PendingGate>& q, const Pla
 // has a register phase.
 static void reduce_programs(std::vector<SweepProgram>& progs, Precision prec)
 {
+    auto reducible = [](const SweepProgram& p) {
+        const int lv = block_level(p.phases);
+        return lv == 0 || lv == 3;
+    };
     size_t last = progs.size();
     for (size_t s = 0; s < progs.size(); ++s)
-        if (block_level(progs[s].phases) == 0)
+        if (reducible(progs[s]))
             for (const SwPhase& ph : progs[s].phases)
                 if (ph.kind == 0) last = s;
     Reduction red;
     for (size_t s = 0; s < progs.size(); ++s)
-        if (block_level(progs[s].phases) == 0) reduce_program(progs[s].phases, progs[s].ops, prec, red, s == last);
+        if (reducible(progs[s])) reduce_program(progs[s].phases, progs[s].ops, prec, red, s == last);
 }
 
 // Wall-time estimate of a gate applied on its own: one read and one write
@@ -415,11 +424,11 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
             key.insert(key.begin(), 1);   // the per-gate planner
             std::vector<int> kind;
             if (!cache_hit(kind)) {
-                steps = plan_gates(queue, n, g, 0, search);
+                steps = plan_gates(queue, n, g, 0, search, true);
                 cache_store(std::vector<int>(steps.size(), 0));
             }
         } else {
-            steps = plan_gates(queue, n, g, 0, search);
+            steps = plan_gates(queue, n, g, 0, search, true);
         }
         progs = build_all(steps, 0);
         return;
@@ -592,7 +601,7 @@ std::vector<std::string> plan_jit_sources(const std::vector<PendingGate>& q, int
 {
     const TileGeom g = tile_geometry_specialised(prec);
     const int K = prec == PREC_C64 && fusion_k > 0 ? std::min(6, std::max(3, fusion_k)) : 0;
-    const std::vector<PlanStep> steps = plan_gates(q, n, g, K, search);
+    const std::vector<PlanStep> steps = plan_gates(q, n, g, K, search, K == 0);
     std::vector<SweepProgram> progs(steps.size());
     for (size_t s = 0; s < steps.size(); ++s)
         if (steps[s].sweep) progs[s] = build_candidate(q, steps[s], g, K, search, factors);
@@ -876,8 +885,8 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
             const int shape = g.M * 16 + g.R;
             if (st.precision() == PREC_C128) {
                 switch (shape) {
-                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, unset[s], col_bytes[s], jf); break;
-                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, 0, unset[s], col_bytes[s], jf); break;
+                case 12 * 16 + 3: slot = launch_sweep<double2, 12, 3, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, unset[s], col_bytes[s], jf); break;
+                case 12 * 16 + 4: slot = launch_sweep<double2, 12, 4, 4>(st, step, dp, np, dop, int(progs[s].ops.size()), dblocks, col_begin, col_end, blk, unset[s], col_bytes[s], jf); break;
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex128 tile shape");
                 }
             } else {

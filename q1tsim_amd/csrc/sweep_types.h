@@ -18,7 +18,7 @@ namespace q1t {
 
 // One in-tile operation of a sweep program (read by every thread of a
 // workgroup; uniform).
-enum SwOpType : int32_t { SW_DENSE1 = 0, SW_PHASE = 1, SW_DIAG1 = 2, SW_BLOCK = 3, SW_APPLY = 4 };
+enum SwOpType : int32_t { SW_DENSE1 = 0, SW_PHASE = 1, SW_DIAG1 = 2, SW_BLOCK = 3, SW_APPLY = 4, SW_PAIR = 5 };
 
 // Body of a SW_DENSE1 op, read off its 2x2 matrix (SwOp::aux).
 // The _SEQ forms round as the general body does (its second product fused):
@@ -65,6 +65,9 @@ struct SwPhase {
                          // tile is scaled by the product of their factors
                          // as it is stored (the program's last phase;
                          // programs of the specialised kernels only)
+                         // 4: a dense gate on two local bits rpos[0] (the
+                         // matrix's high bit) and rpos[1]; ops op_begin ..
+                         // op_begin + 3 hold its rows in m
     uint8_t rpos[8];     // local positions of the register bits (ascending)
     uint8_t tbit[16];    // local positions of the thread bits (ascending)
     // register phases: an affine map over GF(2) of the local index, applied
