@@ -458,7 +458,8 @@ __device__ __forceinline__ void load_leaves(const T* in, uint64_t size, uint64_t
 // it and less) and by launches for small columns, so one launch makes three
 // levels: 256 threads fold 16 entries each, 16 threads the 256 folds, one
 // thread the 16 folds of those.  Sizes are powers of two above 16: every group
-// that exists is full.
+// that exists is full.  A column of 30 qubits complex128 takes 3.1 ms (5.5 TB/s),
+// 3.7 ms with a level per launch and plain loads.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_tree_items(TreeItem one, const TreeItem* __restrict__ items, uint32_t n,
                                                        uint64_t nchunks)

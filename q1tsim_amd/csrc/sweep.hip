@@ -217,8 +217,8 @@ static int whole_bits(int n) { return std::max(n, whole_regs(n)); }
 // threads leave at once (barriers count the waves that are left).
 // Before, one launch per gate (single states: 3.2 us per gate at 12 qubits) or
 // one barrier and a full LDS pass per gate (batches: 9 us per gate at 13
-// qubits).  Measured: 12 qubits complex128, 350 gates 1110 -> 138 us; 112
-// columns of 10 to 13 qubits complex64 in a batch 2850 -> 340 us per round.
+// qubits).  Measured: 12 qubits complex128, 350 gates 1110 -> 115 us; 112
+// columns of 10 to 13 qubits complex64 in a batch 2850 -> 150 us per round.
 template <typename V, int R>
 __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ items,
                                                 const WholePhase* __restrict__ phases,
