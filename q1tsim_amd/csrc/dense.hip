@@ -319,7 +319,9 @@ __global__ void __launch_bounds__(kBlock) k_dense_back(V* __restrict__ amp, cons
 // qubits 48 and 78; complex128, K = 9, 128 KiB: 20 qubits, 128 blocks 159 and
 // 151, 21 qubits 171 and 285).  Up to K = 5 always: its products take
 // microseconds however few the blocks are (18 qubits, K = 4: 9 and 14).  Else
-// k_dense_rows, with as many rows per workgroup as leave two workgroups per CU.
+// k_dense_rows, with as many rows per workgroup as leave two workgroups per CU
+// and at most the matrix's row tiles per wave (1 and 2 at K = 4 and 5: those
+// widths come here with the columns of states too small for k_dense_tile).
 DensePlan plan_dense(const GateOp& op, int n, size_t ncols, size_t elem_bytes)
 {
     DensePlan p;
@@ -340,6 +342,7 @@ DensePlan plan_dense(const GateOp& op, int n, size_t ncols, size_t elem_bytes)
     p.nblocks = uint64_t(1) << (free_bits - p.log_cols);
     const uint64_t blocks = p.nblocks * ncols, tiles = (uint64_t(1) << p.K) / 16;
     p.rtw = blocks * tiles / 16 >= 512 ? 4 : blocks * tiles / 8 >= 512 ? 2 : 1;
+    p.rtw = int(std::min<uint64_t>(uint64_t(p.rtw), tiles));
     p.splits = uint32_t(std::max<uint64_t>(1, tiles / (4 * p.rtw)));
     p.log_slice = p.K;
     while ((elem_bytes << (p.log_slice + p.log_cols)) > kSliceBytes) --p.log_slice;
@@ -425,6 +428,10 @@ void launch_dense(const DensePlan& plan, const GateOp& op, int n, V* a, uint64_t
     }
     const size_t lds = sizeof(V) << (plan.log_slice + plan.log_cols);
     const uint64_t blocks = plan.nblocks * ncols;
+    // a wave takes rtw row tiles or none; all of them are taken once
+    const uint32_t row_tiles = (1u << K) / 16, rtw = uint32_t(plan.rtw);
+    if (row_tiles % rtw || 4 * rtw * plan.splits < row_tiles || 4 * rtw * (plan.splits - 1) >= row_tiles)
+        throw Error(ERR_INVALID_ARGUMENT, "dense plan: the waves do not cover the matrix rows once");
     for (uint64_t f0 = 0; f0 < blocks; f0 += plan.chunk) {
         const uint64_t f1 = std::min(blocks, f0 + plan.chunk);
         const dim3 grid(unsigned(std::min<uint64_t>(f1 - f0, 65536)), plan.splits);
