@@ -105,12 +105,12 @@ int q1t_gvs_measure_with_n0(q1t_gvs* s, size_t qbit, size_t cbit, const size_t* 
 /* No counterpart in the reference.  q1t_gvs_marginal_w0 for callers that
  * cannot allocate device memory (code under graph capture, tight serving
  * loops): the call makes no hipMalloc/hipFree.  Its partial sums live in a
- * fixed 516 KiB device array per GPU, held until the process ends; at most
+ * fixed 515 KiB device array per GPU, held until the process ends; at most
  * 256 branch columns (a larger state is rejected with
  * Q1T_ERR_INVALID_ARGUMENT), no pending gates (flush first), and the device
  * current at the call must be the state's.  Results are bit-identical to
- * q1t_gvs_marginal_w0.  Calls that overlap on one GPU share the array and
- * race: serialise them. */
+ * q1t_gvs_marginal_w0.  Calls on one GPU share the array and take turns: a
+ * call waits until one that runs on another thread has ended. */
 int q1t_gvs_marginal_w0_noalloc(q1t_gvs* s, size_t qbit, double* w0s, size_t len);
 /* QuState::measure_into (qustate.rs:35, vectorstate.rs:237-329). */
 int q1t_gvs_measure_into(q1t_gvs* s, size_t qbit, size_t cbit, uint64_t* res, size_t res_len, const q1t_rng* rng);

@@ -177,9 +177,8 @@ public:
     // folded into the marginal and collapse passes)
     std::vector<double> marginal_w0(size_t qbit, int basis = 0);
     // marginal_w0 without any device allocation: partial sums in a fixed
-    // file-scope device array (at most kNoAllocMaxCols columns), summed on
-    // the device in the host's order (bit-identical results).  Needs no
-    // pending gates.  Calls that overlap on one GPU race on that array.
+    // file-scope device array (at most kNoAllocMaxCols columns), bit-identical
+    // results.  Needs no pending gates.  Calls on one GPU take turns.
     void marginal_w0_noalloc(size_t qbit, double* w0s, size_t len);
     void measure_with_n0(size_t qbit, size_t cbit, const size_t* n0s, const std::vector<double>& w0s,
                          uint64_t* res, size_t res_len, bool collapse, int basis = 0);

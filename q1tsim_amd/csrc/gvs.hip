@@ -1161,35 +1161,42 @@ std::vector<double> GpuVectorState::marginal_w0(size_t qbit, int basis)
 
 // The scratch of marginal_w0_noalloc: kMargBlocks partial sums per column,
 // then one w0 per column, then the columns' counts of finished workgroups
-// (zero at the start, and left zero by every call).  515 KiB; each GPU the
-// library runs on holds its own copy until the process ends.
+// (zero at the start, and left zero by every call that ends).  515 KiB; each
+// GPU the library runs on holds its own copy until the process ends.
 static constexpr size_t kNoAllocMaxCols = 256;
 static constexpr size_t kNoAllocW0 = kNoAllocMaxCols * size_t(kMargBlocks);
 static constexpr size_t kNoAllocDone = kNoAllocW0 + kNoAllocMaxCols;
 static __device__ __align__(256) double scratch[kNoAllocDone + kNoAllocMaxCols / 2];
 
-// The device address of `scratch` on each device, looked up once per device
-// with that device current.  The array's name is not a device address in
-// host code; only these pointers are passed to kernels and copies.
-static constexpr int kMaxDevices = 64;
-static std::mutex g_scratch_mu;
-static double* g_scratch_ptr[kMaxDevices] = {};
-
-static double* noalloc_scratch(int dev)
+__global__ void __launch_bounds__(kNoAllocMaxCols) k_zero_counts(uint32_t* __restrict__ done)
 {
-    if (dev < 0 || dev >= kMaxDevices) throw Error(ERR_HIP, "Device index out of range: " + std::to_string(dev));
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_ptr[dev]) {
-        void* p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p) {
-            (void)hipGetLastError();
-            throw Error(ERR_HIP, std::string("hipGetSymbolAddress of the marginal scratch failed: ") +
-                                     hipGetErrorString(e));
-        }
-        g_scratch_ptr[dev] = static_cast<double*>(p);
+    done[threadIdx.x] = 0;
+}
+
+// The array on one device.  A call holds the mutex from its launch to the end
+// of its stream's work: two calls at once would share the counts, and a count
+// that one of them left non-zero would spoil every later call.
+struct NoAllocScratch {
+    std::mutex mu;
+    double* p = nullptr;      // device address, looked up at the first call
+    bool counts_zero = true;  // false once a call has not come to its end
+};
+static constexpr int kMaxDevices = 64;
+static NoAllocScratch g_scratch[kMaxDevices];
+
+// The device address of `scratch` on the current device.  The array's name is
+// not a device address in host code; only this pointer is passed to kernels
+// and copies.
+static double* noalloc_address()
+{
+    void* p = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    if (e != hipSuccess || !p) {
+        (void)hipGetLastError();
+        throw Error(ERR_HIP, std::string("hipGetSymbolAddress of the marginal scratch failed: ") +
+                                 hipGetErrorString(e));
     }
-    return g_scratch_ptr[dev];
+    return static_cast<double*>(p);
 }
 
 void GpuVectorState::marginal_w0_noalloc(size_t qbit, double* w0s, size_t len)
@@ -1213,13 +1220,25 @@ void GpuVectorState::marginal_w0_noalloc(size_t qbit, double* w0s, size_t len)
     if (dev != device_)
         throw Error(ERR_INVALID_ARGUMENT, "The state lives on device " + std::to_string(device_) +
                                               ", but device " + std::to_string(dev) + " is current");
-    double* part = noalloc_scratch(dev);
+    if (dev < 0 || dev >= kMaxDevices) throw Error(ERR_HIP, "Device index out of range: " + std::to_string(dev));
+    NoAllocScratch& sc = g_scratch[dev];
+    std::lock_guard<std::mutex> lk(sc.mu);
+    if (!sc.p) sc.p = noalloc_address();
+    double* part = sc.p;
     double* w = part + kNoAllocW0;
+    uint32_t* done = reinterpret_cast<uint32_t*>(part + kNoAllocDone);
     const int p = int(nr_bits_ - 1 - qbit);
-    launch_marginal_cols(prec_ == PREC_C64, col_ptr(0), dim(), uint32_t(nc), dim() / 2, p, BASIS_Z, part,
-                         reinterpret_cast<uint32_t*>(part + kNoAllocDone), w, stream_);
+    if (!sc.counts_zero) {
+        HIP_OK(hipDeviceSynchronize());   // the call that failed may still count
+        hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(kNoAllocMaxCols), 0, stream_, done);
+        HIP_OK(hipGetLastError());
+    }
+    sc.counts_zero = false;
+    launch_marginal_cols(prec_ == PREC_C64, col_ptr(0), dim(), uint32_t(nc), dim() / 2, p, BASIS_Z, part, done, w,
+                         stream_);
     HIP_OK(hipMemcpyAsync(w0s, w, nc * sizeof(double), hipMemcpyDeviceToHost, stream_));
     HIP_OK(hipStreamSynchronize(stream_));
+    sc.counts_zero = true;
 }
 
 // The bits written and the collapse of measure_into (vectorstate.rs:237-329)
