@@ -795,6 +795,13 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
     std::vector<PlanStep> steps;
     std::vector<SweepProgram> progs;
     choose_plan(st, queue, g, fusion_k, S, tiles, steps, progs);
+    // recorded sweeps carry the features the planner predicts from: those of
+    // the programs as it chose them
+    std::vector<std::array<float, kSweepFeatures>> feat(st.recording() ? steps.size() : 0);
+    for (size_t s = 0; s < feat.size(); ++s)
+        if (steps[s].sweep)
+            sweep_features(progs[s].phases, progs[s].ops, steps[s], int(st.precision()), g, st.jit_enabled(),
+                           feat[s].data());
     reduce_programs(progs, st.precision());
     for (SweepProgram& p : progs) place_phases(p.phases, g.M, g.R, st.elem_bytes());
 
@@ -897,11 +904,7 @@ void run_planned(GpuVectorState& st, const std::vector<PendingGate>& queue, size
                 default: throw Error(ERR_INVALID_ARGUMENT, "No sweep kernel for this complex64 tile shape");
                 }
             }
-            if (st.recording() && col_end - col_begin <= 65535) {
-                float f[kSweepFeatures];
-                sweep_features(progs[s].phases, progs[s].ops, step, int(st.precision()), g, jf != nullptr, f);
-                st.add_sample(f, tiles, slot);
-            }
+            if (st.recording() && col_end - col_begin <= 65535) st.add_sample(feat[s].data(), tiles, slot);
             stats.launches += 1;
             stats.sweeps += 1;
             stats.gates += step.gates.size();
