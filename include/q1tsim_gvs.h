@@ -147,8 +147,9 @@ int q1t_gvs_flush(q1t_gvs* s);
  * runs that fit an LDS tile in one HBM sweep. */
 int q1t_gvs_set_plan(q1t_gvs* s, int fusion_k, int tiling);
 /* Build-added: local search of the sweep tiles and register phases; mode -1
- * (default) tiles always and phases for states of 512 MiB and more, 0 never,
- * 1 always.  Changes only the schedule, not the gates applied. */
+ * (default) tiles always (in a complex64 batch for states of 512 MiB and more)
+ * and phases for states of 512 MiB and more, 0 never, 1 always.  Changes only
+ * the schedule, not the gates applied. */
 int q1t_gvs_set_plan_search(q1t_gvs* s, int mode);
 /* Build-added, no counterpart in the reference: flush graphs (on = 1).  The
  * kernel launches of a planned flush are captured into one hipGraph; a later
@@ -250,7 +251,7 @@ int q1t_gvs_set_cost_model(q1t_gvs* s, q1t_cost_model* cm, int mode, uint64_t se
 /* record every sweep's features and measured time (turns profiling on) */
 int q1t_gvs_set_recording(q1t_gvs* s, int on);
 /* move up to cap recorded samples out, oldest first (the rest stay):
- * feat[cap][16], tiles[cap] (tiles over all columns), ms[cap] */
+ * feat[cap][Q1T_CM_FEATURES], tiles[cap] (tiles over all columns), ms[cap] */
 int q1t_gvs_take_samples(q1t_gvs* s, float* feat, double* tiles, double* ms, size_t cap, size_t* count);
 
 #ifdef __cplusplus

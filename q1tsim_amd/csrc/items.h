@@ -7,7 +7,7 @@
 // the sampling walk), uploads the item tables in one copy, launches one
 // kernel per kind in dependency order and has the kernels write the results
 // to host memory.  The single-state paths run the same kernels through a queue
-// of their own, so a state gives the same bits alone and in a batch.
+// of their own, so the same amplitudes give the same bits there.
 #pragma once
 
 #include <hip/hip_runtime.h>
