@@ -147,9 +147,10 @@ int q1t_gvs_flush(q1t_gvs* s);
  * runs that fit an LDS tile in one HBM sweep. */
 int q1t_gvs_set_plan(q1t_gvs* s, int fusion_k, int tiling);
 /* Build-added: local search of the sweep tiles and register phases; mode -1
- * (default) tiles always (in a complex64 batch for states of 512 MiB and more)
- * and phases for states of 512 MiB and more, 0 never, 1 always.  Changes only
- * the schedule, not the gates applied. */
+ * (default) tiles always (with dense blocks of 5 and 6 qubits for states of 128
+ * MiB and more, in a complex64 batch of 512 MiB and more) and phases for states
+ * of 512 MiB and more, 0 never, 1 always.  Changes only the schedule, not the
+ * gates applied. */
 int q1t_gvs_set_plan_search(q1t_gvs* s, int mode);
 /* Build-added, no counterpart in the reference: flush graphs (on = 1).  The
  * kernel launches of a planned flush are captured into one hipGraph; a later

@@ -266,13 +266,25 @@ public:
     }
     CostModel* cost_model() const { return cost_model_; }
     int plan_mode() const { return plan_mode_; }
-    // local search of tiles and register phases: -1 tiles always and phases by
-    // state size, 0 off, 1 on
+    // local search of tiles and register phases: -1 by fusion width and state
+    // size, 0 off, 1 on
     void set_plan_search(int mode) { plan_search_ = mode; }
     // Tiles: the search halves the sweeps (20-layer circuits: 16 qubits 10 -> 5,
     // 23 qubits 21 -> 10) for 0.02 ms of host time at 16 qubits and 0.4 ms at
-    // 23, less than a sweep or two.
-    bool tile_search() const { return plan_search_ != 0; }
+    // 23, less than a sweep or two.  Plans with dense blocks of 5 and 6 qubits
+    // search from 128 MiB on: fewer sweeps fill their blocks to the full width,
+    // and composing a block on the host costs 4^width per gate, which outweighs
+    // the sweeps saved on smaller states (ms per flush greedy / searched, 12
+    // layers, width 5: 18 qubits 0.80 / 1.04, 21 1.02 / 1.28, 23 1.82 / 2.13, 24
+    // 2.75 / 2.77, 25 layers 6.02 / 5.89; width 6: 20 qubits 3.12 / 3.77, 24
+    // 7.45 / 6.54; width 4: 18 qubits 0.43 / 0.44, 20 0.50 / 0.53, 24 2.12 / 1.75).
+    bool tile_search(int fusion_k, double state_bytes) const
+    {
+        if (plan_search_ < 0 && fusion_k > 4) return state_bytes >= 128.0 * 1024.0 * 1024.0;
+        return plan_search_ != 0;
+    }
+    // the last plan is kept for a flush of the same structure
+    bool plan_cache() const { return plan_search_ != 0; }
     // Phases: the search saves about a fifth of a sweep's LDS exchanges for
     // 0.04 ms per sweep, which pays once a sweep takes a millisecond.
     bool phase_search(double state_bytes) const

@@ -391,7 +391,9 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
 {
     const int n = int(st.nr_bits());
     const int prec = int(st.precision());
-    const bool search = st.tile_search(), phase_search = st.phase_search(state_bytes);
+    const bool fused = st.precision() == PREC_C64 && fusion_k > 0;
+    const bool search = st.tile_search(fused ? fusion_k : 0, state_bytes);
+    const bool phase_search = st.phase_search(state_bytes), keep = st.plan_cache();
     const bool factors = st.tile_factors();   // specialised kernels only
     auto build_all = [&](const std::vector<PlanStep>& ss, int kind) {
         std::vector<SweepProgram> out(ss.size());
@@ -399,7 +401,6 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
             if (ss[s].sweep) out[s] = build_candidate(queue, ss[s], g, kind, phase_search, factors);
         return out;
     };
-    const bool fused = st.precision() == PREC_C64 && fusion_k > 0;
     // A flush with the previous flush's gate structure (a repeated circuit,
     // new angles allowed) takes that flush's steps and per-sweep program
     // kinds and builds only those programs: the tile searches (and the
@@ -419,7 +420,7 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
                                                       [](void* p) { delete static_cast<PlanCacheEntry*>(p); });
     };
     if (!fused) {
-        if (search) {
+        if (keep) {
             key = plan_key(queue, n, g, 0, search);
             key.insert(key.begin(), 1);   // the per-gate planner
             std::vector<int> kind;
@@ -438,7 +439,7 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
     CostModel* cm = st.cost_model();
     const int mode = st.plan_mode();
     if (mode == PLAN_GREEDY || (mode == PLAN_LEARNED && (!cm || !cm->trained()))) {
-        if (search) {
+        if (keep) {
             key = plan_key(queue, n, g, Kg, search);
             key.insert(key.begin(), 3);   // greedy fusion
             std::vector<int> kind;
@@ -452,7 +453,7 @@ static void choose_plan(GpuVectorState& st, const std::vector<PendingGate>& queu
         progs = build_all(steps, Kg);
         return;
     }
-    const bool cacheable = search && mode == PLAN_LEARNED;
+    const bool cacheable = keep && mode == PLAN_LEARNED;
     if (cacheable) {
         // both tilings' inputs, the block width, the model, the kernels the
         // predictions are for and the bytes swept (single gates are costed
@@ -1052,7 +1053,7 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
         const bool search = live[i]->phase_search(S);
         // complex64: the greedy tiles, whose order of the gates' rounding a
         // seeded batch's outcomes depend on
-        p.steps = plan_gates(q, n, g, K, prec == PREC_C128 ? live[i]->tile_search() : search);
+        p.steps = plan_gates(q, n, g, K, prec == PREC_C128 ? live[i]->tile_search(0, S) : search);
         p.ph.resize(p.steps.size());
         p.ops.resize(p.steps.size());
         int nblocks = 0;

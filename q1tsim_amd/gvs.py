@@ -179,9 +179,10 @@ class GpuVectorState:
         check(lib().q1t_gvs_set_plan(self.h, int(fusion_k), 1 if tiling else 0))
 
     def set_plan_search(self, mode=-1):
-        """Local search of tiles and register phases: -1 tiles always (in a
-        complex64 batch for states of 512 MiB and more) and phases for states
-        of 512 MiB and more, 0 never, 1 always."""
+        """Local search of tiles and register phases: -1 tiles always (with
+        dense blocks of 5 and 6 qubits for states of 128 MiB and more, in a
+        complex64 batch of 512 MiB and more) and phases for states of 512 MiB
+        and more, 0 never, 1 always."""
         check(lib().q1t_gvs_set_plan_search(self.h, int(mode)))
 
     def set_graph(self, on=True):
