@@ -807,8 +807,9 @@ void build_program(const std::vector<PendingGate>& q, const PlanStep& step, int 
     append_factors(tf, M, phases, ops, order);
 }
 
-// A gate's largest entry is at least 2^-1/2 for what reduce_op takes: after
-// this many gates the amplitudes have grown by at most 2^40 (complex64), 2^400.
+// reduce_op takes gates whose rows have a squared norm above 0.75, so the entry
+// it divides by is at least 0.61: after this many gates the amplitudes have grown
+// by at most 2^57 (complex64), 2^566.
 static int reduction_limit(Precision prec) { return prec == PREC_C128 ? 800 : 80; }
 
 static void set_coefs(SwOp& o, cdouble a)

@@ -628,7 +628,8 @@ static bool put_single_gates(const std::vector<PendingGate>& queue, const PlanSt
     bool ok = true;
     for (size_t i : step.gates) {
         const GateOp& op = queue[i].op;
-        // a kernel of 3+ targets uploads its matrix and synchronises
+        // kernels of 4 and more targets upload their matrix and synchronise;
+        // those of 3 run eagerly with them
         if (op.kind == OpKind::Dense && op.targets.size() >= 3) ok = false;
         put(uint64_t(op.kind));
         put(op.ctrl_mask);
