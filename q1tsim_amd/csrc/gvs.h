@@ -255,7 +255,8 @@ public:
     // queue, so it outlives the state): the copy from it is over when the
     // flush has synchronised.
     char* stage(size_t bytes) { return iq().stage(bytes, stream_); }
-    void apply_op(const GateOp& op, size_t col_begin, size_t col_end);
+    // one gate on its own kernel; `fused`: rounded as the whole-state programs do
+    void apply_op(const GateOp& op, size_t col_begin, size_t col_end, bool fused = false);
 
     // planner: learned cost model (not owned) and mode; recording of sweeps
     void set_cost_model(CostModel* cm, int mode, uint64_t seed)

@@ -31,7 +31,9 @@ namespace q1t {
 // ------------------------------------------------------------------ kernels
 
 // One-qubit dense update on every (i0, i0|tbit) pair whose control bits are 1.
-template <typename V>
+// FUSED: the second product is fused into the sum, as in k_whole, for gates that
+// run here in the place of a launch of it.
+template <typename V, bool FUSED>
 __global__ void __launch_bounds__(kBlock) k_dense1(V* __restrict__ amp, uint64_t col_stride, uint64_t nwork,
                                                    PosList pos, uint64_t cmask, uint64_t tbit, V m0, V m1, V m2, V m3)
 {
@@ -40,8 +42,13 @@ __global__ void __launch_bounds__(kBlock) k_dense1(V* __restrict__ amp, uint64_t
     for (uint64_t j = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < nwork; j += step) {
         const uint64_t i0 = deposit(j, pos) | cmask, i1 = i0 | tbit;
         const V x = a[i0], y = a[i1];
-        a[i0] = cadd(cmul(m0, x), cmul(m1, y));
-        a[i1] = cadd(cmul(m2, x), cmul(m3, y));
+        if constexpr (FUSED) {
+            a[i0] = cmac(cmul(m0, x), m1, y);
+            a[i1] = cmac(cmul(m2, x), m3, y);
+        } else {
+            a[i0] = cadd(cmul(m0, x), cmul(m1, y));
+            a[i1] = cadd(cmul(m2, x), cmul(m3, y));
+        }
     }
 }
 
@@ -850,7 +857,7 @@ void GpuVectorState::apply_queue_plain(size_t cb, size_t ce)
 
 template <typename V>
 static void launch_op(const GateOp& op, V* amp, uint64_t col_stride, size_t ncols, int n, hipStream_t st,
-                      GpuVectorState& gs, RunStats& stats)
+                      GpuVectorState& gs, RunStats& stats, bool fused)
 {
     if (op.kind == OpKind::Identity) {
         stats.gates += 1;
@@ -908,9 +915,10 @@ static void launch_op(const GateOp& op, V* amp, uint64_t col_stride, size_t ncol
             if (kt == 1) {
                 kname = "k_dense1";
                 ps = gs.prof_begin();
-                hipLaunchKernelGGL(k_dense1<V>, dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride, nwork,
-                                   pl, op.ctrl_mask, uint64_t(1) << op.targets[0], to_v<V>(op.m[0]),
-                                   to_v<V>(op.m[1]), to_v<V>(op.m[2]), to_v<V>(op.m[3]));
+                auto k = fused ? k_dense1<V, true> : k_dense1<V, false>;
+                hipLaunchKernelGGL(k, dim3(grid_for(nwork), ny), dim3(kBlock), 0, st, a, col_stride, nwork, pl,
+                                   op.ctrl_mask, uint64_t(1) << op.targets[0], to_v<V>(op.m[0]), to_v<V>(op.m[1]),
+                                   to_v<V>(op.m[2]), to_v<V>(op.m[3]));
             } else if (kt == 2) {
                 Mat4<V> m4{};
                 for (int k = 0; k < 16; ++k) m4.m[k] = to_v<V>(op.m[k]);
@@ -976,13 +984,15 @@ void* GpuVectorState::scratch(int slot, size_t bytes)
     return d_slot_[slot];
 }
 
-void GpuVectorState::apply_op(const GateOp& op, size_t cb, size_t ce)
+void GpuVectorState::apply_op(const GateOp& op, size_t cb, size_t ce, bool fused)
 {
     if (ce <= cb) return;
     if (prec_ == PREC_C128)
-        launch_op<double2>(op, static_cast<double2*>(col_ptr(cb)), dim(), ce - cb, int(nr_bits_), stream_, *this, stats_);
+        launch_op<double2>(op, static_cast<double2*>(col_ptr(cb)), dim(), ce - cb, int(nr_bits_), stream_, *this, stats_,
+                           fused);
     else
-        launch_op<float2>(op, static_cast<float2*>(col_ptr(cb)), dim(), ce - cb, int(nr_bits_), stream_, *this, stats_);
+        launch_op<float2>(op, static_cast<float2*>(col_ptr(cb)), dim(), ce - cb, int(nr_bits_), stream_, *this, stats_,
+                           fused);
 }
 
 // collect_conditional_ranges (qustate.rs:100-127): runs of equal control

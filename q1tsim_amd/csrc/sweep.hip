@@ -220,21 +220,21 @@ static int whole_bits(int n) { return std::max(n, whole_regs(n)); }
 // qubits).  Measured: 12 qubits complex128, 350 gates 1110 -> 115 us; 112
 // columns of 10 to 13 qubits complex64 in a batch 2850 -> 150 us per round.
 template <typename V, int R>
-__global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ items,
+__global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ items, uint64_t col_stride,
                                                 const WholePhase* __restrict__ phases,
                                                 const InterpOpT<typename RealOf<V>::type>* __restrict__ ops)
 {
     constexpr int NR = 1 << R;
     extern __shared__ unsigned char smem_whole[];
     V* s = reinterpret_cast<V*>(smem_whole);
-    const WholeItem it = load_uniform(items, blockIdx.x);
+    const WholeItem it = load_uniform(items, col_stride ? 0u : blockIdx.x);
     const int M = int(it.n) > R ? int(it.n) : R, sw = sweep_swizzle_bits(M);
     const uint32_t nth = 1u << (M - R), N = 1u << it.n, tid = threadIdx.x;
     const uint32_t nops = it.nphases ? load_uniform(phases, it.phases + it.nphases - 1).op_end : 0u;
     if (it.nphases) warm_program(phases + it.phases, it.nphases * uint32_t(sizeof(WholePhase)));
     if (nops) warm_program(ops + it.ops, nops * uint32_t(sizeof(InterpOpT<typename RealOf<V>::type>)));
     if (tid >= nth) return;
-    V* a = static_cast<V*>(it.amp);
+    V* a = static_cast<V*>(it.amp) + uint64_t(blockIdx.x) * col_stride;
     {
         V x[NR];
 #pragma unroll
@@ -283,20 +283,21 @@ __global__ void __launch_bounds__(1024) k_whole(const WholeItem* __restrict__ it
     }
 }
 
-// `nitems` columns of states of at most n_max qubits (the LDS and threads of
-// the widest).  Tables in device memory; the op table ends with a spare record.
+// `ncols` columns of states of at most n_max qubits (the LDS and threads of
+// the widest): an item each, or one item for columns at stride col_stride.
+// Tables in device memory; the op table ends with a spare record.
 template <typename V>
-static void launch_whole(int n_max, const WholeItem* items, size_t nitems, const WholePhase* phases,
-                         const InterpOpT<typename RealOf<V>::type>* ops, hipStream_t stream)
+static void launch_whole(int n_max, const WholeItem* items, size_t ncols, uint64_t col_stride,
+                         const WholePhase* phases, const InterpOpT<typename RealOf<V>::type>* ops, hipStream_t stream)
 {
     const int R = whole_regs(n_max), M = whole_bits(n_max);
     const size_t lds = sizeof(V) << M;
-    const dim3 grid{unsigned(nitems)}, block{unsigned(std::max(64, 1 << (M - R)))};
+    const dim3 grid{unsigned(ncols)}, block{unsigned(std::max(64, 1 << (M - R)))};
     auto go = [&](auto kernel) {
         if (lds > (size_t(64) << 10))
             SW_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-        hipLaunchKernelGGL(kernel, grid, block, lds, stream, items, phases, ops);
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, items, col_stride, phases, ops);
     };
     if (R == 3) go(&k_whole<V, 3>);
     else if constexpr (sizeof(V) == 8) go(&k_whole<V, 4>);
@@ -714,6 +715,21 @@ static void run_table(GpuVectorState& st, const char* host, size_t total, std::v
 // A flush of a state that is too small for tiles: whole-state programs
 // (k_whole), one launch for all columns, and single-gate kernels for the gates
 // no register phase takes.
+// A run of few gates between those goes to the single-gate kernels too, with the
+// same rounding (2.9 us a gate): a launch of k_whole reads its program first and
+// holds a column in one workgroup.  us per two-qubit unitary and run of gates,
+// k_whole / single kernels, complex128: 8 qubits 1 gate 8.4 / 7.1, 2 gates 8.4 /
+// 10.4; 12 qubits 1 gate 10.3 / 7.3, 2 10.5 / 10.4, 3 11.2 / 13.4; 13 qubits 2 12.6
+// / 10.5, 3 13.4 / 13.3, 4 14.6 / 16.7; 512 columns of 12 qubits 1 26.6 / 23.5, 2
+// 26.9 / 33.4.  Where the run is the whole flush, one gate more saves the table's
+// upload (8 qubits, 2 gates 17.5 / 14.6, 3 gates 18.2 / 17.2, 4 18.6 / 19.4).
+static size_t lone_gates(int n, size_t ncols, bool whole_flush)
+{
+    const uint64_t amps = uint64_t(ncols) << n;
+    const size_t few = n <= 11 || amps > (uint64_t(1) << 20) ? 1 : n == 12 ? 2 : 3;
+    return few + (whole_flush && amps <= (uint64_t(1) << 17));
+}
+
 template <typename V>
 static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
                       bool fresh, RunStats& stats)
@@ -721,32 +737,42 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
     using R = typename RealOf<V>::type;
     const int n = int(st.nr_bits());
     const size_t ncols = col_end - col_begin;
-    const std::vector<PlanStep> steps = plan_whole(queue, whole_bits(n));
+    bool graph = st.graph_enabled();
+    std::vector<PlanStep> steps = plan_whole(queue, whole_bits(n));
+    // not for a graph, which replays programs with new angles but no single gates,
+    // nor for the first gates of an unwritten state
+    if (!graph) {
+        const size_t few = lone_gates(n, ncols, steps.size() == 1);
+        for (size_t s = fresh ? 1 : 0; s < steps.size(); ++s)
+            if (steps[s].gates.size() <= few) steps[s].sweep = false;
+    }
     WholeTables<R> wt;
     wt.build(queue, steps, n);
+    bool any = false;   // a step of k_whole
+    for (const PlanStep& step : steps) any = any || step.sweep;
     wt.ops.push_back(InterpOpT<R>{});   // the spare record
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
     const size_t ooff = up(wt.phases.size() * sizeof(WholePhase));
     const size_t ioff = up(ooff + wt.ops.size() * sizeof(InterpOpT<R>));
-    const size_t total = up(ioff + steps.size() * ncols * sizeof(WholeItem));
-    char* const host = st.stage(total);
-    std::memcpy(host, wt.phases.data(), wt.phases.size() * sizeof(WholePhase));
-    std::memcpy(host + ooff, wt.ops.data(), wt.ops.size() * sizeof(InterpOpT<R>));
-    WholeItem* items = reinterpret_cast<WholeItem*>(host + ioff);   // step-major
-    for (size_t s = 0; s < steps.size(); ++s)
-        for (size_t c = 0; c < ncols; ++c)
-            items[s * ncols + c] = WholeItem{st.col_ptr(col_begin + c), uint32_t(n), wt.nph[s], wt.ph0[s], wt.op0[s],
-                                             fresh && s == 0, 0};
+    const size_t total = any ? up(ioff + steps.size() * sizeof(WholeItem)) : 0;
+    char* const host = any ? st.stage(total) : nullptr;
+    if (any) {
+        std::memcpy(host, wt.phases.data(), wt.phases.size() * sizeof(WholePhase));
+        std::memcpy(host + ooff, wt.ops.data(), wt.ops.size() * sizeof(InterpOpT<R>));
+        WholeItem* items = reinterpret_cast<WholeItem*>(host + ioff);   // one per step, of its first column
+        for (size_t s = 0; s < steps.size(); ++s)
+            items[s] = WholeItem{st.col_ptr(col_begin), uint32_t(n), wt.nph[s], wt.ph0[s], wt.op0[s], fresh && s == 0, 0};
+    }
     if (fresh && (steps.empty() || !steps[0].sweep)) st.write_zero_state();
     const double S = double(uint64_t(1) << n) * sizeof(V) * double(ncols);
     auto launch_all = [&](char* d) {
         for (size_t s = 0; s < steps.size(); ++s) {
             if (!steps[s].sweep) {
-                for (size_t i : steps[s].gates) st.apply_op(queue[i].op, col_begin, col_end);
+                for (size_t i : steps[s].gates) st.apply_op(queue[i].op, col_begin, col_end, true);
                 continue;
             }
             const int ps = st.prof_begin();
-            launch_whole<V>(n, reinterpret_cast<const WholeItem*>(d + ioff) + s * ncols, ncols,
+            launch_whole<V>(n, reinterpret_cast<const WholeItem*>(d + ioff) + s, ncols, uint64_t(1) << n,
                             reinterpret_cast<const WholePhase*>(d),
                             reinterpret_cast<const InterpOpT<R>*>(d + ooff), st.stream());
             st.prof_end(ps, sizeof(V) == 16 ? "k_whole_c128" : "k_whole_c64", 2.0 * S);
@@ -757,7 +783,6 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
             stats.phases += wt.nph[s];
         }
     };
-    bool graph = st.graph_enabled();
     std::vector<uint64_t> sig;
     if (graph) {
         for (uint64_t x : {uint64_t(n), uint64_t(st.precision()), uint64_t(col_begin), uint64_t(col_end),
@@ -1279,10 +1304,10 @@ void run_planned_batch(const std::vector<GpuVectorState*>& states, hipStream_t s
             const WholeItem* wi = reinterpret_cast<const WholeItem*>(dbase + wioff) + wg.first;
             const WholePhase* wp = reinterpret_cast<const WholePhase*>(dbase + wpoff);
             if (prec == PREC_C128)
-                launch_whole<double2>(wg.n_max, wi, wg.count, wp,
+                launch_whole<double2>(wg.n_max, wi, wg.count, 0, wp,
                                       reinterpret_cast<const InterpOpT<double>*>(dbase + wooff), stream);
             else
-                launch_whole<float2>(wg.n_max, wi, wg.count, wp,
+                launch_whole<float2>(wg.n_max, wi, wg.count, 0, wp,
                                      reinterpret_cast<const InterpOpT<float>*>(dbase + wooff), stream);
             agg.launches += 1;
         }

@@ -133,7 +133,7 @@ struct WholePhase {
 };
 
 struct WholeItem {
-    void* amp;           // the column
+    void* amp;           // the column (the first of a launch with a column stride)
     uint32_t n;          // qubits
     uint32_t nphases;
     uint32_t phases, ops;   // first records in the tables
