@@ -101,6 +101,18 @@ static constexpr uint64_t marg_units(size_t elem_bytes) { return uint64_t(kMargT
 // read.  Smaller ones may be.
 static constexpr uint64_t kStreamBytes = uint64_t(512) << 20;
 
+// Up to this many shares of all columns one launch does it all: the last share of
+// a column adds them.  Its count takes an agent-scope release and acquire, which
+// write back and invalidate an XCD's L2, so that many shares slow each other
+// down: above, they are added by a launch of their own.  us per marginal (Z) in
+// one launch / in two: 20 qubits complex128, 4 columns (512 shares) 30.4 / 23.9, 16
+// columns 95 / 42; 22 qubits complex64, 8 columns 95 / 50; 4096 circuits of 10 to
+// 22 qubits complex128 10050 / 2710.
+static constexpr uint64_t kMargOneLaunch = kMargBlocks;
+// Workgroups of the two launches' first: each takes consecutive shares and looks
+// their item up once (the same circuits in complex64, us: a workgroup per share
+// 1170, 4096 workgroups 920).
+static constexpr uint64_t kMargGrid = 4096;
 // Workgroups of a column: one per marg_units() work units, at most kMargBlocks
 // (one per CU; the partial sums of a column then fit one workgroup).
 static uint32_t marginal_blocks(bool c64, uint64_t nwork)
@@ -163,46 +175,43 @@ __device__ __forceinline__ double marginal_acc(const V* a, uint64_t nwork, int p
     return acc;
 }
 
-__device__ __forceinline__ double marg_block_total(double v)
+template <int THREADS = kMargThreads> __device__ __forceinline__ double marg_block_total(double v)
 {
-    __shared__ double red[kMargThreads / 64];
+    __shared__ double red[THREADS / 64];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     double s = 0.0;
     if (threadIdx.x == 0)
-        for (int k = 0; k < kMargThreads / 64; ++k) s += red[k];
+        for (int k = 0; k < THREADS / 64; ++k) s += red[k];
     __syncthreads();   // red is reused by the next call
     return s;
 }
 
-// The share of workgroup b of nb of one column; the workgroup that finishes
-// last adds the partial sums (a fixed tree, so the result does not depend on
-// which one that is) and writes the weight.  Partial sums and the count of
-// finished workgroups go through agent-scope atomics: the XCDs' L2 caches are
-// not coherent with each other.  The count is zero again when the column is
-// done.
+// Share b of nb of one column.
 template <typename V>
-__device__ __forceinline__ void marginal_block(const V* a, uint64_t nwork, int p, int basis, uint32_t b, uint32_t nb,
-                                               bool stream, double* partial, uint32_t* done, double* w0)
+__device__ __forceinline__ double marginal_share(const V* a, uint64_t nwork, int p, int basis, uint32_t b, uint32_t nb)
 {
-    const double acc = stream ? marginal_acc<V, true>(a, nwork, p, basis, b, nb)
-                              : marginal_acc<V, false>(a, nwork, p, basis, b, nb);
-    double s = marg_block_total(acc);
-    if (nb == 1) {
-        if (threadIdx.x == 0) *w0 = s;
-        return;
-    }
+    const double acc = 2 * nwork * sizeof(V) >= kStreamBytes ? marginal_acc<V, true>(a, nwork, p, basis, b, nb)
+                                                             : marginal_acc<V, false>(a, nwork, p, basis, b, nb);
+    return marg_block_total(acc);
+}
+
+// Another share of a column of nb is in `partial`: the workgroup that brings the
+// last one adds all of them (a fixed tree, so the result does not depend on which
+// one that is) and writes the weight.  Partial sums and the count of finished
+// shares go through agent-scope atomics: the XCDs' L2 caches are not coherent
+// with each other.  The count is zero again when the column is done.
+__device__ __forceinline__ void marginal_finish(uint32_t nb, const double* partial, uint32_t* done, double* w0)
+{
     __shared__ uint32_t last;
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(partial + b, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
-    }
     __syncthreads();
     if (!last) return;
     double v = 0.0;
     if (threadIdx.x < nb) v = __hip_atomic_load(partial + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s = marg_block_total(v);
+    const double s = marg_block_total(v);
     if (threadIdx.x == 0) {
         *w0 = s;
         __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -212,41 +221,105 @@ __device__ __forceinline__ void marginal_block(const V* a, uint64_t nwork, int p
 // Chunk c: share c - chunk0 of its item; partial sums at partial[c].
 template <typename V>
 __global__ void __launch_bounds__(kMargThreads) k_marginal_items(MargItem one, const MargItem* __restrict__ items,
-                                                                 uint32_t n, uint64_t nchunks, double* partial,
-                                                                 uint32_t* done, double* w0)
+                                                                 uint32_t n, double* partial, uint32_t* done,
+                                                                 double* w0)
 {
-    for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const uint32_t it = items ? find_item(items, n, c) : 0;
-        const MargItem m = items ? items[it] : one;
-        marginal_block<V>(static_cast<const V*>(m.amp), m.nwork, m.p, m.basis, uint32_t(c - m.chunk0), m.blocks,
-                          2 * m.nwork * sizeof(V) >= kStreamBytes, partial + m.chunk0, done + it, w0 + it);
-        __syncthreads();   // the shared sums and flag are reused by the next chunk
+    const uint64_t c = blockIdx.x;
+    const uint32_t it = items ? find_item(items, n, c) : 0;
+    const MargItem m = items ? items[it] : one;
+    const double s = marginal_share<V>(static_cast<const V*>(m.amp), m.nwork, m.p, m.basis, uint32_t(c - m.chunk0),
+                                       m.blocks);
+    if (threadIdx.x == 0) {
+        if (m.blocks == 1) w0[it] = s;
+        else __hip_atomic_store(partial + c, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (m.blocks > 1) marginal_finish(m.blocks, partial + m.chunk0, done + it, w0 + it);
+}
+
+// The shares of many columns, `run` consecutive ones per workgroup; partial[c] is
+// added up by k_marginal_sums.
+template <typename V>
+__global__ void __launch_bounds__(kMargThreads) k_marginal_shares(const MargItem* __restrict__ items, uint32_t n,
+                                                                  uint64_t nchunks, uint32_t run,
+                                                                  double* __restrict__ partial,
+                                                                  double* __restrict__ w0)
+{
+    uint64_t c = uint64_t(blockIdx.x) * run;
+    const uint64_t c1 = c + run < nchunks ? c + run : nchunks;
+    for (uint32_t it = find_item(items, n, c); c < c1; ++it) {
+        const MargItem m = items[it];
+        const uint64_t end = m.chunk0 + m.blocks < c1 ? m.chunk0 + m.blocks : c1;
+        for (; c < end; ++c) {
+            const double s = marginal_share<V>(static_cast<const V*>(m.amp), m.nwork, m.p, m.basis,
+                                               uint32_t(c - m.chunk0), m.blocks);
+            if (threadIdx.x == 0) {
+                if (m.blocks == 1) w0[it] = s;
+                else partial[c] = s;
+            }
+        }
     }
 }
 
-// The same for `gridDim.y` columns at stride col_stride (no item table: the
-// allocation-free marginal).
-template <typename V>
+// The weights of the columns of several shares, a workgroup per column: the sum of
+// marginal_finish.  Without a table every column has nb shares, at stride
+// kMargBlocks.
+__global__ void __launch_bounds__(kMargBlocks) k_marginal_sums(const MargItem* __restrict__ items, uint32_t n,
+                                                               uint32_t nb, const double* __restrict__ partial,
+                                                               double* __restrict__ w0)
+{
+    for (uint32_t it = blockIdx.x; it < n; it += gridDim.x) {
+        uint64_t at = uint64_t(it) * kMargBlocks;
+        if (items) {
+            at = items[it].chunk0;
+            nb = items[it].blocks;
+        }
+        if (nb == 1) continue;
+        const double s = marg_block_total<kMargBlocks>(threadIdx.x < nb ? partial[at + threadIdx.x] : 0.0);
+        if (threadIdx.x == 0) w0[it] = s;
+    }
+}
+
+// The shares of `gridDim.y` columns at stride col_stride (no item table: the
+// allocation-free marginal); ONE: added here, else by k_marginal_sums.
+template <typename V, bool ONE>
 __global__ void __launch_bounds__(kMargThreads) k_marginal_cols(const V* __restrict__ amp, uint64_t col_stride,
                                                                 uint64_t nwork, int p, int basis, double* partial,
                                                                 uint32_t* done, double* w0)
 {
-    const uint32_t c = blockIdx.y;
-    marginal_block<V>(amp + uint64_t(c) * col_stride, nwork, p, basis, blockIdx.x, gridDim.x,
-                      2 * nwork * sizeof(V) >= kStreamBytes, partial + uint64_t(c) * kMargBlocks, done + c, w0 + c);
+    const uint32_t c = blockIdx.y, nb = gridDim.x;
+    double* const part = partial + uint64_t(c) * kMargBlocks;
+    const double s = marginal_share<V>(amp + uint64_t(c) * col_stride, nwork, p, basis, blockIdx.x, nb);
+    if (threadIdx.x == 0) {
+        if (nb == 1) w0[c] = s;
+        else __hip_atomic_store(part + blockIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if constexpr (ONE)
+        if (nb > 1) marginal_finish(nb, part, done + c, w0 + c);
+}
+
+template <typename V>
+static void marginal_cols(const V* amp, uint64_t col_stride, uint32_t ncols, uint64_t nwork, int p, int basis,
+                          double* partial, uint32_t* done, double* w0, hipStream_t s)
+{
+    const uint32_t nb = marginal_blocks(sizeof(V) == 8, nwork);
+    const bool one = nb == 1 || uint64_t(nb) * ncols <= kMargOneLaunch;
+    auto k = one ? k_marginal_cols<V, true> : k_marginal_cols<V, false>;
+    hipLaunchKernelGGL(k, dim3(nb, ncols), dim3(kMargThreads), 0, s, amp, col_stride, nwork, p, basis, partial, done,
+                       w0);
+    IQ_OK(hipGetLastError());
+    if (one) return;
+    hipLaunchKernelGGL(k_marginal_sums, dim3(ncols), dim3(kMargBlocks), 0, s, static_cast<const MargItem*>(nullptr),
+                       ncols, nb, partial, w0);
+    IQ_OK(hipGetLastError());
 }
 
 void launch_marginal_cols(bool c64, const void* amp, uint64_t col_stride, uint32_t ncols, uint64_t nwork, int p,
                           int basis, double* partial, uint32_t* done, double* w0, hipStream_t s)
 {
-    const dim3 g(marginal_blocks(c64, nwork), ncols);
     if (c64)
-        hipLaunchKernelGGL(k_marginal_cols<float2>, g, dim3(kMargThreads), 0, s, static_cast<const float2*>(amp),
-                           col_stride, nwork, p, basis, partial, done, w0);
+        marginal_cols(static_cast<const float2*>(amp), col_stride, ncols, nwork, p, basis, partial, done, w0, s);
     else
-        hipLaunchKernelGGL(k_marginal_cols<double2>, g, dim3(kMargThreads), 0, s, static_cast<const double2*>(amp),
-                           col_stride, nwork, p, basis, partial, done, w0);
-    IQ_OK(hipGetLastError());
+        marginal_cols(static_cast<const double2*>(amp), col_stride, ncols, nwork, p, basis, partial, done, w0, s);
 }
 
 // ------------------------------------------------------------- collapses
@@ -841,12 +914,23 @@ void ItemQueue::launch_items(hipStream_t s)
         run(c64_ ? k_op_items<float2> : k_op_items<double2>, grid(op_chunks_, kMaxGrid), kBlock,
             reinterpret_cast<const OpItem*>(d + o_opit), uint32_t(opit_.size()), op_chunks_,
             reinterpret_cast<const ColOp*>(d + o_ops));
-    // marginals and trees: a workgroup per chunk, up to 2^20 of them
-    if (!marg_.empty())
-        run(c64_ ? k_marginal_items<float2> : k_marginal_items<double2>, grid(marg_chunks_, uint64_t(1) << 20),
-            kMargThreads, marg_[0], table(marg_, o_marg), uint32_t(marg_.size()), marg_chunks_,
-            reinterpret_cast<double*>(d + o_part), reinterpret_cast<uint32_t*>(marg_.size() > 1 ? d + o_done : d),
-            reinterpret_cast<double*>(dout + p_w0));
+    if (!marg_.empty()) {
+        const MargItem* const items = table(marg_, o_marg);   // null for one item, which has at most kMargBlocks shares
+        const uint32_t ni = uint32_t(marg_.size());
+        double* const part = reinterpret_cast<double*>(d + o_part);
+        double* const w = reinterpret_cast<double*>(dout + p_w0);
+        if (!items || marg_chunks_ <= kMargOneLaunch) {
+            run(c64_ ? k_marginal_items<float2> : k_marginal_items<double2>, dim3(unsigned(marg_chunks_)), kMargThreads,
+                marg_[0], items, ni, part, reinterpret_cast<uint32_t*>(items ? d + o_done : d), w);
+        } else {
+            const uint64_t share = (marg_chunks_ + kMargGrid - 1) / kMargGrid;
+            run(c64_ ? k_marginal_shares<float2> : k_marginal_shares<double2>,
+                dim3(unsigned((marg_chunks_ + share - 1) / share)), kMargThreads, items, ni, marg_chunks_,
+                uint32_t(share), part, w);
+            run(k_marginal_sums, grid(ni, kMaxGrid), int(kMargBlocks), items, ni, 0u, part, w);
+        }
+    }
+    // trees: a workgroup per chunk, up to 2^20 of them
     for (int k = 0; k < kTreeSteps; ++k)
         if (!tree_[k].empty())
             run(k > 0 ? k_tree_items<double> : c64_ ? k_tree_items<float2> : k_tree_items<double2>,
