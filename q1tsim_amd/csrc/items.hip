@@ -892,6 +892,10 @@ void ItemQueue::launch_items(hipStream_t s)
         upload_table(dbuf_ + 256, hin_, up_bytes, s);
         launches_ += 1;
     }
+    // the next launch may rewrite hin_ once the upload has read it, or the
+    // sampling kernel its uniforms
+    const bool host_read = u_host && u_bytes;
+    if (up_bytes && !host_read) IQ_OK(hipEventRecord(in_done_, s));
     char* d = dbuf_;
     char* dout = out_host ? hout_dev_ : dbuf_ + dev_bytes;
     auto table = [&](const auto& v, size_t off) {
@@ -944,7 +948,7 @@ void ItemQueue::launch_items(hipStream_t s)
             reinterpret_cast<const double*>(u_host ? hin_dev_ + o_u - 256 : d + o_u), nruns,
             reinterpret_cast<uint64_t*>(dout + p_idx), cols_, reinterpret_cast<double*>(dout + p_top));
     }
-    if (in_bytes) IQ_OK(hipEventRecord(in_done_, s));
+    if (host_read) IQ_OK(hipEventRecord(in_done_, s));
     if (out_bytes && !out_host) {
         IQ_OK(hipMemcpyAsync(hout_, dout, out_bytes, hipMemcpyDeviceToHost, s));
         launches_ += 1;
