@@ -931,7 +931,8 @@ void ItemQueue::launch_items(hipStream_t s)
             run(c64_ ? k_marginal_shares<float2> : k_marginal_shares<double2>,
                 dim3(unsigned((marg_chunks_ + share - 1) / share)), kMargThreads, items, ni, marg_chunks_,
                 uint32_t(share), part, w);
-            run(k_marginal_sums, grid(ni, kMaxGrid), int(kMargBlocks), items, ni, 0u, part, w);
+            if (marg_chunks_ > ni)   // else every column is one share
+                run(k_marginal_sums, grid(ni, kMaxGrid), int(kMargBlocks), items, ni, 0u, part, w);
         }
     }
     // trees: a workgroup per chunk, up to 2^20 of them
