@@ -712,24 +712,25 @@ static void run_table(GpuVectorState& st, const char* host, size_t total, std::v
     SW_HIP_OK(hipGraphLaunch(exec, st.stream()));
 }
 
-// A flush of a state that is too small for tiles: whole-state programs
-// (k_whole), one launch for all columns, and single-gate kernels for the gates
-// no register phase takes.
-// A run of few gates between those goes to the single-gate kernels too, with the
-// same rounding (2.9 us a gate): a launch of k_whole reads its program first and
-// holds a column in one workgroup.  us per two-qubit unitary and run of gates,
-// k_whole / single kernels, complex128: 8 qubits 1 gate 8.4 / 7.1, 2 gates 8.4 /
-// 10.4; 12 qubits 1 gate 10.3 / 7.3, 2 10.5 / 10.4, 3 11.2 / 13.4; 13 qubits 2 12.6
-// / 10.5, 3 13.4 / 13.3, 4 14.6 / 16.7; 512 columns of 12 qubits 1 26.6 / 23.5, 2
-// 26.9 / 33.4.  Where the run is the whole flush, one gate more saves the table's
-// upload (8 qubits, 2 gates 17.5 / 14.6, 3 gates 18.2 / 17.2, 4 18.6 / 19.4).
-static size_t lone_gates(int n, size_t ncols, bool whole_flush)
+// Gates up to which a run of a small state goes to the single-gate kernels (2.9 us
+// a gate, with the rounding of k_whole): a launch of k_whole reads its program
+// first and holds a column in one workgroup.  us per two-qubit unitary and run of
+// gates, k_whole / single kernels: complex128, 8 qubits 1 gate 8.4 / 7.1, 2 gates
+// 8.4 / 10.4; 12 qubits 1 10.3 / 7.3, 2 10.5 / 10.4, 3 11.2 / 13.4; 13 qubits 2 12.6 /
+// 10.5, 3 13.4 / 13.3, 4 14.6 / 16.7; complex64, 12 qubits 1 9.9 / 7.2, 2 10.2 / 10.5;
+// 13 qubits 2 10.5 / 10.3, 3 11.1 / 13.2; 512 columns of 12 qubits complex128 1 26.6 /
+// 23.5, 2 26.9 / 33.4.  Where the run is the whole flush, one gate more saves the
+// table's upload (8 qubits, 2 gates 17.5 / 14.6, 3 gates 18.2 / 17.2, 4 18.6 / 19.4).
+static size_t lone_gates(int n, size_t ncols, size_t elem_bytes, bool whole_flush)
 {
     const uint64_t amps = uint64_t(ncols) << n;
-    const size_t few = n <= 11 || amps > (uint64_t(1) << 20) ? 1 : n == 12 ? 2 : 3;
-    return few + (whole_flush && amps <= (uint64_t(1) << 17));
+    const int few = amps > (uint64_t(1) << 20) ? 1 : std::max(1, n - (elem_bytes == 16 ? 10 : 11));
+    return size_t(few) + (whole_flush && amps <= (uint64_t(1) << 17));
 }
 
+// A flush of a state that is too small for tiles: whole-state programs
+// (k_whole), one launch for all columns, and single-gate kernels for the gates
+// no register phase takes and for short runs of gates.
 template <typename V>
 static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue, size_t col_begin, size_t col_end,
                       bool fresh, RunStats& stats)
@@ -742,7 +743,7 @@ static void run_whole(GpuVectorState& st, const std::vector<PendingGate>& queue,
     // not for a graph, which replays programs with new angles but no single gates,
     // nor for the first gates of an unwritten state
     if (!graph) {
-        const size_t few = lone_gates(n, ncols, steps.size() == 1);
+        const size_t few = lone_gates(n, ncols, sizeof(V), steps.size() == 1);
         for (size_t s = fresh ? 1 : 0; s < steps.size(); ++s)
             if (steps[s].gates.size() <= few) steps[s].sweep = false;
     }

@@ -72,9 +72,10 @@ def test_runs_between_dense_pairs(n, precision):
     b.close()
 
 
-@pytest.mark.parametrize("n,lone", [(5, 2), (11, 2), (12, 3), (13, 4)])
-def test_route_of_a_flush(n, lone):
-    s = prepared(n, "c128", 0)
+@pytest.mark.parametrize("precision,n,lone", [("c128", 5, 2), ("c128", 11, 2), ("c128", 12, 3), ("c128", 13, 4),
+                                              ("c64", 11, 2), ("c64", 12, 2), ("c64", 13, 3)])
+def test_route_of_a_flush(precision, n, lone):
+    s = prepared(n, precision, 0)
     for count in (1, lone, lone + 1):
         for m, bits in gates(n, count, 2):
             s.apply_gate(m, bits)
